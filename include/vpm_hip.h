@@ -77,9 +77,9 @@ const char* vpm_last_error(void);
 int vpm_device_count(void);
 
 /* ---- plain FP64 drop-in: one entry point per reference function --------
- * Faithful FP64 restatements of the reference arithmetic (IEEE division and
- * pow), with an LDS-tiled SoA memory design.  Results agree with the FP64
- * oracle to a few ulp of the sum. */
+ * The reference's sums and masks in FP64, its powers and divisions written in
+ * one inverse root per pair.  Results agree with the FP64 oracle to a few ulp
+ * of the sum. */
 
 /* ParticlesPhysicsCuda.py:11-97 (get_induced_velocity_at; same arithmetic in
  * ParticlesPhysics.py:9-74).  out[3][ld_out] at the m targets. */
@@ -104,6 +104,21 @@ int vpm_get_strength_gradients(const vpm_particles_t* p, double* out, int64_t ld
  * (CPU: nu_ij, A + 1e-8).  p->nu must be non-NULL. */
 int vpm_get_strength_gradients_pse(const vpm_particles_t* p, int variant,
                                    double* out, int64_t ld_out, void* stream);
+
+/* The vector sums above with a workspace: small sets then split their sources
+ * among workgroups (the entry points above split them within a workgroup
+ * only).  targets: evaluation points of VELOCITY and VORTICITY; NULL for the
+ * self evaluations VELOCITY, STRETCHING and PSE.  A workspace smaller than
+ * vpm_pair_sum_workspace_bytes (NULL and 0 included) means fewer splits.
+ * VELOCITY at targets and STRETCHING ignore the variant's arithmetic (it is
+ * the same in both plugins). */
+#define VPM_SUM_VELOCITY 0
+#define VPM_SUM_VORTICITY 1
+#define VPM_SUM_STRETCHING 2
+#define VPM_SUM_PSE 3
+size_t vpm_pair_sum_workspace_bytes(int64_t m, int64_t n);
+int vpm_pair_sum(const vpm_points_t* targets, const vpm_particles_t* p, int what, int variant,
+                 double* out, int64_t ld_out, void* workspace, size_t ws_bytes, void* stream);
 
 /* Scalar pair reductions.  *result (device, 1 double) is overwritten; the sum
  * is deterministic (fixed-order two-pass).  workspace must hold

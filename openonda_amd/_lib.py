@@ -43,6 +43,11 @@ PREC_F32C = 1
 SIGMA_GENERAL = 0
 SIGMA_UNIFORM = 1
 
+SUM_VELOCITY = 0
+SUM_VORTICITY = 1
+SUM_STRETCHING = 2
+SUM_PSE = 3
+
 G64_AUTO = 0
 G64_ALWAYS = 1
 G64_NEVER = 2
@@ -119,6 +124,8 @@ SIGNATURES = {
     "vpm_get_vorticity_field_at": (C.c_int, [_P(Points), _P(Particles), C.c_int, _VP, _I64, _VP]),
     "vpm_get_strength_gradients": (C.c_int, [_P(Particles), _VP, _I64, _VP]),
     "vpm_get_strength_gradients_pse": (C.c_int, [_P(Particles), C.c_int, _VP, _I64, _VP]),
+    "vpm_pair_sum_workspace_bytes": (_SZ, [_I64, _I64]),
+    "vpm_pair_sum": (C.c_int, [_P(Points), _P(Particles), C.c_int, C.c_int, _VP, _I64, _VP, _SZ, _VP]),
     "vpm_reduction_workspace_bytes": (_SZ, [_I64]),
     "vpm_get_total_kinetic_energy": (C.c_int, [_P(Particles), C.c_int, _VP, _VP, _SZ, _VP]),
     "vpm_get_total_helicity": (C.c_int, [_P(Particles), C.c_int, _VP, _VP, _SZ, _VP]),

@@ -119,50 +119,47 @@ def _variant(v):
 
 
 # ------------------------------------------------------------ plain drop-in
+def _pair_sum(what, targets, p, pos, m, variant, out):
+    o = _out_vec(out, pos, m)
+    nb = L.load().vpm_pair_sum_workspace_bytes(m, p.n)
+    # a buffer per call, not the shared workspace: it belongs to the current
+    # stream, and to the graph that captures the call
+    ws = torch.empty(nb, dtype=torch.uint8, device=pos.device) if nb else None
+    L.call("vpm_pair_sum", C.byref(targets) if targets is not None else None, C.byref(p), what,
+           variant, o.data_ptr(), _ld(o), ws.data_ptr() if nb else None, nb, _stream(pos))
+    return o
+
+
 def induced_velocity_at(targets, pos, alpha, sigma, out=None):
     """u at M targets (ParticlesPhysicsCuda.py:11-97).  Returns (3, M)."""
     p = _particles(pos, alpha, sigma)
     t = _points(targets)
-    o = _out_vec(out, pos, targets.shape[1])
-    L.call("vpm_get_induced_velocity_at", C.byref(t), C.byref(p), o.data_ptr(), _ld(o),
-           _stream(pos))
-    return o
+    return _pair_sum(L.SUM_VELOCITY, t, p, pos, targets.shape[1], L.VARIANT_CUDA, out)
 
 
 def selfinduced_velocity(pos, alpha, sigma, variant="cuda", out=None):
     """u_i from all j != i (ParticlesPhysicsCuda.py:103-191).  Returns (3, N)."""
     p = _particles(pos, alpha, sigma)
-    o = _out_vec(out, pos, pos.shape[1])
-    L.call("vpm_get_selfinduced_velocity", C.byref(p), _variant(variant), o.data_ptr(), _ld(o),
-           _stream(pos))
-    return o
+    return _pair_sum(L.SUM_VELOCITY, None, p, pos, pos.shape[1], _variant(variant), out)
 
 
 def vorticity_field_at(targets, pos, alpha, sigma, variant="cuda", out=None):
     """Smoothed vorticity at M targets (ParticlesPhysicsCuda.py:198-219,291-346)."""
     p = _particles(pos, alpha, sigma)
     t = _points(targets)
-    o = _out_vec(out, pos, targets.shape[1])
-    L.call("vpm_get_vorticity_field_at", C.byref(t), C.byref(p), _variant(variant), o.data_ptr(),
-           _ld(o), _stream(pos))
-    return o
+    return _pair_sum(L.SUM_VORTICITY, t, p, pos, targets.shape[1], _variant(variant), out)
 
 
 def strength_gradients(pos, alpha, sigma, out=None):
     """Transpose-scheme stretching (ParticlesPhysicsCuda.py:351-445)."""
     p = _particles(pos, alpha, sigma)
-    o = _out_vec(out, pos, pos.shape[1])
-    L.call("vpm_get_strength_gradients", C.byref(p), o.data_ptr(), _ld(o), _stream(pos))
-    return o
+    return _pair_sum(L.SUM_STRETCHING, None, p, pos, pos.shape[1], L.VARIANT_CUDA, out)
 
 
 def strength_gradients_pse(pos, alpha, sigma, nu, variant="cuda", out=None):
     """PSE diffusion (ParticlesPhysicsCuda.py:452-530)."""
     p = _particles(pos, alpha, sigma, nu)
-    o = _out_vec(out, pos, pos.shape[1])
-    L.call("vpm_get_strength_gradients_pse", C.byref(p), _variant(variant), o.data_ptr(), _ld(o),
-           _stream(pos))
-    return o
+    return _pair_sum(L.SUM_PSE, None, p, pos, pos.shape[1], _variant(variant), out)
 
 
 def _reduction(fn, pos, alpha, sigma, variant):
