@@ -316,6 +316,13 @@ int vpm_adjoint(const vpm_particles_t* p, const vpm_adjoint_in_t* in,
 int vpm_induced_velocity_at_adjoint(const vpm_points_t* targets, const vpm_particles_t* src,
                                     const double* lam, int64_t ld_lam, double* dpos, double* dstr,
                                     int64_t ld_out, void* stream);
+/* The same with a workspace, so that few sources split their targets among
+ * workgroups (smaller than the query, NULL and 0 included: fewer splits). */
+size_t vpm_induced_velocity_at_adjoint_workspace_bytes(int64_t m, int64_t n);
+int vpm_induced_velocity_at_adjoint_ws(const vpm_points_t* targets, const vpm_particles_t* src,
+                                       const double* lam, int64_t ld_lam, double* dpos,
+                                       double* dstr, int64_t ld_out, void* workspace,
+                                       size_t ws_bytes, void* stream);
 
 /* ---- device-resident time integration (all FP64, no host sync) ---------
  * The O(N) parts of a reference solver step, so a step can run (and be

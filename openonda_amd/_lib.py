@@ -143,6 +143,8 @@ SIGNATURES = {
     "vpm_adjoint_workspace_bytes": (_SZ, [_I64, _P(ForwardOpts)]),
     "vpm_adjoint": (C.c_int, [_P(Particles), _P(AdjointIn), _P(ForwardOpts), _P(AdjointOut), _VP, _SZ, _VP]),
     "vpm_induced_velocity_at_adjoint": (C.c_int, [_P(Points), _P(Particles), _VP, _I64, _VP, _VP, _I64, _VP]),
+    "vpm_induced_velocity_at_adjoint_workspace_bytes": (_SZ, [_I64, _I64]),
+    "vpm_induced_velocity_at_adjoint_ws": (C.c_int, [_P(Points), _P(Particles), _VP, _I64, _VP, _VP, _I64, _VP, _SZ, _VP]),
     "vpm_axpy3": (C.c_int, [_I64, _I64, _VP, _VP, C.c_double, _VP, _VP]),
     "vpm_rk4_combine": (C.c_int, [_I64, _I64, _VP, _VP, _VP, _VP, _VP, C.c_double, _VP, _VP]),
     "vpm_strength_update": (C.c_int, [_I64, _I64, C.c_int, C.c_double, _VP, _VP, _VP, _VP, _VP, _VP]),

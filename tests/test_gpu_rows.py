@@ -13,7 +13,9 @@ import torch
 
 from openonda_amd import _lib as L
 from openonda_amd import physics as P
+from openonda_amd import autograd as AG
 from oracle import vpm_oracle as O
+from oracle import vpm_torch as T
 
 pytestmark = pytest.mark.gpu
 
@@ -97,6 +99,29 @@ def test_splits_agree_with_the_unsplit_sum(gpu, n):
     assert rel(P.from_soa(P.strength_gradients(dx, da, ds)), P.from_soa(out)) <= 1e-13
     L.call("vpm_get_strength_gradients_pse", C.byref(p), 0, out.data_ptr(), n, st)
     assert rel(P.from_soa(P.strength_gradients_pse(dx, da, ds, dn)), P.from_soa(out)) <= 1e-13
+
+
+@pytest.mark.parametrize("m,n", [(1, 1), (3, 65), (5, 64), (700, 63), (130, 2999)])
+def test_probe_adjoint_at_row_edges(gpu, m, n):
+    """Gradient of the velocity at m points with respect to n particles, one
+    point on a particle (masked), against torch autograd of the oracle."""
+    print(f"[rows-adjoint] m={m} n={n}", flush=True)
+    x, a, s, _ = particles(n, n + 2)
+    y = np.random.default_rng(m).uniform(-1.2, 1.2, (m, 3))
+    if m > 1:
+        y[1] = x[n // 2]
+    lam = np.random.default_rng(m + 1).normal(size=(m, 3))
+    leaf = [torch.from_numpy(t).cuda().requires_grad_() for t in (x, a)]
+    ref = torch.autograd.grad(
+        (T.induced_velocity_at(torch.from_numpy(y).cuda(), *leaf, torch.from_numpy(s).cuda())
+         * torch.from_numpy(lam).cuda()).sum(), leaf)
+    dx, da, ds, _ = dev(x, a, s, s, 3)
+    dx.requires_grad_()
+    da.requires_grad_()
+    got = torch.autograd.grad(AG.probe_velocity(strided(y, 2), dx, da, ds), (dx, da),
+                              strided(lam, 0))
+    for g, r in zip(got, ref):
+        assert rel(P.from_soa(g), r.cpu().numpy()) <= VEC_TOL
 
 
 def test_stretching_along_a_tube(gpu):
