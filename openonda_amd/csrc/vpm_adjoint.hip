@@ -562,6 +562,7 @@ int adj_layout(int64_t n, int presorted, AdjLayout* L) {
 struct OpVelAtAdjoint {
   static constexpr bool kTargetData = true, kRadius = false, kNu = false, kSkipSelf = false;
   static constexpr int kOut = 6;
+  static constexpr bool kSum = false, kSelfTerm = false;
   struct Acc { double A[3] = {0, 0, 0}, L[3] = {0, 0, 0}, X[3] = {0, 0, 0}; };
   static __device__ __forceinline__ void pair(Acc& a, const RowTarget& t, const RowSource& s) {
     const double rx = t.x - s.x, ry = t.y - s.y, rz = t.z - s.z;
@@ -621,8 +622,8 @@ int vel_at_adjoint(const vpm_points_t* targets, const vpm_particles_t* src, cons
   a.ld = targets->ld;
   a.q = lam;
   a.qld = ld_lam;
-  a.out0 = dpos;
-  a.out1 = dstr;
+  a.out[0] = dpos;
+  a.out[1] = dstr;
   a.ld_out = ld_out;
   return row_launch<OpVelAtAdjoint>(a, ws, ws_bytes, as_stream(stream), "vel_at_adjoint");
 }

@@ -36,6 +36,7 @@
 #include <type_traits>
 
 #include "vpm_common.h"
+#include "vpm_forward_rows.h"
 #include "vpm_prepass.h"
 
 namespace vpm {
@@ -1483,14 +1484,8 @@ int launch_f32(const FusedArgs& a, int cfg, hipStream_t st, int* nb) {
 }
 
 template <unsigned OUT>
-int launch_mask(const FusedArgs& a, int prec, bool unif, int cfg, hipStream_t st, int* nb) {
-  if (prec == VPM_PREC_F32C) return unif ? launch_f32<OUT, true>(a, cfg, st, nb)
-                                         : launch_f32<OUT, false>(a, cfg, st, nb);
-  if (unif)
-    return launch_cfg<double, OUT, true, kCfgF64.block, kCfgF64.r, kCfgF64.tile, kCfgF64.sub,
-                      kCfgF64.comp>(a, st, nb);
-  return launch_cfg<double, OUT, false, kCfgF64.block, kCfgF64.r, kCfgF64.tile, kCfgF64.sub,
-                    kCfgF64.comp>(a, st, nb);
+int launch_mask(const FusedArgs& a, bool unif, int cfg, hipStream_t st, int* nb) {
+  return unif ? launch_f32<OUT, true>(a, cfg, st, nb) : launch_f32<OUT, false>(a, cfg, st, nb);
 }
 
 // Output sets with their own instantiation; any other non-empty set runs the
@@ -1503,19 +1498,18 @@ unsigned kernel_mask(unsigned want) {
   return 31u;
 }
 
-int dispatch(const FusedArgs& a, unsigned mask, int prec, bool unif, int cfg, hipStream_t st,
-             int* nb) {
+int dispatch(const FusedArgs& a, unsigned mask, bool unif, int cfg, hipStream_t st, int* nb) {
   switch (mask) {
-    case 1u: return launch_mask<1u>(a, prec, unif, cfg, st, nb);
-    case 2u: return launch_mask<2u>(a, prec, unif, cfg, st, nb);
-    case 3u: return launch_mask<3u>(a, prec, unif, cfg, st, nb);
-    case 4u: return launch_mask<4u>(a, prec, unif, cfg, st, nb);
-    case 7u: return launch_mask<7u>(a, prec, unif, cfg, st, nb);
-    case 8u: return launch_mask<8u>(a, prec, unif, cfg, st, nb);
-    case 16u: return launch_mask<16u>(a, prec, unif, cfg, st, nb);
-    case 24u: return launch_mask<24u>(a, prec, unif, cfg, st, nb);
-    case 27u: return launch_mask<27u>(a, prec, unif, cfg, st, nb);
-    default: return launch_mask<31u>(a, prec, unif, cfg, st, nb);
+    case 1u: return launch_mask<1u>(a, unif, cfg, st, nb);
+    case 2u: return launch_mask<2u>(a, unif, cfg, st, nb);
+    case 3u: return launch_mask<3u>(a, unif, cfg, st, nb);
+    case 4u: return launch_mask<4u>(a, unif, cfg, st, nb);
+    case 7u: return launch_mask<7u>(a, unif, cfg, st, nb);
+    case 8u: return launch_mask<8u>(a, unif, cfg, st, nb);
+    case 16u: return launch_mask<16u>(a, unif, cfg, st, nb);
+    case 24u: return launch_mask<24u>(a, unif, cfg, st, nb);
+    case 27u: return launch_mask<27u>(a, unif, cfg, st, nb);
+    default: return launch_mask<31u>(a, unif, cfg, st, nb);
   }
 }
 
@@ -1545,13 +1539,10 @@ int split_slots(unsigned mask) {
 // Room for the largest source split launch_cfg may choose for this call.
 size_t split_capacity(int64_t n, const vpm_forward_opts_t* o) {
   if (!o || n <= 0) return 0;
-  int br = kCfgF64.block * kCfgF64.r, tile = kCfgF64.tile;
-  if (o->precision == VPM_PREC_F32C) {
-    const int c = effective_config(kernel_mask(o->outputs), o->sigma_mode == VPM_SIGMA_UNIFORM,
-                                   o->tile_config < kNumCfgs ? o->tile_config : -1);
-    br = kCfgs[c].block * kCfgs[c].r;
-    tile = kCfgs[c].tile;
-  }
+  if (forward_rows_wanted(n, o)) return forward_rows_split_bytes(n, kernel_mask(o->outputs));
+  const int c = effective_config(kernel_mask(o->outputs), o->sigma_mode == VPM_SIGMA_UNIFORM,
+                                 o->tile_config < kNumCfgs ? o->tile_config : -1);
+  const int br = kCfgs[c].block * kCfgs[c].r, tile = kCfgs[c].tile;
   const int64_t blocks = ceil_div(n, br);
   const int kmax = max_splits_for(blocks, ceil_div(n, tile));
   if (kmax < 2) return 0;
@@ -2115,9 +2106,12 @@ int forward_run_impl(const vpm_particles_t* p, const vpm_forward_opts_t* o,
     }
     return VPM_OK;
   }
+  const unsigned mask = kernel_mask(want);
+  if (forward_rows_wanted(n, o))
+    return forward_rows(p, o, out, mask, reinterpret_cast<double*>(ws + L.ens_part),
+                        L.split_bytes ? ws + L.split : nullptr, L.split_bytes, st);
   // Unrequested outputs of a superset kernel share one scratch region; a
   // thread writes only its own target's rows there, so they cannot race.
-  const unsigned mask = kernel_mask(want);
   double* scratch = reinterpret_cast<double*>(ws + L.scratch_vec);
   FusedArgs a{};
   a.n = static_cast<int>(n);
@@ -2147,7 +2141,7 @@ int forward_run_impl(const vpm_particles_t* p, const vpm_forward_opts_t* o,
   }
   int nblocks = 0;
   const int cfg = effective_config(mask, o->sigma_mode == VPM_SIGMA_UNIFORM, o->tile_config);
-  int rc = dispatch(a, mask, o->precision, o->sigma_mode == VPM_SIGMA_UNIFORM, cfg, st, &nblocks);
+  int rc = dispatch(a, mask, o->sigma_mode == VPM_SIGMA_UNIFORM, cfg, st, &nblocks);
   if (rc) return rc;
   if (want & VPM_OUT_ENSTROPHY) {
     const double k = (1.0 / (8.0 * kPi)) * kOneOverFourPi;
@@ -2242,12 +2236,15 @@ int vpm_forward_noalloc(const vpm_particles_t* p, const vpm_forward_opts_t* o,
   char* ws = nullptr;
   if ((rc = scratch_ptr(&ws))) return rc;
   hipStream_t st = as_stream(stream);
-  if ((rc = forward_prepare_impl(p, o, ws, L, st))) return rc;
+  if (!forward_rows_wanted(p->n, o) && (rc = forward_prepare_impl(p, o, ws, L, st))) return rc;
   return forward_run_impl(p, o, out, ws, L, st);
 }
 
 int vpm_forward(const vpm_particles_t* p, const vpm_forward_opts_t* o, vpm_forward_out_t* out,
                 void* workspace, size_t ws_bytes, void* stream) {
+  // the rows read the particles in the caller's order: nothing to prepare
+  if (p && o && forward_rows_wanted(p->n, o))
+    return vpm_forward_run(p, o, out, workspace, ws_bytes, stream);
   int rc = vpm_forward_prepare(p, o, workspace, ws_bytes, stream);
   if (rc) return rc;
   return vpm_forward_run(p, o, out, workspace, ws_bytes, stream);

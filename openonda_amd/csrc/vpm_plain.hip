@@ -53,6 +53,7 @@ struct VelKernel {
 struct OpVelAt {
   static constexpr bool kTargetData = false, kRadius = true, kNu = false, kSkipSelf = false;
   static constexpr int kOut = 3;
+  static constexpr bool kSum = false, kSelfTerm = false;
   struct Acc { double ux = 0, uy = 0, uz = 0; };
   static __device__ __forceinline__ void pair(Acc& a, const RowTarget& t, const RowSource& s) {
     const double rx = t.x - s.x, ry = t.y - s.y, rz = t.z - s.z;
@@ -77,6 +78,7 @@ template <bool CPUV>
 struct OpVelSelf {
   static constexpr bool kTargetData = true, kRadius = !CPUV, kNu = false, kSkipSelf = true;
   static constexpr int kOut = 3;
+  static constexpr bool kSum = false, kSelfTerm = false;
   struct Acc { double ux = 0, uy = 0, uz = 0; };
   static __device__ __forceinline__ void pair(Acc& a, const RowTarget& t, const RowSource& s) {
     const double rx = t.x - s.x, ry = t.y - s.y, rz = t.z - s.z;
@@ -99,6 +101,7 @@ template <bool CPUV>
 struct OpVortAt {
   static constexpr bool kTargetData = false, kRadius = true, kNu = false, kSkipSelf = false;
   static constexpr int kOut = 3;
+  static constexpr bool kSum = false, kSelfTerm = false;
   struct Acc { double wx = 0, wy = 0, wz = 0; };
   static __device__ __forceinline__ void pair(Acc& a, const RowTarget& t, const RowSource& s) {
     const double rx = t.x - s.x, ry = t.y - s.y, rz = t.z - s.z;
@@ -138,6 +141,7 @@ struct OpVortAt {
 struct OpStretch {
   static constexpr bool kTargetData = true, kRadius = true, kNu = false, kSkipSelf = true;
   static constexpr int kOut = 3;
+  static constexpr bool kSum = false, kSelfTerm = false;
   struct Acc { double sx = 0, sy = 0, sz = 0, gx = 0, gy = 0, gz = 0; };
   static __device__ __forceinline__ void pair(Acc& a, const RowTarget& t, const RowSource& s) {
     const double rx = t.x - s.x, ry = t.y - s.y, rz = t.z - s.z;
@@ -169,6 +173,7 @@ template <bool CPUV>
 struct OpPse {
   static constexpr bool kTargetData = true, kRadius = true, kNu = true, kSkipSelf = true;
   static constexpr int kOut = 3;
+  static constexpr bool kSum = false, kSelfTerm = false;
   struct Acc { double dx = 0, dy = 0, dz = 0; };
   static __device__ __forceinline__ void pair(Acc& a, const RowTarget& t, const RowSource& s) {
     const double rx = t.x - s.x, ry = t.y - s.y, rz = t.z - s.z;
@@ -302,7 +307,7 @@ int vel_at(const vpm_points_t* t, const vpm_particles_t* src, double* out, int64
   if ((rc = check_particles(src, false, who))) return rc;
   if ((rc = check_out(out, ld_out, t->m, who))) return rc;
   RowArgs a = args_at(t, src);
-  a.out0 = out;
+  a.out[0] = out;
   a.ld_out = ld_out;
   return row_launch<OpVelAt>(a, ws, ws_bytes, as_stream(stream), "vel_at");
 }
@@ -314,7 +319,7 @@ int vort_at(const vpm_points_t* t, const vpm_particles_t* src, int variant, doub
   if ((rc = check_particles(src, false, who))) return rc;
   if ((rc = check_out(out, ld_out, t->m, who))) return rc;
   RowArgs a = args_at(t, src);
-  a.out0 = out;
+  a.out[0] = out;
   a.ld_out = ld_out;
   if (variant == VPM_VARIANT_CUDA)
     return row_launch<OpVortAt<false>>(a, ws, ws_bytes, as_stream(stream), "vort_at");
@@ -331,7 +336,7 @@ int self_sum(const vpm_particles_t* p, int what, int variant, double* out, int64
   if (variant != VPM_VARIANT_CUDA && variant != VPM_VARIANT_CPU)
     return fail(VPM_ERR_ARG, "unknown variant");
   RowArgs a = args_from(p);
-  a.out0 = out;
+  a.out[0] = out;
   a.ld_out = ld_out;
   hipStream_t st = as_stream(stream);
   const bool cpu = variant == VPM_VARIANT_CPU;

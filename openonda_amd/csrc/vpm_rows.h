@@ -62,8 +62,7 @@ struct RowArgs {
   int64_t qld;
   const double* s;      // [n]
   const double* nu;     // [n]
-  double* out0;         // components 0..2, [3][ld_out]
-  double* out1;         // components 3..5
+  double* out[4];       // vector outputs, [3][ld_out] each; a null one is not stored
   int64_t ld_out;
   double* part;         // split partials [split][component][rows * 64], or null
   double* sums;         // one partial per workgroup (scalar operators)
@@ -152,8 +151,9 @@ __device__ __forceinline__ RowTarget row_target(const RowArgs& a, int64_t i) {
 // Vector operators.  grid (rows, splits).
 template <class Op>
 __global__ __launch_bounds__(kRowBlock, 4) void row_kernel(RowArgs a) {
-  constexpr int NA = Op::kOut;
-  __shared__ double red[kRowWaves][NA][kRow];
+  constexpr int NA = Op::kOut;               // vector components
+  constexpr int NV = NA + (Op::kSum ? 1 : 0);  // + one scalar summed over the targets
+  __shared__ double red[kRowWaves][NV][kRow];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kRow;
@@ -165,29 +165,35 @@ __global__ __launch_bounds__(kRowBlock, 4) void row_kernel(RowArgs a) {
   if constexpr (Op::kSkipSelf) {  // the row's own particles [o0, o1): j != i
     const int64_t o0 = row0 < b ? b : (row0 < e ? row0 : e);
     const int64_t o1 = row0 + kRow < b ? b : (row0 + kRow < e ? row0 + kRow : e);
-    for (int64_t j = o0; j < o1; ++j)
+    for (int64_t j = o0; j < o1; ++j) {
       if (j != t.i) Op::pair(acc, t, src.at(j));
+      if constexpr (Op::kSelfTerm) {
+        if (j == t.i) Op::self(acc, t);
+      }
+    }
 #pragma unroll 1
     for (int side = 0; side < 2; ++side) row_sweep<Op>(acc, t, src, side ? o1 : b, side ? e : o0);
   } else {
     row_sweep<Op>(acc, t, src, b, e);
   }
-  double v[NA];
+  double v[NV];
   Op::result(acc, t, v);
 #pragma unroll
-  for (int q = 0; q < NA; ++q) red[wave][q][lane] = v[q];
+  for (int q = 0; q < NV; ++q) red[wave][q][lane] = v[q];
   __syncthreads();
-  if (static_cast<int>(threadIdx.x) < NA * kRow) {
-    const int q = threadIdx.x >> 6;  // one wave per component
+  for (int q = wave; q < NV; q += kRowWaves) {  // one wave per component
     double s = 0.0;
 #pragma unroll
     for (int w = 0; w < kRowWaves; ++w) s += red[w][q][lane];
     const int64_t i = row0 + lane;
-    if (a.part) {
+    if (q == NA) {
+      s = wave_sum(i < a.m ? s : 0.0);
+      if (lane == 0) a.sums[static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x] = s;
+    } else if (a.part) {
       const int64_t pm = static_cast<int64_t>(gridDim.x) * kRow;
       a.part[(static_cast<int64_t>(blockIdx.y) * NA + q) * pm + i] = s;
-    } else if (i < a.m) {
-      (q < 3 ? a.out0 : a.out1)[(q % 3) * a.ld_out + i] = s;
+    } else if (i < a.m && a.out[q / 3]) {
+      a.out[q / 3][(q % 3) * a.ld_out + i] = s;
     }
   }
 }
@@ -196,10 +202,10 @@ __global__ __launch_bounds__(kRowBlock, 4) void row_kernel(RowArgs a) {
 __global__ __launch_bounds__(256) void row_reduce_kernel(RowArgs a, int na, int64_t pm) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   const int q = blockIdx.y;
-  if (i >= a.m) return;
+  if (i >= a.m || !a.out[q / 3]) return;
   double s = 0.0;
   for (int k = 0; k < a.splits; ++k) s += a.part[(static_cast<int64_t>(k) * na + q) * pm + i];
-  (q < 3 ? a.out0 : a.out1)[(q % 3) * a.ld_out + i] = s;
+  a.out[q / 3][(q % 3) * a.ld_out + i] = s;
 }
 
 // Symmetric scalar sums over pairs i != j (each unordered pair once, counted
@@ -263,27 +269,41 @@ inline int row_splits(int64_t groups, int64_t n) {
 
 inline int64_t row_count(int64_t m) { return ceil_div(m, kRow); }
 
-// Bytes of split partials row_launch can use for m targets and n sources.
-inline size_t row_workspace_bytes(int64_t m, int64_t n, int na) {
+// Bytes of one split's partials, and of all that row_launch can use for m
+// targets and n sources.
+inline size_t row_split_bytes(int64_t rows, int na, bool sum) {
+  return (static_cast<size_t>(na) * kRow + (sum ? 1 : 0)) * rows * sizeof(double);
+}
+inline size_t row_workspace_bytes(int64_t m, int64_t n, int na, bool sum = false) {
   const int k = row_splits(row_count(m), n);
-  return k > 1 ? static_cast<size_t>(k) * na * row_count(m) * kRow * sizeof(double) : 0;
+  return k > 1 ? k * row_split_bytes(row_count(m), na, sum) : 0;
 }
 
 // ws may be null or smaller than row_workspace_bytes: fewer splits then.
+// max_splits: 0 or the most splits to use.  kSum operators write one partial
+// per workgroup to a.sums (room for the rows), or behind the split partials;
+// *sums and *nsums say where and how many.
 template <class Op>
-int row_launch(RowArgs a, void* ws, size_t ws_bytes, hipStream_t st, const char* name) {
+int row_launch(RowArgs a, void* ws, size_t ws_bytes, hipStream_t st, const char* name,
+               int max_splits = 0, double** sums = nullptr, int64_t* nsums = nullptr) {
   if (a.m == 0) return VPM_OK;
   const int64_t rows = row_count(a.m);
-  const size_t per = static_cast<size_t>(Op::kOut) * rows * kRow * sizeof(double);
+  const size_t per = row_split_bytes(rows, Op::kOut, Op::kSum);
   int k = row_splits(rows, a.n);
+  if (max_splits > 0) k = std::min(k, max_splits);
   if (!ws || ws_bytes / per < 2) k = 1;
   else k = static_cast<int>(std::min<size_t>(k, ws_bytes / per));
   a.splits = k;
   a.part = k > 1 ? static_cast<double*>(ws) : nullptr;
+  if constexpr (Op::kSum) {
+    if (k > 1) a.sums = a.part + static_cast<int64_t>(k) * Op::kOut * rows * kRow;
+    *sums = a.sums;
+    *nsums = rows * k;
+  }
   hipLaunchKernelGGL(row_kernel<Op>, dim3(static_cast<unsigned>(rows), k), dim3(kRowBlock), 0, st,
                      a);
   VPM_LAUNCH_CHECK(name);
-  if (k > 1) {
+  if (k > 1 && Op::kOut > 0) {
     hipLaunchKernelGGL(row_reduce_kernel, dim3(static_cast<unsigned>(ceil_div(a.m, 256)), Op::kOut),
                        dim3(256), 0, st, a, Op::kOut, rows * kRow);
     VPM_LAUNCH_CHECK("row_reduce_kernel");

@@ -14,6 +14,7 @@ import torch
 from openonda_amd import _lib as L
 from openonda_amd import physics as P
 from openonda_amd import autograd as AG
+from openonda_amd import flow_models as FM
 from oracle import vpm_oracle as O
 from oracle import vpm_torch as T
 
@@ -168,3 +169,74 @@ def test_non_finite_inputs_carry_on_as_in_the_reference(gpu):
     assert np.isnan(P.total_kinetic_energy(dx, da, ds).item())
     assert np.isfinite(P.total_enstrophy(dx, da, ds).item())
     assert np.isfinite(P.from_soa(P.selfinduced_velocity(dx, da, ds))).all()
+
+
+OUTS = [("vel",), ("stretch",), ("vel", "stretch"), ("pse",), ("vort",), ("enstrophy",),
+        ("vel", "stretch", "pse"), ("vort", "enstrophy"), ("vel", "stretch", "vort", "enstrophy"),
+        ("vel", "pse"), ("vel", "stretch", "pse", "vort", "enstrophy")]
+
+
+def plain_outputs(d, outputs):
+    x, a, s, nu = d
+    ref = {"vel": lambda: P.selfinduced_velocity(x, a, s),
+           "stretch": lambda: P.strength_gradients(x, a, s),
+           "pse": lambda: P.strength_gradients_pse(x, a, s, nu),
+           "vort": lambda: P.vorticity_field_at(x, x, a, s),
+           "enstrophy": lambda: P.total_enstrophy(x, a, s)}
+    return {k: ref[k]() for k in outputs}
+
+
+@pytest.mark.parametrize("uniform", [True, False])
+@pytest.mark.parametrize("outputs", OUTS, ids="-".join)
+@pytest.mark.parametrize("n", [1, 65, 1031, 8191])
+def test_fused_rows(gpu, n, outputs, uniform):
+    """The FP64 pass, and the FP32-compensated one up to 8191 particles, are
+    the FP64 rows: the plain kernels' values (pinned to the oracle above) to
+    1e-12 for every output set, radius mode, split count and input stride."""
+    print(f"[rows-forward] n={n} {outputs} uniform={uniform}", flush=True)
+    x, a, s, nu = particles(n, n + 3)
+    if uniform:
+        s[:] = 0.17
+    d = dev(x, a, s, nu, 5)
+    ref = plain_outputs(d, outputs)
+    mode = "uniform" if uniform else "general"
+    for kw in ({"precision": "f64"}, {"precision": "f32c"}, {"precision": "f64", "max_splits": 1}):
+        got = P.forward(*d, outputs=outputs, sigma_mode=mode, **kw)
+        for k in outputs:
+            r, g = ref[k].cpu().numpy(), got[k].cpu().numpy()
+            assert rel(g, r) <= (SCAL_TOL if k == "enstrophy" else VEC_TOL), (k, kw)
+
+
+def test_first_size_past_the_rows(gpu):
+    """One particle more and the FP32-compensated kernels run: 1e-6, not 1e-12;
+    a tile shape asked for by index runs them at any size."""
+    for n, kw in ((8192, {}), (8191, {"tile_config": 5})):
+        x, a, s, nu = particles(n, n)
+        s[:] = 0.17
+        d = dev(x, a, s, nu, 0)
+        ref = plain_outputs(d, ("vel", "stretch"))
+        got = P.forward(*d, outputs=("vel", "stretch"), sigma_mode="uniform", **kw)
+        for k in ref:
+            e = rel(got[k].cpu().numpy(), ref[k].cpu().numpy())
+            assert 1e-10 < e <= 1e-6, (n, k, e)
+
+
+@pytest.mark.parametrize("layout", ["ring", "cloud"])
+@pytest.mark.parametrize("outputs", [("vel", "stretch"), ("vel", "stretch", "pse"),
+                                     ("vel", "stretch", "pse", "vort", "enstrophy")])
+def test_fp32_kernels_at_small_sizes(gpu, layout, outputs):
+    """The FP32-compensated kernels (asked for by tile shape) over near and far
+    tiles in one pass and in splits, against the rows; the empty-split and
+    ragged edges at sizes the default leaves to the rows."""
+    for n in (37, 700, 4096):
+        x, a, s, nu = (FM.torus_ring(-(-n // 64), nu=1e-3) if layout == "ring"
+                       else FM.random_cloud(n, seed=41))
+        x, a, s, nu = x[:n], a[:n], s[:n], np.full(n, 1e-3)
+        d = dev(x, a, s, nu, 0)
+        ref = P.forward(*d, outputs=outputs, precision="f64", sigma_mode="uniform")
+        for splits in (0, 1, 3):
+            got = P.forward(*d, outputs=outputs, sigma_mode="uniform", max_splits=splits,
+                            tile_config=P.tile_config_default(outputs))
+            for k in outputs:
+                e = rel(got[k].cpu().numpy(), ref[k].cpu().numpy())
+                assert e <= 1e-6, (layout, n, splits, k, e)
