@@ -54,6 +54,11 @@ int check_out(const double* out, int64_t ld, int64_t n, const char* who);
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// A particle in sorted order: position, strength, radius, viscosity.
+struct alignas(16) Src8 {
+  double x, y, z, ax, ay, az, s, nu;
+};
+
 // ---- source splits -----------------------------------------------------
 // When the target blocks of an all-pairs pass cannot fill the device, the
 // sources are split among workgroups (grid.y) and FP64 partial sums per

@@ -12,10 +12,6 @@ namespace vpm {
 
 namespace {
 
-struct alignas(16) Src8 {
-  double x, y, z, ax, ay, az, s, nu;
-};
-
 constexpr int kPreBlock = 256;
 constexpr int kBboxBlocks = 512;
 
