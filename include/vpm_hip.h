@@ -143,10 +143,10 @@ int vpm_get_total_enstrophy(const vpm_particles_t* p, int variant, double* resul
  *   PSE      PSE diffusion with nu_i     (:478-530)
  *   VORT     LES smoothed vorticity      (:291-346, targets = particles)
  *   ENSTROPHY total enstrophy scalar     (:756-777,867-920)
- * precision F32C: FP32 pair arithmetic on block-centred offsets of
- * Morton-sorted particles, FP32 sub-tile partials combined with Kahan
- * compensation per source tile and folded into FP64 totals.
- * precision F64: the same pass in FP64 throughout. */
+ * precision F32C: FP32 pair arithmetic on centred offsets of Morton-sorted
+ * particles, FP32 partials of at most 128 sources folded into FP64 totals;
+ * sets below 8,192 particles run the FP64 pass.
+ * precision F64: the same sums in FP64 throughout, in the caller's order. */
 #define VPM_OUT_VEL 1u
 #define VPM_OUT_STRETCH 2u
 #define VPM_OUT_PSE 4u
@@ -164,7 +164,9 @@ typedef struct vpm_forward_opts {
   int32_t precision;    /* VPM_PREC_* */
   int32_t sigma_mode;   /* VPM_SIGMA_* */
   int32_t presorted;    /* 1: particles already spatially coherent, skip the Morton sort */
-  int32_t tile_config;  /* -1: default; else index < vpm_tile_config_count() */
+  int32_t tile_config;  /* -1: the row pass (rows of 64 targets, no tiles); else an
+                         * index < vpm_tile_config_count(): the tiled F32C kernels
+                         * in that shape */
   int32_t max_splits;   /* 0: automatic; k >= 1: at most k source splits.  When the
                          * target blocks alone cannot fill the device, the sources
                          * are split among workgroups and the FP64 partial sums
@@ -227,7 +229,7 @@ size_t vpm_forward_noalloc_capacity(void);
  * autotuner).  Writes block threads, targets per lane, source tile, sub-tile
  * length and compensation mode (0 Kahan+FP64, 1 direct FP64 fold). */
 int vpm_tile_config_count(void);
-/* index used for tile_config = -1 with these outputs: one set with a uniform
+/* the tiled kernels' default shape for these outputs: one set with a uniform
  * radius / a batch (FP32) */
 int vpm_tile_config_default(uint32_t outputs);
 int vpm_batch_tile_config_default(uint32_t outputs);

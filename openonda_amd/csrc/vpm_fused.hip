@@ -1,4 +1,7 @@
-// Fused all-pairs forward pass (the fast path).
+// Tiled all-pairs forward pass: the batched launch, the tile shapes a caller
+// asks for by index, and sets too large for vpm_forward_noalloc's array with
+// the row pass's records.  (Other single-set calls run vpm_row32.hip or
+// vpm_forward_rows.hip.)
 //
 // One pass over all (target, source) pairs computes any subset of the GPU
 // plugin's outputs -- self-induced velocity, transpose-scheme stretching, PSE
@@ -1204,7 +1207,7 @@ constexpr TileCfg kCfgs[] = {
 
 constexpr bool hot_mask(unsigned m) { return m == 3u || m == 7u || m == 27u; }
 
-// Shapes for tile_config = -1, the autotuner's winners on one MI355X:
+// Default shapes, the autotuner's winners on one MI355X:
 //  * velocity + stretching, uniform sigma: config 5 (512 lanes x one target,
 //    128-source FP32 partials: half the folds of config 0; random cloud of
 //    2^20: 685 ms against 693 ms, rel-L2 5.0e-7 against 4.5e-7);
@@ -1358,7 +1361,7 @@ bool wants_far_records(const vpm_forward_opts_t* o) {
 }
 
 bool row32_asked(const vpm_forward_opts_t* o) {
-  return o && row32_wanted(kernel_mask(o->outputs), o->sigma_mode == VPM_SIGMA_UNIFORM, o);
+  return o && row32_wanted(o);
 }
 
 // FP64 partial slots per target of a source split (see Slots::nslot)

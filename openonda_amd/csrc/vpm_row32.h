@@ -5,12 +5,11 @@
 
 namespace vpm {
 
-// Output sets and radius modes the row pass runs when no tile shape is asked
-// for: those without the far-field moment form (it needs velocity, stretching
-// and a uniform radius).
-inline bool row32_wanted(unsigned mask, bool unif, const vpm_forward_opts_t* o) {
-  const bool moment = unif && (mask & VPM_OUT_VEL) && (mask & VPM_OUT_STRETCH);
-  return o->precision == VPM_PREC_F32C && o->tile_config < 0 && !moment;
+// The row pass runs every FP32-compensated call that asks for no tile shape
+// (vpm_row32.hip has both sides measured: it was faster on every output set,
+// radius mode and size from 8,192 to 2^20).
+inline bool row32_wanted(const vpm_forward_opts_t* o) {
+  return o->precision == VPM_PREC_F32C && o->tile_config < 0;
 }
 
 // Bytes of the FP32 records, the chunk boxes and the split partials.

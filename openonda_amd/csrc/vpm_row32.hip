@@ -5,30 +5,35 @@
 // a row's few near chunks spread over the waves.  Every lane of a wave pairs
 // with the same source, so the sources come through scalar loads from FP32
 // records relative to their chunk's centre, and enter the pair instructions
-// as scalar operands: no LDS staging, no barrier in the sweep.  (The staged
-// form read 48 bytes per source and wave from LDS with per-particle radii,
-// 3 x 8 clocks of the CU's LDS return path against about 18 clocks of FP32
-// issue: LDS bound it.)  The target's offset to the chunk centre comes from
-// FP64 positions once per chunk; FP32 partials of a chunk are folded into
-// FP64 totals.
+// as scalar operands: no LDS staging, no barrier in the sweep.  (The tiled
+// kernels read up to 48 bytes per source and wave from LDS, 3 x 8 clocks of
+// the CU's LDS return path against about 18 clocks of FP32 issue: LDS bound
+// them.)  The target's offset to the chunk centre comes from FP64 positions
+// once per chunk; FP32 partials of a chunk are folded into FP64 totals, which
+// wait in LDS meanwhile.
 //
-// Stretching: waves of coherent strengths (coherent_wave) take the sum of
-// g alpha_j and the triple product in FP64 on chunks near the row and in FP32
-// on far ones (gap between the boxes above kFarGap32 times the larger
-// radius), the others in FP32 everywhere, as in the tiled kernels
-// (vpm_fused.hip, which also measures why); sets with vorticity or enstrophy
-// and without PSE sum in FP64 on near chunks in every wave.
+// Far chunks (gap between the row's and the chunk's boxes above kFarGap32
+// times the larger radius) of sets with velocity, stretching and a uniform
+// radius take the moment form (pair_far).  Stretching: rows of coherent
+// strengths (coherent_wave) take the sum of g alpha_j and the triple product
+// in FP64 on near chunks and in FP32 on far ones, the others in FP32
+// everywhere, as in the tiled kernels (vpm_fused.hip, which also measures
+// why); sets with vorticity or enstrophy and without PSE sum in FP64 on near
+// chunks in every row.
 //
 // With s = sigma_ij, D = r^2 + s^2, t = D^-1/2 and w = s^2 t^2 no reciprocal
 // of s is needed: (rho^2 + 2.5) / (A^5/2 s^3) = t^3 (1 + 1.5 w) and so on
 // (vpm_plain.hip).
 //
 // Bound: FP32 issue (velocity alone 2.45e12 pairs/s, 1.55 wave64 instructions
-// per clock and CU).  Tiled kernels -> here, per call at N = 100,000: velocity
-// 4.80 -> 4.17 ms, with per-particle radii 6.80 -> 4.78; stretching of a ring
-// 9.51 -> 7.40, 11.5 -> 7.31; PSE 5.81 -> 4.92, 6.96 -> 5.78; vorticity +
-// enstrophy 4.97 -> 4.73, 7.41 -> 5.98; all five with per-particle radii 16.0
-// -> 14.7 (cloud), 19.4 -> 15.4 (ring); at 8,192 to 35,000 alike.
+// per clock and CU; the moment form 1.8e12).  Tiled kernels -> here, per call.
+// N = 100,000: velocity 4.80 -> 4.17 ms, with per-particle radii 6.80 -> 4.78;
+// stretching of a ring 9.51 -> 7.40, 11.5 -> 7.31; PSE 5.81 -> 4.92, 6.96 ->
+// 5.78; vorticity + enstrophy 4.97 -> 4.73, 7.41 -> 5.98; all five with
+// per-particle radii 16.0 -> 14.7 (cloud), 19.4 -> 15.4 (ring).  Velocity +
+// stretching: cloud of 2^20 614 -> 605, of 20,000 0.448 -> 0.328, ring of
+// 131,072 12.8 -> 11.1; with PSE: ring of 131,072 15.7 -> 13.1, leapfrogging
+// rings of 65,536 4.30 -> 3.49.
 
 #include "vpm_row32.h"
 
@@ -40,20 +45,37 @@ namespace vpm {
 
 namespace {
 
-constexpr int kChunk32 = 64;      // sources per chunk
+constexpr int kMinChunk32 = 64, kMaxChunk32 = 128;  // sources per chunk (Rec32)
 constexpr int kStride32 = 12;     // most floats per record
-constexpr int kGroup32 = 4;       // records per group of scalar loads
+constexpr int kMaxGroup32 = 4;    // records per group of scalar loads (Rec32)
 constexpr int kBox32 = 8;         // doubles per chunk box: centre, half-extent, largest radius
 constexpr double kFarGap32 = 4.0;
+// Waves per SIMD the registers must allow: 73 VGPRs for velocity + stretching
+// (cloud of 2^20: 605 ms; 641 at five waves, 687 at eight, where the records
+// spill scalar registers).
+constexpr int kRow32Waves = 6;
 
-// Record layout: offset (3), strength (3), with per-particle radii sigma/2
-// and sigma^2, with PSE the low parts alpha - fp32(alpha); lengths in units
-// of the first particle's radius.
+// Record layout: offset (3), strength (3); then with the moment form the
+// moment alpha x offset (3; three times it with PSE, pair_far), with
+// per-particle radii sigma/2 and sigma^2; with PSE the low parts
+// alpha - fp32(alpha).  Lengths in units of the first particle's radius.
+// Two groups are in registers at once: of four records, or of two where a
+// record has twelve floats and four would spill scalar registers (velocity +
+// stretching + PSE, cloud of 131,072: 11.4 against 12.5 ms, ring 13.4 against
+// 13.8).  Chunks of 128 sources halve the moment form's set-up and fold per chunk;
+// with the LES outputs 64 keep the vorticity's partials as short as they were
+// (rel-L2 1.0e-7 against 1.5e-7 on a ring of 20,000).
 template <unsigned OUT, bool UNIF>
 struct Rec32 {
   static constexpr bool kLo = OUT & VPM_OUT_PSE;
-  static constexpr int kLoAt = UNIF ? 6 : 8;
-  static constexpr int kStride = kLo ? 12 : (UNIF ? 6 : 8);
+  static constexpr bool kMoment = UNIF && (OUT & VPM_OUT_VEL) && (OUT & VPM_OUT_STRETCH);
+  static constexpr bool kE3 = kMoment && kLo;
+  static constexpr int kLoAt = kMoment ? 9 : UNIF ? 6 : 8;
+  static constexpr int kStride = kLo ? 12 : kMoment ? 9 : UNIF ? 6 : 8;
+  static constexpr int kGroup = kLo ? 2 : kMaxGroup32;
+  static constexpr int kNear = kLo ? 4 : 2;  // sources in flight in the FP64 loop
+  static constexpr int kChunk =
+      kMoment && !(OUT & (VPM_OUT_VORT | VPM_OUT_ENSTROPHY)) ? kMaxChunk32 : kMinChunk32;
 };
 
 __device__ __forceinline__ double held(double v) {  // rounded here, not fused into its use
@@ -61,49 +83,80 @@ __device__ __forceinline__ double held(double v) {  // rounded here, not fused i
   return v;
 }
 
-// One workgroup of 64 lanes per chunk.  Lanes past n write zero-strength
-// padding far away, which adds exactly 0.
-__global__ __launch_bounds__(kChunk32) void row32_records_kernel(const Src8* __restrict__ src,
-                                                                 int n, int stride, int lo_at,
-                                                                 int unif,
-                                                                 float* __restrict__ rec,
-                                                                 double* __restrict__ box) {
+// One workgroup per chunk.  Lanes past n write zero-strength padding far
+// away, which adds exactly 0.
+template <unsigned OUT, bool UNIF>
+__global__ __launch_bounds__((Rec32<OUT, UNIF>::kChunk)) void row32_records_kernel(
+    const Src8* __restrict__ src, int n, float* __restrict__ rec, double* __restrict__ box_) {
+  using R = Rec32<OUT, UNIF>;
+  __shared__ double red[7][R::kChunk / 64];
   const int c = blockIdx.x;
-  const int k = c * kChunk32 + static_cast<int>(threadIdx.x);
+  const int k = c * R::kChunk + static_cast<int>(threadIdx.x);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const bool ok = k < n;
   const double scale = 1.0 / src[0].s;
   Src8 g{};
   if (ok) g = src[k];
   const double p[3] = {held(g.x * scale), held(g.y * scale), held(g.z * scale)};
-  double cen[3];
+  const double sig = g.s * scale;
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
     const double lo = wave_min(ok ? p[q] : INFINITY), hi = wave_max(ok ? p[q] : -INFINITY);
-    cen[q] = 0.5 * (lo + hi);
-    if (threadIdx.x == 0) {
-      box[static_cast<int64_t>(c) * kBox32 + q] = cen[q];
-      box[static_cast<int64_t>(c) * kBox32 + 3 + q] = 0.5 * (hi - lo);
+    if (lane == 0) {
+      red[q][wave] = lo;
+      red[3 + q][wave] = hi;
     }
   }
-  const double sig = g.s * scale, smax = wave_max(ok ? sig : 0.0);
-  if (threadIdx.x == 0) box[static_cast<int64_t>(c) * kBox32 + 6] = smax;
-  float* r = rec + static_cast<int64_t>(k) * stride;
+  const double big = wave_max(ok ? sig : 0.0);
+  if (lane == 0) red[6][wave] = big;
+  __syncthreads();
+  double cen[3];
+  double* box = box_ + static_cast<int64_t>(c) * kBox32;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    double lo = red[q][0], hi = red[3 + q][0];
+#pragma unroll
+    for (int w = 1; w < R::kChunk / 64; ++w) {
+      lo = fmin(lo, red[q][w]);
+      hi = fmax(hi, red[3 + q][w]);
+    }
+    cen[q] = 0.5 * (lo + hi);
+    if (threadIdx.x == 0) {
+      box[q] = cen[q];
+      box[3 + q] = 0.5 * (hi - lo);
+    }
+  }
+  if (threadIdx.x == 0) {
+    double m = red[6][0];
+#pragma unroll
+    for (int w = 1; w < R::kChunk / 64; ++w) m = fmax(m, red[6][w]);
+    box[6] = m;
+    box[7] = 0.0;
+  }
+  float* r = rec + static_cast<int64_t>(k) * R::kStride;
+  const double x = p[0] - cen[0], y = p[1] - cen[1], z = p[2] - cen[2];
   const float ax = static_cast<float>(g.ax), ay = static_cast<float>(g.ay),
               az = static_cast<float>(g.az);
-  for (int q = 0; q < 3; ++q) r[q] = ok ? static_cast<float>(p[q] - cen[q]) : 1e18f;
+  r[0] = ok ? static_cast<float>(x) : 1e18f;
+  r[1] = ok ? static_cast<float>(y) : 1e18f;
+  r[2] = ok ? static_cast<float>(z) : 1e18f;
   r[3] = ax;
   r[4] = ay;
   r[5] = az;
-  if (!unif) {
+  if constexpr (R::kMoment) {
+    constexpr double ms = R::kE3 ? 3.0 : 1.0;
+    r[6] = ok ? static_cast<float>(ms * (g.ay * z - g.az * y)) : 0.0f;
+    r[7] = ok ? static_cast<float>(ms * (g.az * x - g.ax * z)) : 0.0f;
+    r[8] = ok ? static_cast<float>(ms * (g.ax * y - g.ay * x)) : 0.0f;
+  } else if constexpr (!UNIF) {
     r[6] = ok ? static_cast<float>(0.5 * sig) : 0.5f;
     r[7] = ok ? static_cast<float>(sig * sig) : 1.0f;
   }
-  if (stride == 12) {
-    r[lo_at] = static_cast<float>(g.ax - static_cast<double>(ax));
-    r[lo_at + 1] = static_cast<float>(g.ay - static_cast<double>(ay));
-    r[lo_at + 2] = static_cast<float>(g.az - static_cast<double>(az));
-    for (int q = lo_at + 3; q < stride; ++q) r[q] = 0.0f;
-    for (int q = unif ? 6 : 8; q < lo_at; ++q) r[q] = 0.0f;
+  if constexpr (R::kLo) {
+    r[R::kLoAt] = static_cast<float>(g.ax - static_cast<double>(ax));
+    r[R::kLoAt + 1] = static_cast<float>(g.ay - static_cast<double>(ay));
+    r[R::kLoAt + 2] = static_cast<float>(g.az - static_cast<double>(az));
+    for (int q = R::kLoAt + 3; q < R::kStride; ++q) r[q] = 0.0f;
   }
 }
 
@@ -137,9 +190,21 @@ __device__ __forceinline__ void pair32(float* acc, double* g64, const Tgt32& t, 
   const float w = UNIF ? t2 : s2 * t2;
   if constexpr (S::vel || S::str) {
     const float g = t3 * __builtin_fmaf(k.c15, w, 1.0f);
-    const float cx = dy * f[5] - dz * f[4];
-    const float cy = dz * f[3] - dx * f[5];
-    const float cz = dx * f[4] - dy * f[3];
+    float cx, cy, cz, e = 0.0f;
+    if constexpr (G64 && S::str) {
+      const double rx = dx, ry = dy, rz = dz;
+      const double qx = ry * aj[2] - rz * aj[1];
+      const double qy = rz * aj[0] - rx * aj[2];
+      const double qz = rx * aj[1] - ry * aj[0];
+      e = static_cast<float>(ai[0] * qx + ai[1] * qy + ai[2] * qz);
+      cx = static_cast<float>(qx);
+      cy = static_cast<float>(qy);
+      cz = static_cast<float>(qz);
+    } else {
+      cx = dy * f[5] - dz * f[4];
+      cy = dz * f[3] - dx * f[5];
+      cz = dx * f[4] - dy * f[3];
+    }
     if constexpr (S::vel) {
       acc[kU + 0] += g * cx;
       acc[kU + 1] += g * cy;
@@ -147,17 +212,11 @@ __device__ __forceinline__ void pair32(float* acc, double* g64, const Tgt32& t, 
     }
     if constexpr (S::str) {
       const float gG = self ? 0.0f : g;
-      float e;
       if constexpr (G64) {
         const double gd = gG;
         g64[0] = fma(gd, aj[0], g64[0]);
         g64[1] = fma(gd, aj[1], g64[1]);
         g64[2] = fma(gd, aj[2], g64[2]);
-        const double rx = dx, ry = dy, rz = dz;
-        const double qx = ry * aj[2] - rz * aj[1];
-        const double qy = rz * aj[0] - rx * aj[2];
-        const double qz = rx * aj[1] - ry * aj[0];
-        e = static_cast<float>(ai[0] * qx + ai[1] * qy + ai[2] * qz);
       } else {
         acc[kG + 0] += gG * f[3];
         acc[kG + 1] += gG * f[4];
@@ -199,15 +258,71 @@ __device__ __forceinline__ void pair32(float* acc, double* g64, const Tgt32& t, 
   }
 }
 
+// The far-field moment form of velocity + stretching with a uniform radius
+// (pair_moment in vpm_fused.hip derives and measures it): 29 instructions per
+// pair, p = alpha_i x x_i (three times it with PSE).
+template <unsigned OUT>
+__device__ __forceinline__ void pair_far(float* acc, const Tgt32& t, const float* p, const float* f,
+                                         const PairConst<float>& k) {
+  using S = Slots<OUT>;
+  const float dx = t.x - f[0], dy = t.y - f[1], dz = t.z - f[2];
+  const float D = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, 1.0f)));
+  const float t1 = __builtin_amdgcn_rsqf(D);
+  const float t2 = t1 * t1;
+  const float t3 = t2 * t1;
+  const float t5 = t3 * t2;
+  const float g = __builtin_fmaf(k.c15, t5, t3);
+  acc[kG + 0] = __builtin_fmaf(g, f[3], acc[kG + 0]);
+  acc[kG + 1] = __builtin_fmaf(g, f[4], acc[kG + 1]);
+  acc[kG + 2] = __builtin_fmaf(g, f[5], acc[kG + 2]);
+  acc[kH + 0] = __builtin_fmaf(g, f[6], acc[kH + 0]);
+  acc[kH + 1] = __builtin_fmaf(g, f[7], acc[kH + 1]);
+  acc[kH + 2] = __builtin_fmaf(g, f[8], acc[kH + 2]);
+  float e = f[3] * p[0];
+  e = __builtin_fmaf(f[4], p[1], e);
+  e = __builtin_fmaf(f[5], p[2], e);
+  e = __builtin_fmaf(t.ax, f[6], e);
+  e = __builtin_fmaf(t.ay, f[7], e);
+  e = __builtin_fmaf(t.az, f[8], e);
+  const float t7 = t5 * t2;
+  float w;
+  if constexpr (Rec32<OUT, true>::kE3)
+    w = __builtin_fmaf(k.c25, t7, t5) * e;
+  else
+    w = t5 * __builtin_fmaf(k.c75, t2, k.c3) * e;
+  acc[kSd + 0] = __builtin_fmaf(w, dx, acc[kSd + 0]);
+  acc[kSd + 1] = __builtin_fmaf(w, dy, acc[kSd + 1]);
+  acc[kSd + 2] = __builtin_fmaf(w, dz, acc[kSd + 2]);
+  if constexpr (S::vort) {
+    acc[kW + 0] = __builtin_fmaf(t7, f[3], acc[kW + 0]);
+    acc[kW + 1] = __builtin_fmaf(t7, f[4], acc[kW + 1]);
+    acc[kW + 2] = __builtin_fmaf(t7, f[5], acc[kW + 2]);
+  }
+  if constexpr (S::ens) {
+    const float en = __builtin_fmaf(k.c22, t3, t1);
+    acc[kE + 0] = __builtin_fmaf(en, f[3], acc[kE + 0]);
+    acc[kE + 1] = __builtin_fmaf(en, f[4], acc[kE + 1]);
+    acc[kE + 2] = __builtin_fmaf(en, f[5], acc[kE + 2]);
+  }
+  if constexpr (S::pse) {  // sum t9 alpha_j - alpha_i sum t9, the second part per chunk
+    const float t9 = t7 * t2;
+    acc[kP + 0] = __builtin_fmaf(t9, f[3], acc[kP + 0]);
+    acc[kP + 1] = __builtin_fmaf(t9, f[4], acc[kP + 1]);
+    acc[kP + 2] = __builtin_fmaf(t9, f[5], acc[kP + 2]);
+    acc[kT9] += t9;
+  }
+}
+
 // grid (rows, splits)
 template <unsigned OUT, bool UNIF>
-__global__ __launch_bounds__(kRowBlock, 4) void row32_kernel(FusedArgs a, int splits,
-                                                             const float* __restrict__ rec_,
-                                                             const double* __restrict__ box_) {
+__global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
+    FusedArgs a, int splits, const float* __restrict__ rec_, const double* __restrict__ box_) {
   using S = Slots<OUT>;
   using R = Rec32<OUT, UNIF>;
-  constexpr int NS = S::nslot;
-  __shared__ double red[kRowWaves][NS][kRow];
+  constexpr int NS = S::nslot, CH = R::kChunk;
+  // FP64 totals of each wave's share (kept here, not in registers: they are
+  // touched once per chunk) and, at the end, their sums
+  __shared__ double tot[kRowWaves][NS][kRow];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row = blockIdx.x;
@@ -250,134 +365,163 @@ __global__ __launch_bounds__(kRowBlock, 4) void row32_kernel(FusedArgs a, int sp
   }
 
   float part[kNAcc];
-  double tot[kNAcc], gsum[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-  for (int q = 0; q < kNAcc; ++q) {
-    part[q] = 0.0f;
-    tot[q] = 0.0;
-  }
+  for (int q = 0; q < kNAcc; ++q) part[q] = 0.0f;
+#pragma unroll
+  for (int q = 0; q < NS; ++q) tot[wave][q][lane] = 0.0;
   PairConst<float> kc{1.5f, 7.5f, 2.2f, 3.0f, 2.5f};  // in VGPRs (see PairConst)
-  asm volatile("" : "+v"(kc.c15), "+v"(kc.c75), "+v"(kc.c22), "+v"(kc.c3));
+  asm volatile("" : "+v"(kc.c15), "+v"(kc.c75), "+v"(kc.c22), "+v"(kc.c3), "+v"(kc.c25));
 
-  const int nchunk = (a.n + kChunk32 - 1) / kChunk32;
+  const int nchunk = (a.n + CH - 1) / CH;
   const int parts = splits * kRowWaves;
-  for (int c = static_cast<int>(blockIdx.y) * kRowWaves + wave; c < nchunk; c += parts) {
+  const int own = row * kRow / CH;          // the chunk that holds the row
+  uint64_t near = 0;                        // this wave's next 64 chunks near the row
+  int seen = 0;
+  for (int c = static_cast<int>(blockIdx.y) * kRowWaves + wave; c < nchunk; c += parts, ++seen) {
+    bool is_near = true;
+    if constexpr (S::str) {
+      // far tests for 64 of the wave's chunks at a time, one per lane
+      if ((seen & 63) == 0) {
+        const int64_t cc = c + static_cast<int64_t>(lane) * parts;
+        bool nr = false;
+        if (cc < nchunk) {
+          const double* box = box_ + cc * kBox32;
+          double gap2 = 0.0;
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            const double gp = fmax(fabs(box[q] - cen[q]) - half[q] - box[3 + q], 0.0);
+            gap2 += gp * gp;
+          }
+          const double lim = kFarGap32 * fmax(smax, box[6]);
+          nr = !(gap2 > lim * lim);
+        }
+        near = __ballot(nr);
+      }
+      is_near = ((near >> (seen & 63)) & 1u) != 0;
+    }
+    const bool fp64 = g64 && is_near;
     const scalar_double_t* box =
         (const scalar_double_t*)(box_ + static_cast<int64_t>(c) * kBox32);
     t.x = static_cast<float>(X - box[0]);
     t.y = static_cast<float>(Y - box[1]);
     t.z = static_cast<float>(Z - box[2]);
-    const int j0 = c * kChunk32;
+    const int j0 = c * CH;
     const far_float_t* rec =
         (const far_float_t*)(rec_ + static_cast<int64_t>(j0) * R::kStride);
-    bool fp64 = g64;
-    if constexpr (S::str) {
-      if (g64 && c != row) {
-        double gap2 = 0.0;
+    auto load1 = [&](float* f, int q) {
 #pragma unroll
-        for (int q = 0; q < 3; ++q) {
-          const double gp = fmax(fabs(box[q] - cen[q]) - half[q] - box[3 + q], 0.0);
-          gap2 += gp * gp;
-        }
-        const double lim = kFarGap32 * fmax(smax, box[6]);
-        fp64 = __builtin_amdgcn_readfirstlane(static_cast<int>(!(gap2 > lim * lim))) != 0;
-      }
-    }
-    auto load = [&](float* b, int q, int cnt) {
-#pragma unroll
-      for (int u = 0; u < kGroup32 * R::kStride; ++u)
-        if (u < cnt * R::kStride) b[u] = rec[q * R::kStride + u];
+      for (int u = 0; u < R::kStride; ++u) f[u] = rec[q * R::kStride + u];
     };
-    if (S::str && (c == row || fp64)) {
+    // Groups of records in two register buffers: a group's loads issue
+    // after the first pair of the one before it (scalar loads return out of
+    // order, so a wait covers every load in flight); the last reads one group
+    // of padding.
+    auto stream = [&](auto pair) {
+      float bA[R::kGroup * R::kStride], bB[R::kGroup * R::kStride];
+      auto load = [&](float* b, int q) {
+#pragma unroll
+        for (int u = 0; u < R::kGroup * R::kStride; ++u) b[u] = rec[q * R::kStride + u];
+      };
+      auto group = [&](const float* b, float* nb, int qn) {
+        pair(b);
+        __builtin_amdgcn_sched_barrier(0);
+        load(nb, qn);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 1; u < R::kGroup; ++u) pair(b + u * R::kStride);
+      };
+      load(bA, 0);
+#pragma unroll 1
+      for (int q = 0; q < CH; q += 2 * R::kGroup) {
+        group(bA, bB, q + R::kGroup);
+        group(bB, bA, q + 2 * R::kGroup);
+      }
+    };
+    double g64s[3] = {0.0, 0.0, 0.0};
+    if (S::str && (fp64 || c == own)) {
       if constexpr (S::str) {
-        // the row's own chunk, and near chunks of FP64 rows: valid sources only
-        const int cnt = a.n - j0 < kChunk32 ? a.n - j0 : kChunk32;
+        // near chunks of FP64 rows, and the row's own chunk: valid sources only
+        const int cnt = a.n - j0 < CH ? a.n - j0 : CH;
+        const int self = c == own ? lane + (row * kRow - j0) : -1;
         const scalar_double_t* str =
             (const scalar_double_t*)(reinterpret_cast<const double*>(a.src + j0));
         if (fp64) {
-          const bool own = c == row;
-#pragma unroll 2
+#pragma unroll R::kNear
           for (int q = 0; q < cnt; ++q) {
             float f[R::kStride];
-#pragma unroll
-            for (int u = 0; u < R::kStride; ++u) f[u] = rec[q * R::kStride + u];
+            load1(f, q);
             const double aj[3] = {str[q * 8 + 3], str[q * 8 + 4], str[q * 8 + 5]};
-            pair32<OUT, UNIF, true>(part, gsum, t, f, aj, ai, eps, kc, own && q == lane);
+            pair32<OUT, UNIF, true>(part, g64s, t, f, aj, ai, eps, kc, q == self);
           }
         } else {
 #pragma unroll 1
           for (int q = 0; q < cnt; ++q) {
             float f[R::kStride];
-#pragma unroll
-            for (int u = 0; u < R::kStride; ++u) f[u] = rec[q * R::kStride + u];
-            pair32<OUT, UNIF, false>(part, gsum, t, f, nullptr, ai, eps, kc, q == lane);
+            load1(f, q);
+            pair32<OUT, UNIF, false>(part, g64s, t, f, nullptr, ai, eps, kc, q == self);
           }
         }
       }
-    } else {
-      // groups of four in two register buffers: a group's loads issue after
-      // the first pair of the one before it (scalar loads return out of
-      // order, so a wait covers every load in flight); the last reads one
-      // group of padding
-      float bA[kGroup32 * R::kStride], bB[kGroup32 * R::kStride];
-      auto group = [&](const float* b, float* nb, int qn) {
-        pair32<OUT, UNIF, false>(part, gsum, t, b, nullptr, ai, eps, kc, false);
-        __builtin_amdgcn_sched_barrier(0);
-        load(nb, qn, kGroup32);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 1; u < kGroup32; ++u)
-          pair32<OUT, UNIF, false>(part, gsum, t, b + u * R::kStride, nullptr, ai, eps, kc, false);
-      };
-      load(bA, 0, kGroup32);
-#pragma unroll 1
-      for (int q = 0; q < kChunk32; q += 2 * kGroup32) {
-        group(bA, bB, q + kGroup32);
-        group(bB, bA, q + 2 * kGroup32);
+    } else if (!R::kMoment || is_near) {
+      stream([&](const float* f) {
+        pair32<OUT, UNIF, false>(part, g64s, t, f, nullptr, ai, eps, kc, false);
+      });
+    } else if constexpr (R::kMoment) {
+      constexpr float es = R::kE3 ? 3.0f : 1.0f;
+      const float p[3] = {es * (t.ay * t.z - t.az * t.y), es * (t.az * t.x - t.ax * t.z),
+                          es * (t.ax * t.y - t.ay * t.x)};
+      stream([&](const float* f) { pair_far<OUT>(part, t, p, f, kc); });
+      // u += x_i x G + H of the chunk, in FP64
+      const double x = X - box[0], y = Y - box[1], z = Z - box[2];
+      const double gx = part[kG + 0], gy = part[kG + 1], gz = part[kG + 2];
+      constexpr double hs = R::kE3 ? 1.0 / 3.0 : 1.0;
+      double* u = &tot[wave][0][lane];
+      u[0] += (y * gz - z * gy) + static_cast<double>(part[kH + 0]) * hs;
+      u[kRow] += (z * gx - x * gz) + static_cast<double>(part[kH + 1]) * hs;
+      u[2 * kRow] += (x * gy - y * gx) + static_cast<double>(part[kH + 2]) * hs;
+      part[kH + 0] = part[kH + 1] = part[kH + 2] = 0.0f;
+      if constexpr (S::pse) {
+        part[kP + 0] = __builtin_fmaf(-t.ax, part[kT9], part[kP + 0]);
+        part[kP + 1] = __builtin_fmaf(-t.ay, part[kT9], part[kP + 1]);
+        part[kP + 2] = __builtin_fmaf(-t.az, part[kT9], part[kP + 2]);
+        part[kT9] = 0.0f;
       }
     }
 #pragma unroll
     for (int q = 0; q < kNAcc; ++q)
       if (S::used(q)) {
-        tot[q] += static_cast<double>(part[q]);
+        tot[wave][S::packed(q)][lane] += static_cast<double>(part[q]);
         part[q] = 0.0f;
       }
     if constexpr (S::str) {
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
-        gsum[q] += static_cast<double>(part[kG + q]);
+        tot[wave][S::nacc + q][lane] += g64s[q] + static_cast<double>(part[kG + q]);
         part[kG + q] = 0.0f;
       }
     }
   }
 
   // the waves' totals, in wave order
-#pragma unroll
-  for (int q = 0; q < kNAcc; ++q)
-    if (S::used(q)) red[wave][S::packed(q)][lane] = tot[q];
-  if constexpr (S::str) {
-#pragma unroll
-    for (int q = 0; q < 3; ++q) red[wave][S::nacc + q][lane] = gsum[q];
-  }
   __syncthreads();
   for (int q = wave; q < NS; q += kRowWaves) {
     double s = 0.0;
 #pragma unroll
-    for (int w = 0; w < kRowWaves; ++w) s += red[w][q][lane];
+    for (int w = 0; w < kRowWaves; ++w) s += tot[w][q][lane];
     if (a.part)
       a.part[(static_cast<int64_t>(blockIdx.y) * NS + q) * a.pld + kt] = s;
     else
-      red[0][q][lane] = s;  // read by this wave only, above
+      tot[0][q][lane] = s;  // slot q is read by this wave only, above
   }
   if (a.part) return;
   __syncthreads();
   if (wave != 0) return;
   double T[kNAcc], G[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-  for (int q = 0; q < kNAcc; ++q) T[q] = S::used(q) ? red[0][S::packed(q)][lane] : 0.0;
+  for (int q = 0; q < kNAcc; ++q) T[q] = S::used(q) ? tot[0][S::packed(q)][lane] : 0.0;
   if constexpr (S::str) {
 #pragma unroll
-    for (int q = 0; q < 3; ++q) G[q] = red[0][S::nacc + q][lane];
+    for (int q = 0; q < 3; ++q) G[q] = tot[0][S::nacc + q][lane];
   }
   double ens = 0.0;
   if (valid) ens = store_target<OUT, true>(a, ti, a.perm ? a.perm[kt] : kt, T, G, scale);
@@ -397,7 +541,7 @@ template <unsigned OUT, bool UNIF>
 int launch(FusedArgs a, float* rec, double* box, hipStream_t st, int* nblocks) {
   using R = Rec32<OUT, UNIF>;
   const int rows = static_cast<int>(ceil_div(a.n, kRow));
-  const int chunks = static_cast<int>(ceil_div(a.n, kChunk32));
+  const int chunks = static_cast<int>(ceil_div(a.n, R::kChunk));
   const size_t per = static_cast<size_t>(Slots<OUT>::nslot) * rows * kRow * sizeof(double);
   int k = std::min(row_splits(rows, a.n), std::max(1, chunks / kRowWaves));
   if (a.max_splits > 0) k = std::min(k, a.max_splits);
@@ -405,8 +549,8 @@ int launch(FusedArgs a, float* rec, double* box, hipStream_t st, int* nblocks) {
   else k = static_cast<int>(std::min<size_t>(k, a.part_cap / per));
   if (k == 1) a.part = nullptr;
   a.pld = static_cast<int64_t>(rows) * kRow;
-  hipLaunchKernelGGL(row32_records_kernel, dim3(chunks), dim3(kChunk32), 0, st, a.src, a.n,
-                     R::kStride, R::kLoAt, UNIF ? 1 : 0, rec, box);
+  hipLaunchKernelGGL((row32_records_kernel<OUT, UNIF>), dim3(chunks), dim3(R::kChunk), 0, st,
+                     a.src, a.n, rec, box);
   VPM_LAUNCH_CHECK("row32_records_kernel");
   hipLaunchKernelGGL((row32_kernel<OUT, UNIF>), dim3(rows, k), dim3(kRowBlock), 0, st, a, k, rec,
                      box);
@@ -425,12 +569,12 @@ int launch(FusedArgs a, float* rec, double* box, hipStream_t st, int* nblocks) {
 
 // Records of whole chunks, and one group read ahead past the last.
 size_t row32_record_bytes(int64_t n) {
-  return (static_cast<size_t>(ceil_div(n > 0 ? n : 1, kChunk32)) * kChunk32 + kGroup32) *
+  return (static_cast<size_t>(ceil_div(n > 0 ? n : 1, kMaxChunk32)) * kMaxChunk32 + kMaxGroup32) *
          kStride32 * sizeof(float);
 }
 
 size_t row32_box_bytes(int64_t n) {
-  return static_cast<size_t>(ceil_div(n > 0 ? n : 1, kChunk32)) * kBox32 * sizeof(double);
+  return static_cast<size_t>(ceil_div(n > 0 ? n : 1, kMinChunk32)) * kBox32 * sizeof(double);
 }
 
 size_t row32_split_bytes(int64_t n, unsigned mask) {
@@ -445,8 +589,9 @@ int row32_run(const FusedArgs& a, unsigned mask, bool unif, float* rec, double* 
 #define VPM_ROW32(M, U)      \
   case (M) | ((U) ? 32u : 0u): \
     return launch<M, U>(a, rec, box, st, nblocks);
-    VPM_ROW32(1u, true) VPM_ROW32(2u, true) VPM_ROW32(4u, true) VPM_ROW32(8u, true)
-    VPM_ROW32(16u, true) VPM_ROW32(24u, true)
+    VPM_ROW32(1u, true) VPM_ROW32(2u, true) VPM_ROW32(3u, true) VPM_ROW32(4u, true)
+    VPM_ROW32(7u, true) VPM_ROW32(8u, true) VPM_ROW32(16u, true) VPM_ROW32(24u, true)
+    VPM_ROW32(27u, true) VPM_ROW32(31u, true)
     VPM_ROW32(1u, false) VPM_ROW32(2u, false) VPM_ROW32(3u, false) VPM_ROW32(4u, false)
     VPM_ROW32(7u, false) VPM_ROW32(8u, false) VPM_ROW32(16u, false) VPM_ROW32(24u, false)
     VPM_ROW32(27u, false) VPM_ROW32(31u, false)

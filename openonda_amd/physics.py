@@ -221,7 +221,8 @@ def forward(pos, alpha, sigma, nu=None, outputs=("vel", "stretch"), precision="f
     tensor.  ``precision`` is "f32c" (FP32 pairs, compensated FP64 totals)
     or "f64".  ``sigma_mode`` "uniform" asserts sigma_i == sigma_0 (not
     checked), "general" uses sigma_ij per pair, "auto" checks on the device.
-    ``tile_config``: -1 (default shape), an index of :func:`tile_configs`, or
+    ``tile_config``: -1 (the row pass), an index of :func:`tile_configs` (the
+    tiled kernels in that shape), or
     "auto" (the autotuner's cached winner for this N).
     ``max_splits``: 0 lets the library split the sources among workgroups
     when the targets alone cannot fill the device (small N); k >= 1 caps
@@ -297,7 +298,7 @@ def forward(pos, alpha, sigma, nu=None, outputs=("vel", "stretch"), precision="f
 
 
 def tile_config_default(outputs=("vel", "stretch")):
-    """Index of the tile configuration used for ``tile_config=-1`` (uniform radius)."""
+    """Index of the tiled kernels' default shape (uniform radius)."""
     if isinstance(outputs, str):
         outputs = (outputs,)
     mask = 0

@@ -1,5 +1,4 @@
-"""The FP32-compensated row pass (output sets without the far-field moment
-form): edges of rows, chunks, waves and splits, against the FP64 pass.
+"""The FP32-compensated row pass: edges of rows, chunks, waves and splits, against the FP64 pass.
 
 Bar: rel-L2 <= 1e-6 on every output (the pass's documented accuracy).
 """
@@ -16,10 +15,10 @@ from openonda_amd import physics as P
 pytestmark = pytest.mark.gpu
 
 TOL = 1e-6
-UNIFORM = [("vel",), ("stretch",), ("pse",), ("vort",), ("enstrophy",), ("vort", "enstrophy")]
-GENERAL = UNIFORM + [("vel", "stretch"), ("vel", "stretch", "pse"),
-                     ("vel", "stretch", "vort", "enstrophy"),
-                     ("vel", "stretch", "pse", "vort", "enstrophy")]
+UNIFORM = [("vel",), ("stretch",), ("pse",), ("vort",), ("enstrophy",), ("vort", "enstrophy"),
+           ("vel", "stretch"), ("vel", "stretch", "pse"), ("vel", "stretch", "vort", "enstrophy"),
+           ("vel", "stretch", "pse", "vort", "enstrophy")]
+GENERAL = UNIFORM
 
 
 def particles(layout, n, general):
