@@ -22,13 +22,12 @@
 // Sums over j of g a_j, g lam_j and f phi a_j are accumulated per target and
 // crossed with the target's vectors once; the three radial terms share one
 // accumulator.
-// The same block-centred FP32 offsets, LDS tiles and FP32-partial / FP64-total
-// accumulation as the forward pass are used (precision F32C); F64 runs the
-// same pass in double.
+// Precision F32C runs the rows of vpm_adj32.hip; the kernels here are F64's.
 
 #include <algorithm>
 #include <type_traits>
 
+#include "vpm_adj32.h"
 #include "vpm_common.h"
 #include "vpm_prepass.h"
 #include "vpm_rows.h"
@@ -499,25 +498,27 @@ int launch_adj(const AdjArgs& a0, hipStream_t st) {
   return VPM_OK;
 }
 
-template <typename Real, bool UNIF>
+template <bool UNIF>
 int adj_mask(const AdjArgs& a, unsigned mask, hipStream_t st) {
   switch (mask) {
-    case 1u: return launch_adj<Real, 1u, UNIF>(a, st);
-    case 2u: return launch_adj<Real, 2u, UNIF>(a, st);
-    case 3u: return launch_adj<Real, 3u, UNIF>(a, st);
-    case 4u: return launch_adj<Real, 4u, UNIF>(a, st);
-    case 5u: return launch_adj<Real, 5u, UNIF>(a, st);
-    case 6u: return launch_adj<Real, 6u, UNIF>(a, st);
-    default: return launch_adj<Real, 7u, UNIF>(a, st);
+    case 1u: return launch_adj<double, 1u, UNIF>(a, st);
+    case 2u: return launch_adj<double, 2u, UNIF>(a, st);
+    case 3u: return launch_adj<double, 3u, UNIF>(a, st);
+    case 4u: return launch_adj<double, 4u, UNIF>(a, st);
+    case 5u: return launch_adj<double, 5u, UNIF>(a, st);
+    case 6u: return launch_adj<double, 6u, UNIF>(a, st);
+    default: return launch_adj<double, 7u, UNIF>(a, st);
   }
 }
 
 struct AdjLayout {
-  size_t bbox_part, bbox, keys_in, keys_out, idx_in, perm, sorted, split, cub, total, cub_bytes,
-      split_bytes;
+  size_t bbox_part, bbox, keys_in, keys_out, idx_in, perm, sorted, box, split, cub, total,
+      cub_bytes, split_bytes;
 };
 
-int adj_layout(int64_t n, int presorted, AdjLayout* L) {
+// sorted: the FP64 pass's sorted arrays, or the records of the FP32 rows.
+int adj_layout(int64_t n, const vpm_forward_opts_t* o, AdjLayout* L) {
+  const bool f32 = o && o->precision == VPM_PREC_F32C;
   const size_t N = static_cast<size_t>(n > 0 ? n : 1);
   size_t off = 0;
   auto take = [&](size_t b) {
@@ -531,16 +532,18 @@ int adj_layout(int64_t n, int presorted, AdjLayout* L) {
   L->keys_out = take(N * 4);
   L->idx_in = take(N * 4);
   L->perm = take(N * 4);
-  L->sorted = take(17 * N * sizeof(double));
+  L->sorted = take(f32 ? adj32_record_bytes(n) : 17 * N * sizeof(double));
+  L->box = take(f32 ? adj32_box_bytes(n) : 0);
   // room for the largest source split, sized for all cotangents present
   const int64_t blocks = ceil_div(n, kAdjBlock);
   const int kmax = max_splits_for(blocks, ceil_div(n, kAdjTile));
-  L->split_bytes = kmax > 1 ? static_cast<size_t>(kmax) * AdjSlots<7u>::nslot *
-                                  static_cast<size_t>(blocks * kAdjBlock) * sizeof(double)
-                            : 0;
+  L->split_bytes = f32        ? adj32_split_bytes(n)
+                   : kmax > 1 ? static_cast<size_t>(kmax) * AdjSlots<7u>::nslot *
+                                    static_cast<size_t>(blocks * kAdjBlock) * sizeof(double)
+                              : 0;
   L->split = take(L->split_bytes);
   size_t cb = 0;
-  if (!presorted) {
+  if (!o || !o->presorted) {
     const int rc = sort_temp_bytes(n, &cb);
     if (rc) return rc;
   }
@@ -638,7 +641,7 @@ extern "C" {
 
 size_t vpm_adjoint_workspace_bytes(int64_t n, const vpm_forward_opts_t* opts) {
   AdjLayout L{};
-  if (adj_layout(n, opts ? opts->presorted : 0, &L) != VPM_OK) return 0;
+  if (adj_layout(n, opts, &L) != VPM_OK) return 0;
   return L.total;
 }
 
@@ -661,7 +664,7 @@ int vpm_adjoint(const vpm_particles_t* p, const vpm_adjoint_in_t* in, const vpm_
   if (out->ld < n || (n && (!out->dpos || !out->dstr)))
     return fail(VPM_ERR_ARG, "vpm_adjoint: bad output");
   AdjLayout L{};
-  if ((rc = adj_layout(n, o->presorted, &L))) return rc;
+  if ((rc = adj_layout(n, o, &L))) return rc;
   if (!workspace || ws_bytes < L.total) {
     set_error("vpm_adjoint: workspace %zu bytes < required %zu", ws_bytes, L.total);
     return VPM_ERR_WORKSPACE;
@@ -678,6 +681,16 @@ int vpm_adjoint(const vpm_particles_t* p, const vpm_adjoint_in_t* in, const vpm_
                      perm, ws + L.cub, L.cub_bytes, st);
     if (rc) return rc;
   }
+  if (o->max_splits < 0) return fail(VPM_ERR_ARG, "vpm_adjoint: max_splits < 0");
+  if (mask == 0) mask = VPM_OUT_VEL;  // all cotangents null: zero gradients from the vel pass
+  const bool unif = o->sigma_mode == VPM_SIGMA_UNIFORM;
+  double* part = L.split_bytes ? reinterpret_cast<double*>(ws + L.split) : nullptr;
+  if (o->precision == VPM_PREC_F32C)
+    return adj32_run(Adj32Args{*p, in->lam, in->mu, in->xi, in->ld, perm, out->dpos, out->dstr,
+                               out->ld, reinterpret_cast<float*>(ws + L.sorted),
+                               reinterpret_cast<double*>(ws + L.box), part, L.split_bytes,
+                               o->max_splits},
+                     mask, unif, st);
   double* sorted = reinterpret_cast<double*>(ws + L.sorted);
   const int ni = static_cast<int>(n);
   hipLaunchKernelGGL(adj_gather_kernel, dim3(static_cast<unsigned>(ceil_div(n, 256))), dim3(256), 0,
@@ -693,15 +706,10 @@ int vpm_adjoint(const vpm_particles_t* p, const vpm_adjoint_in_t* in, const vpm_
   a.dpos = out->dpos;
   a.dstr = out->dstr;
   a.ld = out->ld;
-  a.part = L.split_bytes ? reinterpret_cast<double*>(ws + L.split) : nullptr;
+  a.part = part;
   a.part_cap = L.split_bytes;
-  if (o->max_splits < 0) return fail(VPM_ERR_ARG, "vpm_adjoint: max_splits < 0");
   a.max_splits = o->max_splits;
-  if (mask == 0) mask = VPM_OUT_VEL;  // all cotangents null: zero gradients from the vel pass
-  const bool unif = o->sigma_mode == VPM_SIGMA_UNIFORM;
-  if (o->precision == VPM_PREC_F32C)
-    return unif ? adj_mask<float, true>(a, mask, st) : adj_mask<float, false>(a, mask, st);
-  return unif ? adj_mask<double, true>(a, mask, st) : adj_mask<double, false>(a, mask, st);
+  return unif ? adj_mask<true>(a, mask, st) : adj_mask<false>(a, mask, st);
 }
 
 int vpm_induced_velocity_at_adjoint(const vpm_points_t* targets, const vpm_particles_t* src,
