@@ -280,6 +280,14 @@ int vpm_batch_prepare(const vpm_particles_t* p, const vpm_batch_desc_t* d, int r
 int vpm_batch_run(const vpm_particles_t* p, const vpm_batch_desc_t* d,
                   const vpm_forward_opts_t* opts, vpm_forward_out_t* out, void* workspace,
                   size_t ws_bytes, void* stream);
+/* The same launch over rows of 64 targets (VPM_PREC_F32C): one workgroup per
+ * row, handed out in the item list's order, so the list keeps its largest
+ * sets first; `targets_per_item` says how many targets an item of the list
+ * stands for (64, 128, ... 512).  opts->tile_config and desc->grid do not
+ * apply. */
+int vpm_batch_run_rows(const vpm_particles_t* p, const vpm_batch_desc_t* desc, int targets_per_item,
+                       const vpm_forward_opts_t* opts, vpm_forward_out_t* out, void* workspace,
+                       size_t ws_bytes, void* stream);
 /* Per-set dynamic LES filter (vpmModule.py:887-962), one workgroup per set:
  * state[3*s..] = {C_nu, enstrophy_ref, has_ref}; writes nu_t (if the set's
  * max exceeds 1e-9) and nu_eff = nu + nu_t. */

@@ -139,6 +139,7 @@ SIGNATURES = {
     "vpm_batch_workspace_bytes": (_SZ, [_I64, C.c_int, C.c_int]),
     "vpm_batch_prepare": (C.c_int, [_P(Particles), _P(BatchDesc), C.c_int, _VP, _SZ, _VP]),
     "vpm_batch_run": (C.c_int, [_P(Particles), _P(BatchDesc), _P(ForwardOpts), _P(ForwardOut), _VP, _SZ, _VP]),
+    "vpm_batch_run_rows": (C.c_int, [_P(Particles), _P(BatchDesc), C.c_int, _P(ForwardOpts), _P(ForwardOut), _VP, _SZ, _VP]),
     "vpm_batch_les_update": (C.c_int, [_P(BatchDesc), _I64, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _SZ, _I64, _VP]),
     "vpm_adjoint_workspace_bytes": (_SZ, [_I64, _P(ForwardOpts)]),
     "vpm_adjoint": (C.c_int, [_P(Particles), _P(AdjointIn), _P(ForwardOpts), _P(AdjointOut), _VP, _SZ, _VP]),

@@ -49,8 +49,9 @@ class BatchedSystem:
 
     def __init__(self, sets, dt, precision="f32c", tile_config=-1, pse=True, les=True,
                  device=None, grid=0, resort_every=0, autotune_cache=None):
-        """``tile_config``: -1 (the library's default shape for the batch),
-        an index of physics.tile_configs(), or "auto" (the batch autotuner's
+        """``tile_config``: -1 (rows of 64 targets, one workgroup each), an
+        index of physics.tile_configs() (the persistent tiled launch), or
+        "auto" (the batch autotuner's
         cached (shape, grid) for this output set and total pair count, else
         the default).  ``grid``: persistent workgroups (0: as many as fit on
         the device).  ``resort_every``: re-sort the sets by Morton key every
@@ -75,6 +76,7 @@ class BatchedSystem:
 
             self.autotuned = autotune.best_batch_config(sizes, self.stage_mask, path=autotune_cache)
             tile_config, grid = self.autotuned if self.autotuned else (-1, grid)
+        rows = tile_config < 0 and grid == 0 and precision == "f32c"
         self.tile_config = (int(tile_config) if tile_config >= 0
                             else int(L.load().vpm_batch_tile_config_default(self.stage_mask)))
         for k, s in enumerate(sets):
@@ -99,7 +101,7 @@ class BatchedSystem:
         off[1:] = np.cumsum(self.sizes)
         self.offsets = off
         self.ws, self.wsb = None, 0
-        self.set_launch(self.tile_config, grid)
+        self.set_launch(self.tile_config, grid, rows)
         e = lambda: torch.zeros((3, n), dtype=torch.float64, device=d)
         self.kx = [e() for _ in range(4)]
         self.ka = [e() for _ in range(4)]
@@ -114,19 +116,22 @@ class BatchedSystem:
         self.steps_done = 0
         self._sorted = False
 
-    def set_launch(self, tile_config, grid=0):
-        """Selects the persistent launch's tile shape and grid: rebuilds the
+    def set_launch(self, tile_config, grid=0, rows=False):
+        """Selects the persistent launch's tile shape and grid, or (``rows``)
+        the row pass, whose items are that shape's target blocks: rebuilds the
         work list (its items are the shape's target blocks) and grows the
         workspace if needed; the sorted order in the workspace is kept.  A
         captured graph is dropped (it holds the old launch)."""
         d = self.device
         self.tile_config = int(tile_config)
         self.grid = int(grid)
+        self.rows = bool(rows)
         if self.precision == "f64":
             tpi = 256
         else:
             b, r = P.tile_configs()[self.tile_config][:2]
             tpi = b * r
+        self.targets_per_item = tpi
         item_set, item_block, first, count = work_list(self.sizes, tpi)
         t = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.int32)).to(d)
         self._desc_t = [t(self.offsets), t(np.repeat(np.arange(self.nsets), self.sizes)),
@@ -185,8 +190,12 @@ class BatchedSystem:
         stretch = self.str_ if stretch is None else stretch
         fo = L.ForwardOut(max(self.n, 1), vel.data_ptr(), stretch.data_ptr(),
                           self.pse_.data_ptr(), self.vort.data_ptr(), self.enstrophy.data_ptr())
-        L.call("vpm_batch_run", C.byref(p), C.byref(self.desc), C.byref(o), C.byref(fo),
-               self.ws.data_ptr(), self.wsb, stream)
+        if self.rows:
+            L.call("vpm_batch_run_rows", C.byref(p), C.byref(self.desc), self.targets_per_item,
+                   C.byref(o), C.byref(fo), self.ws.data_ptr(), self.wsb, stream)
+        else:
+            L.call("vpm_batch_run", C.byref(p), C.byref(self.desc), C.byref(o), C.byref(fo),
+                   self.ws.data_ptr(), self.wsb, stream)
 
     def _axpy(self, x, y, c, out, stream):
         L.call("vpm_axpy3", self.n, max(self.n, 1), x.data_ptr(), y.data_ptr(), float(c),

@@ -1592,15 +1592,17 @@ __global__ __launch_bounds__(256) void set_keys_kernel(const double* __restrict_
 }
 
 // per-set enstrophy: one block per set sums the partials of its items
+// (per_item partials each)
 __global__ __launch_bounds__(256) void set_enstrophy_kernel(const double* __restrict__ part,
                                                             const int* __restrict__ first,
                                                             const int* __restrict__ count,
-                                                            double scale,
+                                                            int per_item, double scale,
                                                             double* __restrict__ out) {
   __shared__ double red[4];
   const int s = blockIdx.x;
   double v = 0.0;
-  for (int k = threadIdx.x; k < count[s]; k += 256) v += part[first[s] + k];
+  const int64_t b = static_cast<int64_t>(first[s]) * per_item;
+  for (int k = threadIdx.x; k < count[s] * per_item; k += 256) v += part[b + k];
   v = block_sum<256>(v, red);
   if (threadIdx.x == 0) out[s] = v * scale;
 }
@@ -1740,8 +1742,10 @@ unsigned batch_mask(unsigned want) {
 
 struct BatchLayout {
   size_t bbox, keys_in, keys_out, idx_in, perm, src8, ens_part, cand, scratch_vec, counter,
-      set_chunk0, far_rec, far_box, cub, total, cub_bytes;
+      set_chunk0, far_rec, far_box, split, cub, total, cub_bytes, split_bytes;
 };
+
+constexpr int kMaxItemRows = 8;  // rows of 64 targets per item (512-target blocks)
 
 int batch_layout(int64_t n, int nsets, int n_items, BatchLayout* L, bool need_cub = true) {
   const size_t N = static_cast<size_t>(n > 0 ? n : 1);
@@ -1757,7 +1761,8 @@ int batch_layout(int64_t n, int nsets, int n_items, BatchLayout* L, bool need_cu
   L->idx_in = take(N * 4);
   L->perm = take(N * 4);
   L->src8 = take(N * sizeof(Src8));
-  L->ens_part = take(static_cast<size_t>(n_items > 0 ? n_items : 1) * sizeof(double));
+  L->ens_part = take(static_cast<size_t>(n_items > 0 ? n_items : 1) * kMaxItemRows *
+                     sizeof(double));
   L->cand = take(N * sizeof(double));
   L->scratch_vec = take(3 * N * sizeof(double));
   L->counter = take(64);
@@ -1765,8 +1770,13 @@ int batch_layout(int64_t n, int nsets, int n_items, BatchLayout* L, bool need_cu
   // chunk per set, plus one group read ahead past the last
   const size_t S = static_cast<size_t>(nsets > 0 ? nsets : 1);
   L->set_chunk0 = take((S + 1) * sizeof(int));
-  L->far_rec = take((N + kMaxFarChunk * S + kFarGroup) * kMaxFarStride * sizeof(float));
-  L->far_box = take((N / kMinFarChunk + S + 1) * 6 * sizeof(double));
+  L->far_rec = take(std::max((N + kMaxFarChunk * S + kFarGroup) * kMaxFarStride * sizeof(float),
+                             row32_batch_record_bytes(n, nsets)));
+  L->far_box = take(std::max((N / kMinFarChunk + S + 1) * 6 * sizeof(double),
+                             row32_batch_box_bytes(n, nsets)));
+  // the row pass's source splits (one row per item is the most it can need)
+  L->split_bytes = row32_batch_split_bytes(n, row32_batch_splits(n, n_items, 1));
+  L->split = take(L->split_bytes);
   size_t cb = 0;
   if (need_cub) {
     hipError_t e = hipcub::DeviceRadixSort::SortPairs(
@@ -2206,9 +2216,12 @@ int vpm_batch_prepare(const vpm_particles_t* p, const vpm_batch_desc_t* d, int r
   return VPM_OK;
 }
 
-int vpm_batch_run(const vpm_particles_t* p, const vpm_batch_desc_t* d, const vpm_forward_opts_t* o,
-                  vpm_forward_out_t* out, void* workspace, size_t ws_bytes, void* stream) {
-  clear_error();
+namespace {
+
+// item_targets: 0 for the tiled kernels, else targets per item of the row pass.
+int batch_run(const vpm_particles_t* p, const vpm_batch_desc_t* d, int item_targets,
+              const vpm_forward_opts_t* o, vpm_forward_out_t* out, void* workspace,
+              size_t ws_bytes, void* stream) {
   int rc = check_desc(d, p, "vpm_batch_run");
   if (rc) return rc;
   if (!o || !out) return fail(VPM_ERR_ARG, "vpm_batch_run: null opts/out");
@@ -2264,18 +2277,51 @@ int vpm_batch_run(const vpm_particles_t* p, const vpm_batch_desc_t* d, const vpm
   b.n_total = static_cast<int>(n);
   b.n_items = d->n_items;
   b.counter = reinterpret_cast<int*>(ws + L.counter);
-  if ((rc = dispatch_batch(b, batch_mask(want), o->precision,
-                           o->tile_config < 0 ? default_batch_config(batch_mask(want))
-                                              : o->tile_config,
-                           d->grid, st)))
+  int per_item = 1;
+  if (item_targets > 0) {
+    per_item = item_targets / 64;
+    b.f.src = b.src;
+    b.f.perm = b.perm;
+    b.f.n = static_cast<int>(n);
+    b.f.part = L.split_bytes ? reinterpret_cast<double*>(ws + L.split) : nullptr;
+    const Row32Batch rows{d->set_off, d->item_set, d->item_block, d->nsets, d->n_items, per_item,
+                          row32_batch_splits(n, d->n_items, per_item),
+                          reinterpret_cast<int*>(ws + L.set_chunk0),
+                          reinterpret_cast<float*>(ws + L.far_rec),
+                          reinterpret_cast<double*>(ws + L.far_box)};
+    if ((rc = row32_batch_run(b.f, rows, batch_mask(want), st))) return rc;
+  } else if ((rc = dispatch_batch(b, batch_mask(want), o->precision,
+                                  o->tile_config < 0 ? default_batch_config(batch_mask(want))
+                                                     : o->tile_config,
+                                  d->grid, st))) {
     return rc;
+  }
   if ((want & VPM_OUT_ENSTROPHY) && d->nsets > 0) {
     const double k = (1.0 / (8.0 * kPi)) * kOneOverFourPi;
     hipLaunchKernelGGL(set_enstrophy_kernel, dim3(d->nsets), dim3(256), 0, st, b.f.ens_part,
-                       d->set_item_first, d->set_item_count, k, out->enstrophy);
+                       d->set_item_first, d->set_item_count, per_item, k, out->enstrophy);
     VPM_LAUNCH_CHECK("set_enstrophy_kernel");
   }
   return VPM_OK;
+}
+
+}  // namespace
+
+int vpm_batch_run(const vpm_particles_t* p, const vpm_batch_desc_t* d, const vpm_forward_opts_t* o,
+                  vpm_forward_out_t* out, void* workspace, size_t ws_bytes, void* stream) {
+  clear_error();
+  return batch_run(p, d, 0, o, out, workspace, ws_bytes, stream);
+}
+
+int vpm_batch_run_rows(const vpm_particles_t* p, const vpm_batch_desc_t* d, int targets_per_item,
+                       const vpm_forward_opts_t* o, vpm_forward_out_t* out, void* workspace,
+                       size_t ws_bytes, void* stream) {
+  clear_error();
+  if (targets_per_item < 64 || targets_per_item > 64 * kMaxItemRows || targets_per_item % 64)
+    return fail(VPM_ERR_ARG, "vpm_batch_run_rows: targets_per_item must be 64, 128, ... 512");
+  if (o && o->precision != VPM_PREC_F32C)
+    return fail(VPM_ERR_UNSUPPORTED, "vpm_batch_run_rows: VPM_PREC_F32C only");
+  return batch_run(p, d, targets_per_item, o, out, workspace, ws_bytes, stream);
 }
 
 int vpm_batch_les_update(const vpm_batch_desc_t* d, int64_t ld, const double* vorticity,

@@ -22,4 +22,25 @@ size_t row32_split_bytes(int64_t n, unsigned mask);
 int row32_run(const FusedArgs& a, unsigned mask, bool unif, float* rec, double* box,
               hipStream_t st, int* nblocks);
 
+// ---- many sets in one launch (vpm_batch_run_rows) ----
+struct Row32Batch {
+  const int* set_off;     // [S + 1]
+  const int* item_set;    // [items]
+  const int* item_block;  // [items] target block of rows_per_item rows
+  int nsets, n_items, rows_per_item, splits;
+  int* chunk0;            // [S + 1] filled here
+  float* rec;
+  double* box;
+};
+
+// Source splits of every row for these items, and the bytes they take.
+int row32_batch_splits(int64_t n, int n_items, int rows_per_item);
+size_t row32_batch_split_bytes(int64_t n, int splits);
+size_t row32_batch_record_bytes(int64_t n, int nsets);
+size_t row32_batch_box_bytes(int64_t n, int nsets);
+
+// a: outputs, src, perm, n (all sets'), ens_part with n_items * rows_per_item
+// slots, part (b.splits > 1).  mask: 3, 7, 27 or 31.
+int row32_batch_run(const FusedArgs& a, const Row32Batch& b, unsigned mask, hipStream_t st);
+
 }  // namespace vpm

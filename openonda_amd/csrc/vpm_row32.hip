@@ -83,14 +83,14 @@ __device__ __forceinline__ double held(double v) {  // rounded here, not fused i
   return v;
 }
 
-// One workgroup per chunk.  Lanes past n write zero-strength padding far
-// away, which adds exactly 0.
+// The records and box of chunk c of a set of n sorted particles, by one
+// workgroup of kChunk lanes; rec and box_ are the set's.  Lanes past n write
+// zero-strength padding far away, which adds exactly 0.
 template <unsigned OUT, bool UNIF>
-__global__ __launch_bounds__((Rec32<OUT, UNIF>::kChunk)) void row32_records_kernel(
-    const Src8* __restrict__ src, int n, float* __restrict__ rec, double* __restrict__ box_) {
+__device__ __forceinline__ void row32_records(const Src8* __restrict__ src, int n, int c,
+                                              float* __restrict__ rec, double* __restrict__ box_) {
   using R = Rec32<OUT, UNIF>;
   __shared__ double red[7][R::kChunk / 64];
-  const int c = blockIdx.x;
   const int k = c * R::kChunk + static_cast<int>(threadIdx.x);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const bool ok = k < n;
@@ -158,6 +158,12 @@ __global__ __launch_bounds__((Rec32<OUT, UNIF>::kChunk)) void row32_records_kern
     r[R::kLoAt + 2] = static_cast<float>(g.az - static_cast<double>(az));
     for (int q = R::kLoAt + 3; q < R::kStride; ++q) r[q] = 0.0f;
   }
+}
+
+template <unsigned OUT, bool UNIF>
+__global__ __launch_bounds__((Rec32<OUT, UNIF>::kChunk)) void row32_records_kernel(
+    const Src8* __restrict__ src, int n, float* __restrict__ rec, double* __restrict__ box) {
+  row32_records<OUT, UNIF>(src, n, static_cast<int>(blockIdx.x), rec, box);
 }
 
 struct Tgt32 {
@@ -313,10 +319,55 @@ __device__ __forceinline__ void pair_far(float* acc, const Tgt32& t, const float
   }
 }
 
-// grid (rows, splits)
-template <unsigned OUT, bool UNIF>
+// Rows of many sets in one launch (24 rings and clouds of 2,048 to 32,768
+// particles, RK4 step with PSE and LES: 29.2 ms with persistent 256-target
+// items, whose one round the largest sets' items outlasted, 17.3 ms here):
+// workgroup w takes row w % rows_per_item of
+// item w / rows_per_item (an item is a target block of a set; the list runs
+// from the largest set to the smallest, and the dispatcher hands out
+// workgroups in that order).  Rows past the set's end leave at once, with a
+// zero enstrophy partial.
+struct Row32Item {
+  int set, off, n, row;
+};
+
+__device__ __forceinline__ bool row32_item(const Row32Batch& b, int w, Row32Item* it) {
+  const int item = w / b.rows_per_item;
+  it->set = b.item_set[item];
+  it->off = b.set_off[it->set];
+  it->n = b.set_off[it->set + 1] - it->off;
+  it->row = b.item_block[item] * b.rows_per_item + w % b.rows_per_item;
+  return it->row * kRow < it->n;
+}
+
+// grid (rows, splits); batched: (items * rows_per_item, splits).  (One kernel
+// with the set picked at its top: as a device function called from two kernels
+// the same body took up to 46 more VGPRs, into scratch.)
+template <unsigned OUT, bool UNIF, bool BATCH>
 __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
-    FusedArgs a, int splits, const float* __restrict__ rec_, const double* __restrict__ box_) {
+    FusedArgs a, Row32Batch b, int splits, const float* __restrict__ rec_,
+    const double* __restrict__ box_) {
+  const int split = static_cast<int>(blockIdx.y);
+  int n = a.n, row = static_cast<int>(blockIdx.x);
+  const Src8* src = a.src;
+  const int* perm = a.perm;
+  double* part_out =
+      a.part ? a.part + static_cast<int64_t>(split) * Slots<OUT>::nslot * a.pld : nullptr;
+  if constexpr (BATCH) {
+    Row32Item it;
+    if (!row32_item(b, row, &it)) {
+      if (threadIdx.x == 0 && split == 0) a.ens_part[row] = 0.0;
+      return;
+    }
+    const int64_t c0 = b.chunk0[it.set];
+    rec_ = b.rec + c0 * Rec32<OUT, UNIF>::kChunk * Rec32<OUT, UNIF>::kStride;
+    box_ = b.box + c0 * kBox32;
+    n = it.n;
+    row = it.row;
+    src += it.off;
+    perm += it.off;
+    if (part_out) part_out += it.off;
+  }
   using S = Slots<OUT>;
   using R = Rec32<OUT, UNIF>;
   constexpr int NS = S::nslot, CH = R::kChunk;
@@ -325,12 +376,11 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
   __shared__ double tot[kRowWaves][NS][kRow];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int row = blockIdx.x;
   const int kt = row * kRow + lane;
-  const bool valid = kt < a.n;
-  const double scale = 1.0 / a.src[0].s;
+  const bool valid = kt < n;
+  const double scale = 1.0 / src[0].s;
   Src8 ti{0, 0, 0, 0, 0, 0, 1, 0};
-  if (valid) ti = a.src[kt];
+  if (valid) ti = src[kt];
   const double X = held(ti.x * scale), Y = held(ti.y * scale), Z = held(ti.z * scale);
   Tgt32 t;
   t.ax = static_cast<float>(ti.ax);
@@ -340,8 +390,14 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
   t.lx = static_cast<float>(ti.ax - static_cast<double>(t.ax));
   t.ly = static_cast<float>(ti.ay - static_cast<double>(t.ay));
   t.lz = static_cast<float>(ti.az - static_cast<double>(t.az));
-  const double ai[3] = {ti.ax, ti.ay, ti.az};
   const float eps = static_cast<float>(kEpsPair * scale * scale);
+  // The target's FP64 record is read again where it is needed (FP64 chunks,
+  // the epilogue) instead of staying in registers through the sweep.
+  auto target = [&]() {
+    int k = valid ? kt : row * kRow;
+    asm volatile("" : "+v"(k));
+    return src[k];
+  };
 
   // stretching: G mode, and the row's box for the far test
   bool g64 = false;
@@ -372,12 +428,12 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
   PairConst<float> kc{1.5f, 7.5f, 2.2f, 3.0f, 2.5f};  // in VGPRs (see PairConst)
   asm volatile("" : "+v"(kc.c15), "+v"(kc.c75), "+v"(kc.c22), "+v"(kc.c3), "+v"(kc.c25));
 
-  const int nchunk = (a.n + CH - 1) / CH;
+  const int nchunk = (n + CH - 1) / CH;
   const int parts = splits * kRowWaves;
   const int own = row * kRow / CH;          // the chunk that holds the row
   uint64_t near = 0;                        // this wave's next 64 chunks near the row
   int seen = 0;
-  for (int c = static_cast<int>(blockIdx.y) * kRowWaves + wave; c < nchunk; c += parts, ++seen) {
+  for (int c = split * kRowWaves + wave; c < nchunk; c += parts, ++seen) {
     bool is_near = true;
     if constexpr (S::str) {
       // far tests for 64 of the wave's chunks at a time, one per lane
@@ -441,11 +497,13 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
     if (S::str && (fp64 || c == own)) {
       if constexpr (S::str) {
         // near chunks of FP64 rows, and the row's own chunk: valid sources only
-        const int cnt = a.n - j0 < CH ? a.n - j0 : CH;
+        const int cnt = n - j0 < CH ? n - j0 : CH;
         const int self = c == own ? lane + (row * kRow - j0) : -1;
         const scalar_double_t* str =
-            (const scalar_double_t*)(reinterpret_cast<const double*>(a.src + j0));
+            (const scalar_double_t*)(reinterpret_cast<const double*>(src + j0));
         if (fp64) {
+          const Src8 tr = target();
+          const double ai[3] = {tr.ax, tr.ay, tr.az};
 #pragma unroll R::kNear
           for (int q = 0; q < cnt; ++q) {
             float f[R::kStride];
@@ -458,13 +516,13 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
           for (int q = 0; q < cnt; ++q) {
             float f[R::kStride];
             load1(f, q);
-            pair32<OUT, UNIF, false>(part, g64s, t, f, nullptr, ai, eps, kc, q == self);
+            pair32<OUT, UNIF, false>(part, g64s, t, f, nullptr, nullptr, eps, kc, q == self);
           }
         }
       }
     } else if (!R::kMoment || is_near) {
       stream([&](const float* f) {
-        pair32<OUT, UNIF, false>(part, g64s, t, f, nullptr, ai, eps, kc, false);
+        pair32<OUT, UNIF, false>(part, g64s, t, f, nullptr, nullptr, eps, kc, false);
       });
     } else if constexpr (R::kMoment) {
       constexpr float es = R::kE3 ? 3.0f : 1.0f;
@@ -508,12 +566,12 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
     double s = 0.0;
 #pragma unroll
     for (int w = 0; w < kRowWaves; ++w) s += tot[w][q][lane];
-    if (a.part)
-      a.part[(static_cast<int64_t>(blockIdx.y) * NS + q) * a.pld + kt] = s;
-    else
+    if (!part_out)
       tot[0][q][lane] = s;  // slot q is read by this wave only, above
+    else if (valid)
+      part_out[q * a.pld + kt] = s;
   }
-  if (a.part) return;
+  if (part_out) return;
   __syncthreads();
   if (wave != 0) return;
   double T[kNAcc], G[3] = {0.0, 0.0, 0.0};
@@ -524,10 +582,85 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
     for (int q = 0; q < 3; ++q) G[q] = tot[0][S::nacc + q][lane];
   }
   double ens = 0.0;
-  if (valid) ens = store_target<OUT, true>(a, ti, a.perm ? a.perm[kt] : kt, T, G, scale);
+  if (valid) ens = store_target<OUT, true>(a, target(), perm ? perm[kt] : kt, T, G, scale);
   if constexpr (S::ens) {
     ens = wave_sum(ens);
-    if (lane == 0) a.ens_part[row] = ens;
+    if (lane == 0) a.ens_part[blockIdx.x] = ens;
+  }
+}
+
+// set_chunk0[s] = chunks of the sets before s; set_chunk0[S] = all.
+__global__ __launch_bounds__(1024) void row32_chunks_kernel(const int* __restrict__ off, int nsets,
+                                                            int ch, int* __restrict__ chunk0) {
+  __shared__ int part[1024];
+  const int t = threadIdx.x;
+  const int per = (nsets + 1023) / 1024;
+  const int b = min(nsets, t * per), e = min(nsets, b + per);
+  int sum = 0;
+  for (int s = b; s < e; ++s) sum += (off[s + 1] - off[s] + ch - 1) / ch;
+  part[t] = sum;
+  __syncthreads();
+  for (int d = 1; d < 1024; d <<= 1) {  // inclusive scan
+    const int v = t >= d ? part[t - d] : 0;
+    __syncthreads();
+    part[t] += v;
+    __syncthreads();
+  }
+  int acc = part[t] - sum;
+  for (int s = b; s < e; ++s) {
+    chunk0[s] = acc;
+    acc += (off[s + 1] - off[s] + ch - 1) / ch;
+  }
+  if (t == 1023) chunk0[nsets] = part[1023];
+}
+
+// Workgroup g builds chunk g of all sets' chunks (its set by binary search).
+template <unsigned OUT>
+__global__ __launch_bounds__((Rec32<OUT, true>::kChunk)) void row32_set_records_kernel(
+    Row32Batch b, const Src8* __restrict__ src) {
+  using R = Rec32<OUT, true>;
+  const int g = blockIdx.x;
+  if (g >= b.chunk0[b.nsets]) return;  // uniform over the workgroup
+  int lo = 0, hi = b.nsets - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) / 2;
+    if (b.chunk0[mid] <= g) lo = mid;
+    else hi = mid - 1;
+  }
+  const int off = b.set_off[lo];
+  const int64_t c0 = b.chunk0[lo];
+  row32_records<OUT, true>(src + off, b.set_off[lo + 1] - off, g - static_cast<int>(c0),
+                           b.rec + c0 * R::kChunk * R::kStride, b.box + c0 * kBox32);
+}
+
+// Adds the splits of a row in order and stores.  grid (items * rows_per_item)
+template <unsigned OUT>
+__global__ __launch_bounds__(kRow) void row32_batch_reduce_kernel(FusedArgs a, Row32Batch b,
+                                                                  int splits) {
+  using S = Slots<OUT>;
+  const int w = static_cast<int>(blockIdx.x);
+  Row32Item it;
+  if (!row32_item(b, w, &it)) return;
+  const int kt = it.row * kRow + static_cast<int>(threadIdx.x);
+  double ens = 0.0;
+  if (kt < it.n) {
+    const int64_t k = static_cast<int64_t>(it.off) + kt;
+    double T[kNAcc], G[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < kNAcc; ++q) T[q] = 0.0;
+    for (int sp = 0; sp < splits; ++sp) {
+      const double* P = a.part + static_cast<int64_t>(sp) * S::nslot * a.pld;
+#pragma unroll
+      for (int q = 0; q < kNAcc; ++q)
+        if (S::used(q)) T[q] += P[S::packed(q) * a.pld + k];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) G[c] += P[(S::nacc + c) * a.pld + k];
+    }
+    ens = store_target<OUT, true>(a, a.src[k], a.perm[k], T, G, 1.0 / a.src[it.off].s);
+  }
+  if constexpr (S::ens) {
+    ens = wave_sum(ens);
+    if (threadIdx.x == 0) a.ens_part[w] = ens;
   }
 }
 
@@ -552,8 +685,8 @@ int launch(FusedArgs a, float* rec, double* box, hipStream_t st, int* nblocks) {
   hipLaunchKernelGGL((row32_records_kernel<OUT, UNIF>), dim3(chunks), dim3(R::kChunk), 0, st,
                      a.src, a.n, rec, box);
   VPM_LAUNCH_CHECK("row32_records_kernel");
-  hipLaunchKernelGGL((row32_kernel<OUT, UNIF>), dim3(rows, k), dim3(kRowBlock), 0, st, a, k, rec,
-                     box);
+  hipLaunchKernelGGL((row32_kernel<OUT, UNIF, false>), dim3(rows, k), dim3(kRowBlock), 0, st, a,
+                     Row32Batch{}, k, rec, box);
   VPM_LAUNCH_CHECK("row32_kernel");
   *nblocks = rows;
   if (k > 1) {
@@ -561,6 +694,32 @@ int launch(FusedArgs a, float* rec, double* box, hipStream_t st, int* nblocks) {
     hipLaunchKernelGGL((split_reduce_kernel<OUT, true>), dim3(rb), dim3(256), 0, st, a, k);
     VPM_LAUNCH_CHECK("split_reduce_kernel");
     *nblocks = rb;
+  }
+  return VPM_OK;
+}
+
+template <unsigned OUT>
+int launch_batch(FusedArgs a, const Row32Batch& b, hipStream_t st) {
+  using R = Rec32<OUT, true>;
+  const int64_t groups = static_cast<int64_t>(b.n_items) * b.rows_per_item;
+  if (groups == 0 || a.n == 0) return VPM_OK;
+  const int k = a.part ? b.splits : 1;
+  if (k == 1) a.part = nullptr;
+  a.pld = a.n;
+  hipLaunchKernelGGL(row32_chunks_kernel, dim3(1), dim3(1024), 0, st, b.set_off, b.nsets,
+                     R::kChunk, b.chunk0);
+  VPM_LAUNCH_CHECK("row32_chunks_kernel");
+  const int64_t chunks = ceil_div(a.n, R::kChunk) + b.nsets;  // bound; extra groups leave
+  hipLaunchKernelGGL(row32_set_records_kernel<OUT>, dim3(static_cast<unsigned>(chunks)),
+                     dim3(R::kChunk), 0, st, b, a.src);
+  VPM_LAUNCH_CHECK("row32_set_records_kernel");
+  hipLaunchKernelGGL((row32_kernel<OUT, true, true>), dim3(static_cast<unsigned>(groups), k),
+                     dim3(kRowBlock), 0, st, a, b, k, nullptr, nullptr);
+  VPM_LAUNCH_CHECK("row32_kernel");
+  if (k > 1) {
+    hipLaunchKernelGGL(row32_batch_reduce_kernel<OUT>, dim3(static_cast<unsigned>(groups)),
+                       dim3(kRow), 0, st, a, b, k);
+    VPM_LAUNCH_CHECK("row32_batch_reduce_kernel");
   }
   return VPM_OK;
 }
@@ -598,6 +757,36 @@ int row32_run(const FusedArgs& a, unsigned mask, bool unif, float* rec, double* 
 #undef VPM_ROW32
     default:
       return fail(VPM_ERR_ARG, "row32: output set has the far-field moment form");
+  }
+}
+
+int row32_batch_splits(int64_t n, int n_items, int rows_per_item) {
+  // Rows of equal sets run in rounds of 768 workgroups; unequal ones, largest
+  // first, need a few rounds' worth to end together.
+  const int64_t rows = std::min<int64_t>(static_cast<int64_t>(n_items) * rows_per_item,
+                                         ceil_div(n, kRow) + n_items);
+  return static_cast<int>(std::clamp<int64_t>(3 * 768 / std::max<int64_t>(rows, 1), 1, 8));
+}
+
+size_t row32_batch_split_bytes(int64_t n, int splits) {
+  return splits > 1 ? static_cast<size_t>(splits) * nslots(31u) * n * sizeof(double) : 0;
+}
+
+size_t row32_batch_record_bytes(int64_t n, int nsets) {
+  return (static_cast<size_t>(n) + static_cast<size_t>(kMaxChunk32) * nsets + kMaxGroup32) *
+         kStride32 * sizeof(float);
+}
+
+size_t row32_batch_box_bytes(int64_t n, int nsets) {
+  return (static_cast<size_t>(n) / kMinChunk32 + nsets + 1) * kBox32 * sizeof(double);
+}
+
+int row32_batch_run(const FusedArgs& a, const Row32Batch& b, unsigned mask, hipStream_t st) {
+  switch (mask) {
+    case 3u: return launch_batch<3u>(a, b, st);
+    case 7u: return launch_batch<7u>(a, b, st);
+    case 27u: return launch_batch<27u>(a, b, st);
+    default: return launch_batch<31u>(a, b, st);
   }
 }
 
