@@ -31,6 +31,9 @@ struct OpForward {
   static constexpr bool kTargetData = true, kRadius = !UNIF, kNu = pse, kSkipSelf = true;
   static constexpr bool kSum = ens, kSelfTerm = ens;
   static constexpr int kOut = 3 * (vel + str + pse + vort);
+  // The set of a solver step with the plain kernels' arithmetic takes the
+  // stretching's sum as they do: a_i x sum g (a_j - a_i) (vpm_plain.hip).
+  static constexpr bool kDelta = OUT == (VPM_OUT_STRETCH | VPM_OUT_VORT | VPM_OUT_ENSTROPHY);
   struct Acc {
     double u[3] = {0, 0, 0}, g[3] = {0, 0, 0}, s[3] = {0, 0, 0}, p[3] = {0, 0, 0},
            w[3] = {0, 0, 0}, e[3] = {0, 0, 0};
@@ -65,9 +68,9 @@ struct OpForward {
         a.u[2] = fma(g, cz, a.u[2]);
       }
       if constexpr (str) {
-        a.g[0] = fma(g, s.ax, a.g[0]);
-        a.g[1] = fma(g, s.ay, a.g[1]);
-        a.g[2] = fma(g, s.az, a.g[2]);
+        a.g[0] = fma(g, kDelta ? s.ax - t.ax : s.ax, a.g[0]);
+        a.g[1] = fma(g, kDelta ? s.ay - t.ay : s.ay, a.g[1]);
+        a.g[2] = fma(g, kDelta ? s.az - t.az : s.az, a.g[2]);
         const double e = fma(t.ax, cx, fma(t.ay, cy, t.az * cz));
         const double f = ((t2 * t1) * t2) * fma(7.5, w, 3.0) * e;
         a.s[0] = fma(f, rx, a.s[0]);
@@ -188,7 +191,8 @@ int forward_rows(const vpm_particles_t* p, const vpm_forward_opts_t* o, vpm_forw
 #define VPM_ROWS(M) \
   case M: return launch_mode<M>(p, o, out, ens_part, split, split_bytes, st);
     VPM_ROWS(1u) VPM_ROWS(2u) VPM_ROWS(3u) VPM_ROWS(4u) VPM_ROWS(7u) VPM_ROWS(8u) VPM_ROWS(16u)
-    VPM_ROWS(24u) VPM_ROWS(27u)
+    VPM_ROWS(24u) VPM_ROWS(26u)
+    VPM_ROWS(27u)
 #undef VPM_ROWS
     default: return launch_mode<31u>(p, o, out, ens_part, split, split_bytes, st);
   }

@@ -1329,6 +1329,14 @@ unsigned kernel_mask(unsigned want) {
   return 31u;
 }
 
+// The row passes also have the solver step's stretching + vorticity +
+// enstrophy.
+unsigned row_mask(unsigned want) {
+  constexpr unsigned step = VPM_OUT_STRETCH | VPM_OUT_VORT | VPM_OUT_ENSTROPHY;
+  const unsigned m = kernel_mask(want);
+  return (want & ~step) == 0 && m == 27u ? step : m;
+}
+
 int dispatch(const FusedArgs& a, unsigned mask, bool unif, int cfg, hipStream_t st, int* nb) {
   switch (mask) {
     case 1u: return launch_mask<1u>(a, unif, cfg, st, nb);
@@ -1374,8 +1382,8 @@ int split_slots(unsigned mask) {
 // Room for the largest source split launch_cfg may choose for this call.
 size_t split_capacity(int64_t n, const vpm_forward_opts_t* o) {
   if (!o || n <= 0) return 0;
-  if (forward_rows_wanted(n, o)) return forward_rows_split_bytes(n, kernel_mask(o->outputs));
-  if (row32_asked(o)) return row32_split_bytes(n, kernel_mask(o->outputs));
+  if (forward_rows_wanted(n, o)) return forward_rows_split_bytes(n, row_mask(o->outputs));
+  if (row32_asked(o)) return row32_split_bytes(n, row_mask(o->outputs));
   const int c = effective_config(kernel_mask(o->outputs), o->sigma_mode == VPM_SIGMA_UNIFORM,
                                  o->tile_config < kNumCfgs ? o->tile_config : -1);
   const int br = kCfgs[c].block * kCfgs[c].r, tile = kCfgs[c].tile;
@@ -1955,7 +1963,8 @@ int forward_run_impl(const vpm_particles_t* p, const vpm_forward_opts_t* o,
     }
     return VPM_OK;
   }
-  const unsigned mask = kernel_mask(want);
+  const unsigned mask = forward_rows_wanted(n, o) || row32_asked(o) ? row_mask(want)
+                                                                     : kernel_mask(want);
   if (forward_rows_wanted(n, o))
     return forward_rows(p, o, out, mask, reinterpret_cast<double*>(ws + L.ens_part),
                         L.split_bytes ? ws + L.split : nullptr, L.split_bytes, st);

@@ -750,10 +750,10 @@ int row32_run(const FusedArgs& a, unsigned mask, bool unif, float* rec, double* 
     return launch<M, U>(a, rec, box, st, nblocks);
     VPM_ROW32(1u, true) VPM_ROW32(2u, true) VPM_ROW32(3u, true) VPM_ROW32(4u, true)
     VPM_ROW32(7u, true) VPM_ROW32(8u, true) VPM_ROW32(16u, true) VPM_ROW32(24u, true)
-    VPM_ROW32(27u, true) VPM_ROW32(31u, true)
+    VPM_ROW32(26u, true) VPM_ROW32(27u, true) VPM_ROW32(31u, true)
     VPM_ROW32(1u, false) VPM_ROW32(2u, false) VPM_ROW32(3u, false) VPM_ROW32(4u, false)
     VPM_ROW32(7u, false) VPM_ROW32(8u, false) VPM_ROW32(16u, false) VPM_ROW32(24u, false)
-    VPM_ROW32(27u, false) VPM_ROW32(31u, false)
+    VPM_ROW32(26u, false) VPM_ROW32(27u, false) VPM_ROW32(31u, false)
 #undef VPM_ROW32
     default:
       return fail(VPM_ERR_ARG, "row32: output set has the far-field moment form");

@@ -15,7 +15,7 @@ from openonda_amd import physics as P
 pytestmark = pytest.mark.gpu
 
 TOL = 1e-6
-UNIFORM = [("vel",), ("stretch",), ("pse",), ("vort",), ("enstrophy",), ("vort", "enstrophy"),
+UNIFORM = [("stretch", "vort", "enstrophy"), ("vel",), ("stretch",), ("pse",), ("vort",), ("enstrophy",), ("vort", "enstrophy"),
            ("vel", "stretch"), ("vel", "stretch", "pse"), ("vel", "stretch", "vort", "enstrophy"),
            ("vel", "stretch", "pse", "vort", "enstrophy")]
 GENERAL = UNIFORM

@@ -171,7 +171,7 @@ def test_non_finite_inputs_carry_on_as_in_the_reference(gpu):
     assert np.isfinite(P.from_soa(P.selfinduced_velocity(dx, da, ds))).all()
 
 
-OUTS = [("vel",), ("stretch",), ("vel", "stretch"), ("pse",), ("vort",), ("enstrophy",),
+OUTS = [("stretch", "vort", "enstrophy"), ("vel",), ("stretch",), ("vel", "stretch"), ("pse",), ("vort",), ("enstrophy",),
         ("vel", "stretch", "pse"), ("vort", "enstrophy"), ("vel", "stretch", "vort", "enstrophy"),
         ("vel", "pse"), ("vel", "stretch", "pse", "vort", "enstrophy")]
 
