@@ -50,6 +50,7 @@ PRECISION = "plain"
 # radius <= 0 or a viscosity < 0 raises NonFiniteError (status
 # VPM_ERR_NONFINITE) instead of returning NaN as the reference does.
 CHECK_FINITE = True
+_PINNED_BYTES = 4 << 20
 
 
 def _arr(a, name, cols=3, bad=0):
@@ -80,10 +81,6 @@ def _dev():
     return torch.device("cuda", torch.cuda.current_device())
 
 
-def _soa(a, dev):
-    return torch.from_numpy(np.ascontiguousarray(a.T)).to(dev)
-
-
 def _src(x, a, s, nu=None, targets=None):
     """Validates every array on the host (before any GPU call), then uploads:
     returns ([targets,] x, a, s[, nu]) as device tensors."""
@@ -99,11 +96,24 @@ def _src(x, a, s, nu=None, targets=None):
         if nu.shape[0] != n:
             raise ValueError("viscosities must have the same length as positions")
     dev = _dev()
-    out = [_soa(x, dev), _soa(a, dev), torch.from_numpy(np.ascontiguousarray(s)).to(dev)]
+    # One host buffer and one copy: positions, strengths, radii[, viscosities].
+    # Three pageable copies took 50 us at 1,000 particles, one from pinned
+    # memory 14 (8,192: 56 and 26); large sets stay pageable, so that torch's
+    # pinned-memory cache stays small.
+    k = 7 if nu is None else 8
+    buf = torch.empty((k, n), dtype=torch.float64, pin_memory=0 < k * n * 8 <= _PINNED_BYTES)
+    rows = buf.numpy()
+    rows[0:3] = x.T
+    rows[3:6] = a.T
+    rows[6] = s
     if nu is not None:
-        out.append(torch.from_numpy(np.ascontiguousarray(nu)).to(dev))
+        rows[7] = nu
+    d = buf.to(dev, non_blocking=True)
+    out = [d[0:3], d[3:6], d[6]]
+    if nu is not None:
+        out.append(d[7])
     if y is not None:
-        out.insert(0, _soa(y, dev))
+        out.insert(0, torch.from_numpy(np.ascontiguousarray(y.T)).to(dev))
     return out
 
 
