@@ -22,7 +22,8 @@
 // Sums over j of g a_j, g lam_j and f phi a_j are accumulated per target and
 // crossed with the target's vectors once; the three radial terms share one
 // accumulator.
-// Precision F32C runs the rows of vpm_adj32.hip; the kernels here are F64's.
+// Precision F32C runs the rows of vpm_adj32.hip above kAdjRowsMax particles,
+// F64 and smaller sets the FP64 rows here.
 
 #include <algorithm>
 #include <type_traits>
@@ -36,489 +37,252 @@ namespace vpm {
 
 namespace {
 
-// Sorted SoA arrays of the adjoint pass (workspace), component c of particle
-// k at base[c * n + k].
-struct AdjSorted {
-  const double* pos;   // [3][n]
-  const double* str;   // [3][n]
-  const double* lam;   // [3][n]
-  const double* mu;    // [3][n]
-  const double* z;     // [3][n] nu * xi
-  const double* sig;   // [n]
-  const double* nu;    // [n]
-};
+// ---- FP64 rows (vpm_rows.h): any subset of the cotangents, sigma_ij ------
+// The lengths are not scaled: sc = 1 in the formulas above.  Per pair
+//   k = lam_j x r - Q_j,  E = lam_m.c - a_m.k + a_j.P_m,
+// G = sum g a_j, Lam = sum g lam_j, A = sum g k + 105 p (z_j - z_m),
+// B = sum f phi c, X = sum [f E - 2 h psi phi + 945 q (a_j - a_m).(z_j - z_m)] r,
+// Y = sum f phi a_j, D = sum f psi (mu_m - mu_j); then
+//   dA = C (A + G x mu_m + B),  dX = C (X - G x lam_m + a_m x Lam + Y x a_m + D).
+// The pair j = m is left out: its terms cancel or vanish.
+//
+// Bound by FP64 issue (about 95 instructions per pair with all three
+// cotangents).  One rsq64 per pair in place of an IEEE square root and
+// division, the sums G, Lam, Y, D crossed once per particle, the sources as
+// scalar operands and rows of 64 in place of blocks of 256: all cotangents,
+// general radius, 1,000 particles 483 -> 29 us, 10,007 825 -> 369 us, 50,021
+// 13.7 -> 8.0 ms.
 
-__global__ __launch_bounds__(256) void adj_gather_kernel(vpm_particles_t p, const double* __restrict__ lam,
-                                                         const double* __restrict__ mu,
-                                                         const double* __restrict__ xi, int64_t ldc,
-                                                         int n, const int* __restrict__ perm,
-                                                         double* __restrict__ out) {
-  const int k = blockIdx.x * 256 + threadIdx.x;
-  if (k >= n) return;
-  const int i = perm ? perm[k] : k;
-  const int64_t N = n;
-  double* pos = out;
-  double* str = out + 3 * N;
-  double* la = out + 6 * N;
-  double* m = out + 9 * N;
-  double* z = out + 12 * N;
-  double* sg = out + 15 * N;
-  double* nu = out + 16 * N;
-  const double nui = p.nu ? p.nu[i] : 0.0;
+// Record of one particle, in the caller's order: x 0, a 3, lam 6, mu 9,
+// z = nu xi 12, Q = a x mu 15, sigma 18.
+constexpr int kRec64 = 20;
+
+__global__ __launch_bounds__(256) void adj64_records_kernel(vpm_particles_t p,
+                                                            const double* __restrict__ lam,
+                                                            const double* __restrict__ mu,
+                                                            const double* __restrict__ xi,
+                                                            int64_t ldc, double* __restrict__ rec) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= p.n) return;
+  double* r = rec + i * kRec64;
+  const double nu = xi ? p.nu[i] : 0.0;
+  double a[3], m[3];
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    pos[c * N + k] = p.pos[c * p.ld + i];
-    str[c * N + k] = p.str[c * p.ld + i];
-    la[c * N + k] = lam ? lam[c * ldc + i] : 0.0;
-    m[c * N + k] = mu ? mu[c * ldc + i] : 0.0;
-    z[c * N + k] = xi ? nui * xi[c * ldc + i] : 0.0;
+    a[c] = p.str[c * p.ld + i];
+    m[c] = mu ? mu[c * ldc + i] : 0.0;
+    r[c] = p.pos[c * p.ld + i];
+    r[3 + c] = a[c];
+    r[6 + c] = lam ? lam[c * ldc + i] : 0.0;
+    r[9 + c] = m[c];
+    r[12 + c] = xi ? nu * xi[c * ldc + i] : 0.0;
   }
-  sg[k] = p.sigma[i];
-  nu[k] = nui;
+  r[15] = a[1] * m[2] - a[2] * m[1];
+  r[16] = a[2] * m[0] - a[0] * m[2];
+  r[17] = a[0] * m[1] - a[1] * m[0];
+  r[18] = p.sigma[i];
+  r[19] = 0.0;
 }
 
-template <typename Real>
-struct Ar;
-template <>
-struct Ar<float> {
-  static __device__ inline float rsq(float a) { return __builtin_amdgcn_rsqf(a); }
-  static __device__ inline float rcp(float a) { return __builtin_amdgcn_rcpf(a); }
-};
-template <>
-struct Ar<double> {
-  static __device__ inline double rsq(double a) { return 1.0 / sqrt(a); }
-  static __device__ inline double rcp(double a) { return 1.0 / a; }
+struct Adj64Acc {
+  double G[3], L[3], A[3], B[3], X[3], Y[3], D[3];
 };
 
-// LDS record of one partner.
-template <typename Real>
-struct alignas(16) AdjSrc {
-  Real x, y, z, ax, ay, az, lx, ly, lz, mx, my, mz, qx, qy, qz, zx, zy, zz, hs, pad;
-};
+__device__ __forceinline__ double dot3(const double* a, const double* b, double c) {
+  return ::fma(a[2], b[2], ::fma(a[1], b[1], ::fma(a[0], b[0], c)));
+}
+__device__ __forceinline__ void add3(double* s, double w, const double* v) {
+  s[0] = ::fma(w, v[0], s[0]);
+  s[1] = ::fma(w, v[1], s[1]);
+  s[2] = ::fma(w, v[2], s[2]);
+}
+__device__ __forceinline__ void add_cross(double* o, const double* a, const double* b) {
+  o[0] = ::fma(-a[2], b[1], ::fma(a[1], b[2], o[0]));
+  o[1] = ::fma(-a[0], b[2], ::fma(a[2], b[0], o[1]));
+  o[2] = ::fma(-a[1], b[0], ::fma(a[0], b[1], o[2]));
+}
 
-template <typename Real>
-struct AdjTgt {
-  Real x, y, z, ax, ay, az, lx, ly, lz, mx, my, mz, px, py, pz, zx, zy, zz, hs;
-};
-
-// Accumulator slots (per target).  Terms with the same sigma scaling share
-// an accumulator; sc = 1/sigma with a uniform radius (offsets pre-scaled),
-// 1 otherwise (per-pair 1/sigma_ij powers folded into g, f, h, p, q):
-//   aG = sum g a_j, aL = sum g lam_j                      (crossed in the epilogue)
-//   aA = sum g (lam_j x r) + 105 p (z_j - z_m)            dA, scale C/s^2
-//   aB = sum f phi c - g Q_j                              dA, scale C/s^3
-//   aX = sum [f e + sc (f dw - 2 h psi phi) + 945 q dd] r dX, scale C/s^3
-//        with dd = (a_j - a_m).(z_j - z_m)
-//   aY = sum f phi a_j,  aD = sum f psi d_mu              dX, scale C/s^4
-enum : int { aG = 0, aL = 3, aA = 6, aB = 9, aX = 12, aY = 15, aD = 18, aN = 21 };
-
+// t: the target's record (half its radius at 18), s: the source's.
 template <unsigned OUT>
-struct AdjSlots {
-  static constexpr bool vel = OUT & VPM_OUT_VEL, str = OUT & VPM_OUT_STRETCH,
-                        pse = OUT & VPM_OUT_PSE;
-  static __host__ __device__ constexpr bool used(int k) {
-    return (k < 3 && (vel || str)) || (k >= 3 && k < 6 && vel) ||
-           (k >= 6 && k < 9 && (vel || pse)) || (k >= 9 && k < 12 && str) ||
-           (k >= 12 && k < 15) || (k >= 15 && str);
-  }
-  // position of slot k among the used ones (the split partial layout)
-  static __host__ __device__ constexpr int packed(int k) {
-    int c = 0;
-    for (int q = 0; q < k; ++q) c += used(q) ? 1 : 0;
-    return c;
-  }
-  static constexpr int nslot = packed(aN);
-};
-
-// Non-inline constants of the pair terms, kept in registers by the caller
-// (literal operands halve an instruction's issue rate on gfx950).
-template <typename Real>
-struct AdjConst {
-  Real c15, c3, c75, c2625, c105, c945;
-};
-
-template <typename Real, unsigned OUT, bool UNIF>
-__device__ __forceinline__ void adj_pair(Real* acc, const AdjTgt<Real>& t, const AdjSrc<Real>& s,
-                                         Real sc, const AdjConst<Real>& k) {
-  using S = AdjSlots<OUT>;
-  using M = Ar<Real>;
-  const Real dx = t.x - s.x, dy = t.y - s.y, dz = t.z - s.z;
-  Real A, inv = Real(1), inv2 = Real(1);
-  if constexpr (UNIF) {
-    A = dz * dz + (dy * dy + (dx * dx + Real(1)));
-  } else {
-    inv = M::rcp(t.hs + s.hs);
-    inv2 = inv * inv;
-    A = (dx * dx + dy * dy + dz * dz) * inv2 + Real(1);
-  }
-  // A t^2 = 1: each factor (rho^2 + c) t^k is written in powers of t alone
-  const Real t1 = M::rsq(A);
-  const Real t2 = t1 * t1;
-  const Real t3 = t2 * t1;
-  const Real t5 = t3 * t2;
-  const Real t7 = t5 * t2;
-  Real xc = Real(0);  // radial coefficient of aX
-  if constexpr (S::vel || S::str) {
-    Real g = k.c15 * t5 + t3;                        // (rho^2 + 2.5) t^5
-    Real f = t5 * (k.c75 * t2 + k.c3);               // 3 (rho^2 + 3.5) t^7
-    if constexpr (!UNIF) {
-      const Real inv3 = inv2 * inv;
-      g *= inv3;
-      f *= inv3 * inv2;
+__device__ __forceinline__ void adj64_pair(Adj64Acc& acc, const double* t, const double* s) {
+  constexpr bool vel = OUT & VPM_OUT_VEL, str = OUT & VPM_OUT_STRETCH, pse = OUT & VPM_OUT_PSE;
+  const double d[3] = {t[0] - s[0], t[1] - s[1], t[2] - s[2]};
+  const double sg = ::fma(0.5, s[18], t[18]);
+  const double s2 = sg * sg;
+  const double D = dot3(d, d, s2);
+  const double t1 = (vel || str) ? rsq64(D) : rsq64_inf(D);
+  const double t2 = t1 * t1, t3 = t2 * t1, w = s2 * t2;
+  const double *a = s + 3, *l = s + 6, *m = s + 9, *z = s + 12, *Q = s + 15;
+  double xc = 0.0;
+  if constexpr (vel || str) {
+    const double t5 = t3 * t2;
+    const double g = t3 * ::fma(1.5, w, 1.0);
+    const double f = t5 * ::fma(7.5, w, 3.0);
+    const double c[3] = {d[1] * a[2] - d[2] * a[1], d[2] * a[0] - d[0] * a[2],
+                         d[0] * a[1] - d[1] * a[0]};
+    double k[3] = {0.0, 0.0, 0.0}, E = 0.0;
+    add3(acc.G, g, a);
+    if constexpr (vel) {
+      k[0] = l[1] * d[2] - l[2] * d[1];
+      k[1] = l[2] * d[0] - l[0] * d[2];
+      k[2] = l[0] * d[1] - l[1] * d[0];
+      add3(acc.L, g, l);
+      E = dot3(t + 6, c, 0.0);
     }
-    const Real cx = dy * s.az - dz * s.ay;            // c = r x a_j
-    const Real cy = dz * s.ax - dx * s.az;
-    const Real cz = dx * s.ay - dy * s.ax;
-    acc[aG + 0] += g * s.ax;
-    acc[aG + 1] += g * s.ay;
-    acc[aG + 2] += g * s.az;
-    if constexpr (S::vel) {
-      const Real kx = s.ly * dz - s.lz * dy;          // lam_j x r
-      const Real ky = s.lz * dx - s.lx * dz;
-      const Real kz = s.lx * dy - s.ly * dx;
-      acc[aA + 0] += g * kx;
-      acc[aA + 1] += g * ky;
-      acc[aA + 2] += g * kz;
-      acc[aL + 0] += g * s.lx;
-      acc[aL + 1] += g * s.ly;
-      acc[aL + 2] += g * s.lz;
-      const Real e = (t.lx * cx + t.ly * cy + t.lz * cz) - (t.ax * kx + t.ay * ky + t.az * kz);
-      xc = f * e;
+    if constexpr (str) {
+      k[0] -= Q[0];
+      k[1] -= Q[1];
+      k[2] -= Q[2];
+      E = dot3(t + 15, a, E);
     }
-    if constexpr (S::str) {
-      Real h = t7 * (k.c2625 * t2 + k.c75);            // 7.5 (rho^2 + 4.5) t^9
-      if constexpr (!UNIF) h *= inv2 * inv2 * inv2 * inv;
-      const Real dmx = t.mx - s.mx, dmy = t.my - s.my, dmz = t.mz - s.mz;
-      const Real phi = dmx * dx + dmy * dy + dmz * dz;
-      const Real psi = t.ax * cx + t.ay * cy + t.az * cz;
-      const Real dw = (s.ax * t.px + s.ay * t.py + s.az * t.pz) +
-                      (t.ax * s.qx + t.ay * s.qy + t.az * s.qz);
-      const Real fphi = f * phi;
-      acc[aB + 0] += fphi * cx - g * s.qx;
-      acc[aB + 1] += fphi * cy - g * s.qy;
-      acc[aB + 2] += fphi * cz - g * s.qz;
-      acc[aY + 0] += fphi * s.ax;
-      acc[aY + 1] += fphi * s.ay;
-      acc[aY + 2] += fphi * s.az;
-      const Real fpsi = f * psi;
-      acc[aD + 0] += fpsi * dmx;
-      acc[aD + 1] += fpsi * dmy;
-      acc[aD + 2] += fpsi * dmz;
-      xc += sc * (f * dw - Real(2) * h * psi * phi);
+    add3(acc.A, g, k);
+    xc = f * (E - dot3(t + 3, k, 0.0));
+    if constexpr (str) {
+      const double dm[3] = {t[9] - m[0], t[10] - m[1], t[11] - m[2]};
+      const double phi = dot3(dm, d, 0.0), psi = dot3(t + 3, c, 0.0);
+      const double fphi = f * phi;
+      add3(acc.B, fphi, c);
+      add3(acc.Y, fphi, a);
+      add3(acc.D, f * psi, dm);
+      const double h = (t5 * t2) * ::fma(-52.5, w, -15.0);  // -2 h
+      xc = ::fma(h * psi, phi, xc);
     }
   }
-  if constexpr (S::pse) {
-    Real p = t7 * t2, q = p * t2;                     // t^9, t^11
-    if constexpr (!UNIF) {
-      p *= inv2;
-      q *= inv2 * inv2;
-    }
-    const Real zx = s.zx - t.zx, zy = s.zy - t.zy, zz = s.zz - t.zz;
-    const Real p105 = k.c105 * p;
-    acc[aA + 0] += p105 * zx;
-    acc[aA + 1] += p105 * zy;
-    acc[aA + 2] += p105 * zz;
-    // (a_j - a_m).(z_m - z_j) = -(a_j - a_m).dz
-    const Real dd = (s.ax - t.ax) * zx + (s.ay - t.ay) * zy + (s.az - t.az) * zz;
-    xc += k.c945 * q * dd;
+  if constexpr (pse) {
+    const double p = (sg * t3) * (w * w * w);
+    const double dz[3] = {z[0] - t[12], z[1] - t[13], z[2] - t[14]};
+    const double da[3] = {a[0] - t[3], a[1] - t[4], a[2] - t[5]};
+    add3(acc.A, 105.0 * p, dz);
+    xc = ::fma(945.0 * (p * t2), dot3(da, dz, 0.0), xc);
   }
-  acc[aX + 0] += xc * dx;
-  acc[aX + 1] += xc * dy;
-  acc[aX + 2] += xc * dz;
+  add3(acc.X, xc, d);
 }
 
-struct AdjArgs {
-  int n;
-  AdjSorted s;
-  const int* perm;
-  double* dpos;
-  double* dstr;
-  int64_t ld;
-  // source split (see vpm_common.h): workgroup (b, k) sums sources
-  // [k*chunk, (k+1)*chunk) into part + k*nslot*pld; part == null: one split
-  double* part;
-  size_t part_cap;
-  int64_t pld;
-  int chunk;
-  int max_splits;  // 0: automatic
-};
-
-// FP64 epilogue of one sorted target k from its pair sums T (AdjSlots layout).
-template <unsigned OUT, bool UNIF>
-__device__ __forceinline__ void adj_store(const AdjArgs& a, int k, const double* T,
-                                          double scale) {
-  using S = AdjSlots<OUT>;
-  const int64_t N = a.n;
-  const AdjSorted& A = a.s;
-  const double ax = A.str[k], ay = A.str[N + k], az = A.str[2 * N + k];
-  double lx = 0, ly = 0, lz = 0, mx = 0, my = 0, mz = 0;
-  if constexpr (S::vel) {
-    lx = A.lam[k]; ly = A.lam[N + k]; lz = A.lam[2 * N + k];
+// grid (rows, splits); components 0..2 dL/dx, 3..5 dL/dalpha.
+template <unsigned OUT>
+__global__ __launch_bounds__(kRowBlock, 4) void adj64_kernel(RowArgs A,
+                                                             const double* __restrict__ rec) {
+  __shared__ double red[kRowWaves][6][kRow];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kRow;
+  const int64_t i = row0 + lane;
+  double t[19];
+  {
+    const double* r = rec + (i < A.m ? i : row0) * kRec64;
+#pragma unroll
+    for (int q = 0; q < 19; ++q) t[q] = r[q];
+    t[18] *= 0.5;
   }
-  if constexpr (S::str) {
-    mx = A.mu[k]; my = A.mu[N + k]; mz = A.mu[2 * N + k];
+  int64_t b, e;
+  row_share(0, A.n, static_cast<int>(blockIdx.y) * kRowWaves + wave, A.splits * kRowWaves, &b, &e);
+  const int64_t o0 = row0 < b ? b : (row0 < e ? row0 : e);
+  const int64_t o1 = row0 + kRow < b ? b : (row0 + kRow < e ? row0 + kRow : e);
+  Adj64Acc acc{};
+  auto load = [&](double* s, int64_t j) {
+    const scalar_double_t* r = (const scalar_double_t*)(rec + j * kRec64);
+#pragma unroll
+    for (int q = 0; q < 19; ++q) s[q] = r[q];
+  };
+  for (int64_t j = o0; j < o1; ++j) {
+    double s[19];
+    load(s, j);
+    if (j != i) adj64_pair<OUT>(acc, t, s);
   }
-  const double C = kOneOverFourPi;
-  double s2 = 1.0, s3 = 1.0, s4 = 1.0;
-  if constexpr (UNIF) {
-    s2 = scale * scale;
-    s3 = s2 * scale;
-    s4 = s2 * s2;
-  }
-  double dA[3], dX[3];
-  for (int c = 0; c < 3; ++c) {
-    dA[c] = C * s2 * T[aA + c];
-    dX[c] = C * s3 * T[aX + c];
-  }
-  const double G[3] = {T[aG], T[aG + 1], T[aG + 2]};
-  if constexpr (S::vel) {  // - C/s^3 (G x lam_m - a_m x Lambda)
-    const double Lm[3] = {T[aL], T[aL + 1], T[aL + 2]};
-    dX[0] -= C * s3 * ((G[1] * lz - G[2] * ly) - (ay * Lm[2] - az * Lm[1]));
-    dX[1] -= C * s3 * ((G[2] * lx - G[0] * lz) - (az * Lm[0] - ax * Lm[2]));
-    dX[2] -= C * s3 * ((G[0] * ly - G[1] * lx) - (ax * Lm[1] - ay * Lm[0]));
-  }
-  if constexpr (S::str) {  // dA += C/s^3 (G x mu_m + B);  dX += C/s^4 (Y x a_m + D)
-    dA[0] += C * s3 * ((G[1] * mz - G[2] * my) + T[aB]);
-    dA[1] += C * s3 * ((G[2] * mx - G[0] * mz) + T[aB + 1]);
-    dA[2] += C * s3 * ((G[0] * my - G[1] * mx) + T[aB + 2]);
-    const double Y[3] = {T[aY], T[aY + 1], T[aY + 2]};
-    dX[0] += C * s4 * ((Y[1] * az - Y[2] * ay) + T[aD]);
-    dX[1] += C * s4 * ((Y[2] * ax - Y[0] * az) + T[aD + 1]);
-    dX[2] += C * s4 * ((Y[0] * ay - Y[1] * ax) + T[aD + 2]);
-  }
-  const int64_t o = a.perm ? a.perm[k] : k;
-  for (int c = 0; c < 3; ++c) {
-    a.dpos[c * a.ld + o] = dX[c];
-    a.dstr[c * a.ld + o] = dA[c];
-  }
-}
-
-// grid (target blocks, source splits)
-template <typename Real, unsigned OUT, bool UNIF, int BLOCK, int TILE, int SUB>
-__global__ __launch_bounds__(BLOCK) void adjoint_kernel(AdjArgs a) {
-  using S = AdjSlots<OUT>;
-  const int lo = static_cast<int>(blockIdx.y) * a.chunk;
-  const int hi = a.chunk < a.n - lo ? lo + a.chunk : a.n;
-  constexpr bool kF32 = std::is_same<Real, float>::value;
-  __shared__ AdjSrc<Real> lds[TILE];
-  __shared__ double red[6][BLOCK / 64];
-  __shared__ double centre[3];
-  const int tid = threadIdx.x;
-  const int k = blockIdx.x * BLOCK + tid;
-  const bool valid = k < a.n;
-  const int64_t N = a.n;
-  const AdjSorted& A = a.s;
-
-  double px = 0, py = 0, pz = 0;
-  if (valid) {
-    px = A.pos[k];
-    py = A.pos[N + k];
-    pz = A.pos[2 * N + k];
+#pragma unroll 1
+  for (int side = 0; side < 2; ++side) {
+    const int64_t j1 = side ? e : o0;
+    for (int64_t j = side ? o1 : b; j < j1; ++j) {
+      double s[19];
+      load(s, j);
+      adj64_pair<OUT>(acc, t, s);
+    }
   }
   {
-    double mn[3] = {valid ? px : INFINITY, valid ? py : INFINITY, valid ? pz : INFINITY};
-    double mx[3] = {valid ? px : -INFINITY, valid ? py : -INFINITY, valid ? pz : -INFINITY};
-    const int lane = tid & 63, wave = tid >> 6;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const double lo = wave_min(mn[c]), hi = wave_max(mx[c]);
-      if (lane == 0) {
-        red[c][wave] = lo;
-        red[3 + c][wave] = hi;
+    constexpr bool vel = OUT & VPM_OUT_VEL, str = OUT & VPM_OUT_STRETCH;
+    double v[6] = {acc.X[0], acc.X[1], acc.X[2], acc.A[0], acc.A[1], acc.A[2]};
+    if constexpr (vel) {
+      add_cross(v, t + 6, acc.G);
+      add_cross(v, t + 3, acc.L);
+    }
+    if constexpr (str) {
+      add_cross(v, acc.Y, t + 3);
+      add_cross(v + 3, acc.G, t + 9);
+      for (int q = 0; q < 3; ++q) {
+        v[q] += acc.D[q];
+        v[3 + q] += acc.B[q];
       }
     }
-    __syncthreads();
-    if (tid < 3) {
-      double lo = red[tid][0], hi = red[3 + tid][0];
-      for (int w = 1; w < BLOCK / 64; ++w) {
-        lo = fmin(lo, red[tid][w]);
-        hi = fmax(hi, red[3 + tid][w]);
-      }
-      centre[tid] = 0.5 * (lo + hi);
-    }
-    __syncthreads();
-  }
-  const double cx = centre[0], cy = centre[1], cz = centre[2];
-  const double sigma0 = UNIF ? A.sig[0] : 1.0;
-  const double scale = UNIF ? 1.0 / sigma0 : 1.0;
-
-  AdjTgt<Real> t{};
-  double ax = 0, ay = 0, az = 0, lx = 0, ly = 0, lz = 0, mx = 0, my = 0, mz = 0;
-  double zx = 0, zy = 0, zz = 0, sg = 1.0;
-  if (valid) {
-    ax = A.str[k]; ay = A.str[N + k]; az = A.str[2 * N + k];
-    lx = A.lam[k]; ly = A.lam[N + k]; lz = A.lam[2 * N + k];
-    mx = A.mu[k]; my = A.mu[N + k]; mz = A.mu[2 * N + k];
-    zx = A.z[k]; zy = A.z[N + k]; zz = A.z[2 * N + k];
-    sg = A.sig[k];
-  }
-  t.x = static_cast<Real>((px - cx) * scale);
-  t.y = static_cast<Real>((py - cy) * scale);
-  t.z = static_cast<Real>((pz - cz) * scale);
-  t.ax = static_cast<Real>(ax); t.ay = static_cast<Real>(ay); t.az = static_cast<Real>(az);
-  t.lx = static_cast<Real>(lx); t.ly = static_cast<Real>(ly); t.lz = static_cast<Real>(lz);
-  t.mx = static_cast<Real>(mx); t.my = static_cast<Real>(my); t.mz = static_cast<Real>(mz);
-  t.px = static_cast<Real>(ay * mz - az * my);   // P_m = a_m x mu_m
-  t.py = static_cast<Real>(az * mx - ax * mz);
-  t.pz = static_cast<Real>(ax * my - ay * mx);
-  t.zx = static_cast<Real>(zx); t.zy = static_cast<Real>(zy); t.zz = static_cast<Real>(zz);
-  t.hs = static_cast<Real>(0.5 * sg);
-
-  const Real rsc = static_cast<Real>(scale);
-  Real part[aN];
-  double tot[aN];
 #pragma unroll
-  for (int q = 0; q < aN; ++q) {
-    part[q] = Real(0);
-    tot[q] = 0.0;
+    for (int q = 0; q < 6; ++q) red[wave][q][lane] = kOneOverFourPi * v[q];
   }
-
-  AdjConst<Real> kc{Real(1.5), Real(3), Real(7.5), Real(26.25), Real(105), Real(945)};
-  if constexpr (kF32)  // keep them in VGPRs
-    asm volatile("" : "+v"(kc.c15), "+v"(kc.c3), "+v"(kc.c75), "+v"(kc.c2625), "+v"(kc.c105),
-                 "+v"(kc.c945));
-
-  for (int t0 = lo; t0 < hi; t0 += TILE) {
-    __syncthreads();
+  __syncthreads();
+  if (wave >= 6) return;
+  double s = 0.0;
 #pragma unroll
-    for (int kk = tid; kk < TILE; kk += BLOCK) {
-      const int j = t0 + kk;
-      AdjSrc<Real> s;
-      if (j < hi) {
-        const double sax = A.str[j], say = A.str[N + j], saz = A.str[2 * N + j];
-        const double smx = A.mu[j], smy = A.mu[N + j], smz = A.mu[2 * N + j];
-        s.x = static_cast<Real>((A.pos[j] - cx) * scale);
-        s.y = static_cast<Real>((A.pos[N + j] - cy) * scale);
-        s.z = static_cast<Real>((A.pos[2 * N + j] - cz) * scale);
-        s.ax = static_cast<Real>(sax); s.ay = static_cast<Real>(say); s.az = static_cast<Real>(saz);
-        s.lx = static_cast<Real>(A.lam[j]);
-        s.ly = static_cast<Real>(A.lam[N + j]);
-        s.lz = static_cast<Real>(A.lam[2 * N + j]);
-        s.mx = static_cast<Real>(smx); s.my = static_cast<Real>(smy); s.mz = static_cast<Real>(smz);
-        s.qx = static_cast<Real>(say * smz - saz * smy);   // Q_j = a_j x mu_j
-        s.qy = static_cast<Real>(saz * smx - sax * smz);
-        s.qz = static_cast<Real>(sax * smy - say * smx);
-        s.zx = static_cast<Real>(A.z[j]);
-        s.zy = static_cast<Real>(A.z[N + j]);
-        s.zz = static_cast<Real>(A.z[2 * N + j]);
-        s.hs = static_cast<Real>(0.5 * A.sig[j]);
-      } else {  // far away, all data zero: every term vanishes (PSE's -k_ij
-                // lambda_i too: at this distance its powers of t underflow to 0
-                // in either precision)
-        s = AdjSrc<Real>{};
-        s.x = s.y = s.z = static_cast<Real>(std::is_same<Real, float>::value ? 1e18 : 1e40);
-        s.hs = Real(0.5);
-      }
-      s.pad = Real(0);
-      lds[kk] = s;
-    }
-    __syncthreads();
-    if (valid) {
-      for (int sb = 0; sb < TILE; sb += SUB) {
-#pragma unroll 4
-        for (int q = 0; q < SUB; ++q) adj_pair<Real, OUT, UNIF>(part, t, lds[sb + q], rsc, kc);
-        if constexpr (kF32) {
-#pragma unroll
-          for (int q = 0; q < aN; ++q) {
-            if (!S::used(q)) continue;
-            tot[q] += static_cast<double>(part[q]);
-            part[q] = Real(0);
-          }
-        }
-      }
-    }
+  for (int w = 0; w < kRowWaves; ++w) s += red[w][wave][lane];
+  if (A.part) {
+    const int64_t pm = static_cast<int64_t>(gridDim.x) * kRow;
+    A.part[(static_cast<int64_t>(blockIdx.y) * 6 + wave) * pm + i] = s;
+  } else if (i < A.m) {
+    A.out[wave / 3][(wave % 3) * A.ld_out + i] = s;
   }
-  if (!valid) return;
-  if constexpr (!kF32) {
-#pragma unroll
-    for (int q = 0; q < aN; ++q) tot[q] = static_cast<double>(part[q]);
-  }
-
-  if (a.part) {  // one split of several: raw sums, coalesced by sorted index
-    double* P = a.part + static_cast<int64_t>(blockIdx.y) * S::nslot * a.pld;
-#pragma unroll
-    for (int q = 0; q < aN; ++q)
-      if (S::used(q)) P[S::packed(q) * a.pld + k] = tot[q];
-    return;
-  }
-  adj_store<OUT, UNIF>(a, k, tot, scale);
 }
 
-// Adds the splits' sums in split order and runs the epilogue.
-template <unsigned OUT, bool UNIF>
-__global__ __launch_bounds__(256) void adj_reduce_kernel(AdjArgs a, int nsplit) {
-  using S = AdjSlots<OUT>;
-  const int k = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
-  if (k >= a.n) return;
-  double T[aN];
-#pragma unroll
-  for (int q = 0; q < aN; ++q) T[q] = 0.0;
-  for (int sp = 0; sp < nsplit; ++sp) {
-    const double* P = a.part + static_cast<int64_t>(sp) * S::nslot * a.pld;
-#pragma unroll
-    for (int q = 0; q < aN; ++q)
-      if (S::used(q)) T[q] += P[S::packed(q) * a.pld + k];
-  }
-  adj_store<OUT, UNIF>(a, k, T, UNIF ? 1.0 / a.s.sig[0] : 1.0);
-}
-
-constexpr int kAdjBlock = 256, kAdjTile = 256, kAdjSub = 32;
-
-template <typename Real, unsigned OUT, bool UNIF>
-int launch_adj(const AdjArgs& a0, hipStream_t st) {
-  const int blocks = static_cast<int>(ceil_div(a0.n, kAdjBlock));
-  auto kern = adjoint_kernel<Real, OUT, UNIF, kAdjBlock, kAdjTile, kAdjSub>;
-  AdjArgs a = a0;
-  const int ntiles = static_cast<int>(ceil_div(a.n, kAdjTile));
-  const int64_t pld = static_cast<int64_t>(blocks) * kAdjBlock;
-  const size_t per_split = static_cast<size_t>(AdjSlots<OUT>::nslot) * pld * sizeof(double);
-  int ks = 1;
-  if (a.part) {
-    int kmax = max_splits_for(blocks, ntiles);
-    const size_t by_cap = a.part_cap / per_split;
-    if (by_cap < static_cast<size_t>(kmax)) kmax = static_cast<int>(by_cap);
-    if (a.max_splits > 0 && a.max_splits < kmax) kmax = a.max_splits;
-    if (kmax > 1) ks = choose_splits(blocks, ntiles, kmax, resident_blocks(kern, kAdjBlock));
-  }
-  if (ks > 1) {
-    a.chunk = static_cast<int>(ceil_div(ntiles, ks)) * kAdjTile;  // ks is effective
-    a.pld = pld;
-  } else {
-    a.part = nullptr;
-    a.chunk = a.n;
-    a.pld = 0;
-  }
-  hipLaunchKernelGGL(kern, dim3(blocks, ks), dim3(kAdjBlock), 0, st, a);
-  VPM_LAUNCH_CHECK("adjoint_kernel");
-  if (ks > 1) {
-    hipLaunchKernelGGL((adj_reduce_kernel<OUT, UNIF>), dim3(static_cast<unsigned>(ceil_div(a.n, 256))),
-                       dim3(256), 0, st, a, ks);
-    VPM_LAUNCH_CHECK("adj_reduce_kernel");
+template <unsigned OUT>
+int launch_adj64(RowArgs a, const double* rec, void* part, size_t part_bytes, int max_splits,
+                 hipStream_t st) {
+  const int64_t rows = row_count(a.m);
+  const size_t per = row_split_bytes(rows, 6, false);
+  int k = row_splits(rows, a.n);
+  if (max_splits > 0) k = std::min(k, max_splits);
+  k = part ? static_cast<int>(std::max<size_t>(1, std::min<size_t>(k, part_bytes / per))) : 1;
+  a.splits = k;
+  a.part = k > 1 ? static_cast<double*>(part) : nullptr;
+  hipLaunchKernelGGL(adj64_kernel<OUT>, dim3(static_cast<unsigned>(rows), k), dim3(kRowBlock), 0,
+                     st, a, rec);
+  VPM_LAUNCH_CHECK("adj64_kernel");
+  if (k > 1) {
+    hipLaunchKernelGGL(row_reduce_kernel, dim3(static_cast<unsigned>(ceil_div(a.m, 256)), 6),
+                       dim3(256), 0, st, a, 6, rows * kRow);
+    VPM_LAUNCH_CHECK("row_reduce_kernel");
   }
   return VPM_OK;
 }
 
-template <bool UNIF>
-int adj_mask(const AdjArgs& a, unsigned mask, hipStream_t st) {
+int adj64_run(const RowArgs& a, unsigned mask, const double* rec, void* part, size_t part_bytes,
+              int max_splits, hipStream_t st) {
   switch (mask) {
-    case 1u: return launch_adj<double, 1u, UNIF>(a, st);
-    case 2u: return launch_adj<double, 2u, UNIF>(a, st);
-    case 3u: return launch_adj<double, 3u, UNIF>(a, st);
-    case 4u: return launch_adj<double, 4u, UNIF>(a, st);
-    case 5u: return launch_adj<double, 5u, UNIF>(a, st);
-    case 6u: return launch_adj<double, 6u, UNIF>(a, st);
-    default: return launch_adj<double, 7u, UNIF>(a, st);
+    case 1u: return launch_adj64<1u>(a, rec, part, part_bytes, max_splits, st);
+    case 2u: return launch_adj64<2u>(a, rec, part, part_bytes, max_splits, st);
+    case 3u: return launch_adj64<3u>(a, rec, part, part_bytes, max_splits, st);
+    case 4u: return launch_adj64<4u>(a, rec, part, part_bytes, max_splits, st);
+    case 5u: return launch_adj64<5u>(a, rec, part, part_bytes, max_splits, st);
+    case 6u: return launch_adj64<6u>(a, rec, part, part_bytes, max_splits, st);
+    default: return launch_adj64<7u>(a, rec, part, part_bytes, max_splits, st);
   }
 }
 
+// Sets up to this size run the FP64 rows also in the FP32-compensated
+// precision: the FP32 rows are twice as fast per pair, but first sort and
+// write records (about 25 us).  All three cotangents, uniform radius, FP64 /
+// FP32 rows: cloud of 1,000 26 / 56 us, 4,000 73 / 97, 5,000 108 / 125, 6,000
+// 148 / 138, 8,000 239 / 187; velocity and stretching only at 5,000 90 / 111,
+// 6,000 124 / 122; velocity only at 6,000 89 / 93.
+constexpr int64_t kAdjRowsMax = 5120;
+
+bool adj_rows_wanted(int64_t n, const vpm_forward_opts_t* o) {
+  return !o || o->precision == VPM_PREC_F64 || n <= kAdjRowsMax;
+}
+
 struct AdjLayout {
-  size_t bbox_part, bbox, keys_in, keys_out, idx_in, perm, sorted, box, split, cub, total,
-      cub_bytes, split_bytes;
+  size_t bbox_part, bbox, keys_in, keys_out, idx_in, perm, rec, box, split, cub, total, cub_bytes,
+      split_bytes;
 };
 
-// sorted: the FP64 pass's sorted arrays, or the records of the FP32 rows.
+// rec: the FP64 rows' records, or those of the FP32 rows.
 int adj_layout(int64_t n, const vpm_forward_opts_t* o, AdjLayout* L) {
-  const bool f32 = o && o->precision == VPM_PREC_F32C;
+  const bool rows = adj_rows_wanted(n, o);
   const size_t N = static_cast<size_t>(n > 0 ? n : 1);
   size_t off = 0;
   auto take = [&](size_t b) {
@@ -532,18 +296,12 @@ int adj_layout(int64_t n, const vpm_forward_opts_t* o, AdjLayout* L) {
   L->keys_out = take(N * 4);
   L->idx_in = take(N * 4);
   L->perm = take(N * 4);
-  L->sorted = take(f32 ? adj32_record_bytes(n) : 17 * N * sizeof(double));
-  L->box = take(f32 ? adj32_box_bytes(n) : 0);
-  // room for the largest source split, sized for all cotangents present
-  const int64_t blocks = ceil_div(n, kAdjBlock);
-  const int kmax = max_splits_for(blocks, ceil_div(n, kAdjTile));
-  L->split_bytes = f32        ? adj32_split_bytes(n)
-                   : kmax > 1 ? static_cast<size_t>(kmax) * AdjSlots<7u>::nslot *
-                                    static_cast<size_t>(blocks * kAdjBlock) * sizeof(double)
-                              : 0;
+  L->rec = take(rows ? N * kRec64 * sizeof(double) : adj32_record_bytes(n));
+  L->box = take(rows ? 0 : adj32_box_bytes(n));
+  L->split_bytes = rows ? row_workspace_bytes(n, n, 6) : adj32_split_bytes(n);
   L->split = take(L->split_bytes);
   size_t cb = 0;
-  if (!o || !o->presorted) {
+  if (!rows && !o->presorted) {
     const int rc = sort_temp_bytes(n, &cb);
     if (rc) return rc;
   }
@@ -670,8 +428,23 @@ int vpm_adjoint(const vpm_particles_t* p, const vpm_adjoint_in_t* in, const vpm_
     return VPM_ERR_WORKSPACE;
   }
   if (n == 0) return VPM_OK;
+  if (o->max_splits < 0) return fail(VPM_ERR_ARG, "vpm_adjoint: max_splits < 0");
+  if (mask == 0) mask = VPM_OUT_VEL;  // all cotangents null: zero gradients from the vel pass
   hipStream_t st = as_stream(stream);
   char* ws = static_cast<char*>(workspace);
+  void* part = L.split_bytes ? ws + L.split : nullptr;
+  if (adj_rows_wanted(n, o)) {
+    double* rec = reinterpret_cast<double*>(ws + L.rec);
+    hipLaunchKernelGGL(adj64_records_kernel, dim3(static_cast<unsigned>(ceil_div(n, 256))),
+                       dim3(256), 0, st, *p, in->lam, in->mu, in->xi, in->ld, rec);
+    VPM_LAUNCH_CHECK("adj64_records_kernel");
+    RowArgs a{};
+    a.m = a.n = n;
+    a.out[0] = out->dpos;
+    a.out[1] = out->dstr;
+    a.ld_out = out->ld;
+    return adj64_run(a, mask, rec, part, L.split_bytes, o->max_splits, st);
+  }
   int* perm = nullptr;
   if (!o->presorted) {
     perm = reinterpret_cast<int*>(ws + L.perm);
@@ -681,35 +454,11 @@ int vpm_adjoint(const vpm_particles_t* p, const vpm_adjoint_in_t* in, const vpm_
                      perm, ws + L.cub, L.cub_bytes, st);
     if (rc) return rc;
   }
-  if (o->max_splits < 0) return fail(VPM_ERR_ARG, "vpm_adjoint: max_splits < 0");
-  if (mask == 0) mask = VPM_OUT_VEL;  // all cotangents null: zero gradients from the vel pass
-  const bool unif = o->sigma_mode == VPM_SIGMA_UNIFORM;
-  double* part = L.split_bytes ? reinterpret_cast<double*>(ws + L.split) : nullptr;
-  if (o->precision == VPM_PREC_F32C)
-    return adj32_run(Adj32Args{*p, in->lam, in->mu, in->xi, in->ld, perm, out->dpos, out->dstr,
-                               out->ld, reinterpret_cast<float*>(ws + L.sorted),
-                               reinterpret_cast<double*>(ws + L.box), part, L.split_bytes,
-                               o->max_splits},
-                     mask, unif, st);
-  double* sorted = reinterpret_cast<double*>(ws + L.sorted);
-  const int ni = static_cast<int>(n);
-  hipLaunchKernelGGL(adj_gather_kernel, dim3(static_cast<unsigned>(ceil_div(n, 256))), dim3(256), 0,
-                     st, *p, in->lam, in->mu, in->xi, in->ld, ni, static_cast<const int*>(perm),
-                     sorted);
-  VPM_LAUNCH_CHECK("adj_gather_kernel");
-  AdjArgs a{};
-  a.n = ni;
-  const int64_t N = n;
-  a.s = AdjSorted{sorted, sorted + 3 * N, sorted + 6 * N, sorted + 9 * N, sorted + 12 * N,
-                  sorted + 15 * N, sorted + 16 * N};
-  a.perm = perm;
-  a.dpos = out->dpos;
-  a.dstr = out->dstr;
-  a.ld = out->ld;
-  a.part = part;
-  a.part_cap = L.split_bytes;
-  a.max_splits = o->max_splits;
-  return unif ? adj_mask<true>(a, mask, st) : adj_mask<false>(a, mask, st);
+  return adj32_run(Adj32Args{*p, in->lam, in->mu, in->xi, in->ld, perm, out->dpos, out->dstr,
+                             out->ld, reinterpret_cast<float*>(ws + L.rec),
+                             reinterpret_cast<double*>(ws + L.box), static_cast<double*>(part),
+                             L.split_bytes, o->max_splits},
+                   mask, o->sigma_mode == VPM_SIGMA_UNIFORM, st);
 }
 
 int vpm_induced_velocity_at_adjoint(const vpm_points_t* targets, const vpm_particles_t* src,

@@ -33,7 +33,7 @@ def particles(layout, n, general, seed):
 @pytest.mark.parametrize("layout", ["cloud", "ring"])
 def test_subsets_at_row_edges(gpu, layout, subset, general):
     mode = "general" if general else "uniform"
-    for n in (2, 63, 65, 700, 4097, 12345):
+    for n in (2, 63, 65, 700, 4097, 5121, 5184, 5185, 12345):
         print(f"[adj32] {layout} n={n} {subset} general={general}", flush=True)
         d, cots = particles(layout, n, general, n)
         cots = [c if f else None for c, f in zip(cots, subset)]
