@@ -6,12 +6,13 @@
 namespace vpm {
 
 // Sets up to this size run the FP64 rows also in the FP32-compensated
-// precision: the FP32 kernels sum pairs two to three times as fast, but their
-// sort, records and few target blocks cost 45-100 us first.  Velocity +
-// stretching, uniform radius, rows / FP32 kernels: cloud of 2,048 21 / 252 us,
-// 4,096 38 / 102, 8,192 102 / 118, 12,288 200 / 193; ring of 4,096 38 / 124,
-// 12,288 197 / 250; with PSE 8,192 116 / 148 (ring), vorticity and enstrophy
-// 78 / 83.
+// precision: the FP32 rows sum pairs up to three times as fast, but first sort
+// and write records, and their near chunks fill with few particles.  FP64 /
+// FP32 rows, uniform radius: velocity, ring of 2,000 21 / 46 us, 8,000 69 /
+// 80, 10,000 102 / 98; velocity + stretching, cloud of 4,000 35 / 67, 8,000
+// 92 / 107, 10,000 144 / 138, ring of 8,000 92 / 132, 10,000 142 / 168;
+// vorticity + enstrophy + stretching, cloud of 8,000 120 / 140, 10,000 187 /
+// 184, general radii 8,000 150 / 155, 10,000 236 / 212.
 constexpr int64_t kForwardRowsMax = 8191;
 
 // The FP64 pass always; the FP32-compensated pass for small sets with no
