@@ -265,10 +265,10 @@ int adj64_run(const RowArgs& a, unsigned mask, const double* rec, void* part, si
 
 // Sets up to this size run the FP64 rows also in the FP32-compensated
 // precision: the FP32 rows are twice as fast per pair, but first sort and
-// write records (about 25 us).  All three cotangents, uniform radius, FP64 /
-// FP32 rows: cloud of 1,000 26 / 56 us, 4,000 73 / 97, 5,000 108 / 125, 6,000
-// 148 / 138, 8,000 239 / 187; velocity and stretching only at 5,000 90 / 111,
-// 6,000 124 / 122; velocity only at 6,000 89 / 93.
+// write records.  FP64 / FP32 rows, cloud, uniform radius: all three
+// cotangents, 1,000 particles 28 / 54 us, 4,000 73 / 86, 5,000 107 / 106,
+// 6,000 145 / 120; velocity and stretching only 5,000 90 / 92, 6,000 122 /
+// 104; velocity only 5,000 65 / 67, 6,000 88 / 74.
 constexpr int64_t kAdjRowsMax = 5120;
 
 bool adj_rows_wanted(int64_t n, const vpm_forward_opts_t* o) {
@@ -292,7 +292,7 @@ int adj_layout(int64_t n, const vpm_forward_opts_t* o, AdjLayout* L) {
   };
   L->bbox_part = take(kBboxBlocks * 6 * sizeof(double));
   L->bbox = take(8 * sizeof(double));
-  L->keys_in = take(N * 4);
+  L->keys_in = take((N + kSamples) * 4);
   L->keys_out = take(N * 4);
   L->idx_in = take(N * 4);
   L->perm = take(N * 4);
@@ -451,7 +451,7 @@ int vpm_adjoint(const vpm_particles_t* p, const vpm_adjoint_in_t* in, const vpm_
     rc = morton_sort(p, reinterpret_cast<double*>(ws + L.bbox_part),
                      reinterpret_cast<double*>(ws + L.bbox), reinterpret_cast<uint32_t*>(ws + L.keys_in),
                      reinterpret_cast<uint32_t*>(ws + L.keys_out), reinterpret_cast<int*>(ws + L.idx_in),
-                     perm, ws + L.cub, L.cub_bytes, st);
+                     perm, ws + L.cub, L.cub_bytes, nullptr, st);
     if (rc) return rc;
   }
   return adj32_run(Adj32Args{*p, in->lam, in->mu, in->xi, in->ld, perm, out->dpos, out->dstr,

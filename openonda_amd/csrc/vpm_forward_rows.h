@@ -7,12 +7,12 @@ namespace vpm {
 
 // Sets up to this size run the FP64 rows also in the FP32-compensated
 // precision: the FP32 rows sum pairs up to three times as fast, but first sort
-// and write records, and their near chunks fill with few particles.  FP64 /
-// FP32 rows, uniform radius: velocity, ring of 2,000 21 / 46 us, 8,000 69 /
-// 80, 10,000 102 / 98; velocity + stretching, cloud of 4,000 35 / 67, 8,000
-// 92 / 107, 10,000 144 / 138, ring of 8,000 92 / 132, 10,000 142 / 168;
-// vorticity + enstrophy + stretching, cloud of 8,000 120 / 140, 10,000 187 /
-// 184, general radii 8,000 150 / 155, 10,000 236 / 212.
+// and write records, and rings leave them few far chunks.  FP64 / FP32 rows,
+// uniform radius: velocity, cloud of 4,096 28 / 37 us, 7,000 60 / 55, 9,000
+// 85 / 71; velocity + stretching, cloud of 4,096 35 / 54, 8,000 93 / 86, 9,000
+// 119 / 107, ring of 8,000 92 / 108, 10,000 143 / 149; with PSE, ring of 8,000
+// 109 / 113, 9,000 141 / 141; vorticity + enstrophy + stretching, cloud of
+// 8,000 120 / 117, 9,000 156 / 146.
 constexpr int64_t kForwardRowsMax = 8191;
 
 // The FP64 pass always; the FP32-compensated pass for small sets with no

@@ -1409,7 +1409,7 @@ int layout(int64_t n, const vpm_forward_opts_t* o, WsLayout* L, bool need_cub = 
   };
   L->bbox_part = take(kBboxBlocks * 6 * sizeof(double));
   L->bbox = take(8 * sizeof(double));
-  L->keys_in = take(N * sizeof(uint32_t));
+  L->keys_in = take((N + kSamples) * sizeof(uint32_t));
   L->keys_out = take(N * sizeof(uint32_t));
   L->idx_in = take(N * sizeof(int));
   L->perm = take(N * sizeof(int));
@@ -1910,21 +1910,17 @@ int forward_prepare_impl(const vpm_particles_t* p, const vpm_forward_opts_t* o, 
                          const WsLayout& L, hipStream_t st) {
   const int64_t n = p->n;
   if (n == 0) return VPM_OK;
-  const int ni = static_cast<int>(n);
-  int* perm = nullptr;
-  if (!o->presorted) {
-    perm = reinterpret_cast<int*>(ws + L.perm);
-    const int rc = morton_sort(p, reinterpret_cast<double*>(ws + L.bbox_part),
-                               reinterpret_cast<double*>(ws + L.bbox),
-                               reinterpret_cast<uint32_t*>(ws + L.keys_in),
-                               reinterpret_cast<uint32_t*>(ws + L.keys_out),
-                               reinterpret_cast<int*>(ws + L.idx_in), perm, ws + L.cub,
-                               L.cub_bytes, st);
-    if (rc) return rc;
-  }
   Src8* src8 = reinterpret_cast<Src8*>(ws + L.src8);
+  if (!o->presorted)
+    return morton_sort(p, reinterpret_cast<double*>(ws + L.bbox_part),
+                       reinterpret_cast<double*>(ws + L.bbox),
+                       reinterpret_cast<uint32_t*>(ws + L.keys_in),
+                       reinterpret_cast<uint32_t*>(ws + L.keys_out),
+                       reinterpret_cast<int*>(ws + L.idx_in), reinterpret_cast<int*>(ws + L.perm),
+                       ws + L.cub, L.cub_bytes, src8, st);
   hipLaunchKernelGGL(gather_kernel, dim3(static_cast<unsigned>(ceil_div(n, kPreBlock))),
-                     dim3(kPreBlock), 0, st, *p, ni, static_cast<const int*>(perm), src8);
+                     dim3(kPreBlock), 0, st, *p, static_cast<int>(n),
+                     static_cast<const int*>(nullptr), src8);
   VPM_LAUNCH_CHECK("gather_kernel");
   return VPM_OK;
 }

@@ -1,6 +1,7 @@
 // Shared prepass of the fused forward and the adjoint: bounding box, 30-bit
-// Morton keys, hipCUB radix sort of (key, index) and the packed FP64 record
-// gather.  Kernels live in an anonymous namespace: each translation unit that
+// Morton keys, the stable sort of (key, index) and the packed FP64 record
+// gather.  Sets of up to kBlockSortMax particles are sorted by two kernels
+// here, larger ones by hipCUB's radix sort.  Kernels live in an anonymous namespace: each translation unit that
 // includes this header gets its own copies.
 #pragma once
 
@@ -82,13 +83,8 @@ __device__ inline uint32_t spread10(uint32_t v) {
   return v;
 }
 
-__global__ __launch_bounds__(kPreBlock) void morton_kernel(const double* __restrict__ pos,
-                                                           int64_t ld, int n,
-                                                           const double* __restrict__ bbox,
-                                                           uint32_t* __restrict__ keys,
-                                                           int* __restrict__ idx) {
-  const int i = blockIdx.x * kPreBlock + threadIdx.x;
-  if (i >= n) return;
+__device__ inline uint32_t morton_key(const double* __restrict__ pos, int64_t ld, int i,
+                                      const double* bbox) {
   uint32_t q[3];
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
@@ -98,8 +94,130 @@ __global__ __launch_bounds__(kPreBlock) void morton_kernel(const double* __restr
     v = v < 0 ? 0 : (v > 1023 ? 1023 : v);
     q[c] = static_cast<uint32_t>(v);
   }
-  keys[i] = spread10(q[0]) | (spread10(q[1]) << 1) | (spread10(q[2]) << 2);
+  return spread10(q[0]) | (spread10(q[1]) << 1) | (spread10(q[2]) << 2);
+}
+
+__global__ __launch_bounds__(kPreBlock) void morton_kernel(const double* __restrict__ pos,
+                                                           int64_t ld, int n,
+                                                           const double* __restrict__ bbox,
+                                                           uint32_t* __restrict__ keys,
+                                                           int* __restrict__ idx) {
+  const int i = blockIdx.x * kPreBlock + threadIdx.x;
+  if (i >= n) return;
+  keys[i] = morton_key(pos, ld, i, bbox);
   idx[i] = i;
+}
+
+// ---- sort of small sets: sorted blocks, then every particle's rank --------
+// A radix sort of some ten thousand keys is a dozen launches of 4-6 us each,
+// whatever its size.  Here one kernel sorts blocks of 1024 keys in registers
+// and LDS, and a second adds up a key's positions in all blocks, which is its
+// place in the whole order (equal keys in index order: the sort is stable).
+// Bound by latency: the searches cost n^2 / 1024 binary searches, split over
+// eight lanes per key.
+constexpr int kSortBlock = 1024;
+constexpr int kSamples = 32;     // per block: the last key of each 32
+// Velocity of a cloud, radix sort and gather / these kernels: 8,193 particles
+// 84 / 66 us, 20,011 240 / 210, 34,914 584 / 563, 65,536 1,872 / 1,863;
+// 100,000 4,199 / 4,224, 200,000 16,425 / 16,592.
+constexpr int kBlockSortMax = 65536;
+constexpr int kSortLanes = 8;    // lanes per key in the second kernel
+
+// Folds the partial boxes, makes the block's keys and sorts them (bitonic, on
+// key and place in the block).
+__global__ __launch_bounds__(kSortBlock) void sort_block_kernel(
+    const double* __restrict__ pos, int64_t ld, int n, const double* __restrict__ part, int nb,
+    uint32_t* __restrict__ keys, int* __restrict__ idx, uint32_t* __restrict__ samples) {
+  __shared__ double box[6];
+  __shared__ uint64_t sh[2][kSortBlock];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  if (wave < 6) {
+    const bool lo = wave < 3;
+    double v = lo ? INFINITY : -INFINITY;
+    for (int b = lane; b < nb; b += 64) {
+      const double x = part[b * 6 + wave];
+      v = lo ? fmin(v, x) : fmax(v, x);
+    }
+    v = lo ? wave_min(v) : wave_max(v);
+    if (lane == 0) box[wave] = v;
+  }
+  __syncthreads();
+  const int base = blockIdx.x * kSortBlock;
+  uint64_t v = ~uint64_t(0);
+  if (base + t < n) v = (static_cast<uint64_t>(morton_key(pos, ld, base + t, box)) << 10) | t;
+  int flip = 0;
+#pragma unroll
+  for (int k = 2; k <= kSortBlock; k <<= 1) {
+#pragma unroll
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      uint64_t o;
+      if (j >= 64) {
+        sh[flip][t] = v;
+        __syncthreads();
+        o = sh[flip][t ^ j];
+        flip ^= 1;
+      } else {
+        o = __shfl_xor(static_cast<unsigned long long>(v), j, 64);
+      }
+      const bool low = ((t & k) == 0) == ((t & j) == 0);
+      v = (v < o) == low ? v : o;
+    }
+  }
+  const uint32_t key = static_cast<uint32_t>(v >> 10);  // 2^32 - 1 past n
+  if (base + t < n) {
+    keys[base + t] = key;
+    idx[base + t] = base + static_cast<int>(v & 1023);
+  }
+  if (t % (kSortBlock / kSamples) == kSortBlock / kSamples - 1)
+    samples[blockIdx.x * kSamples + t / (kSortBlock / kSamples)] = key;
+}
+
+// Eight lanes per key; they also gather its particle's record, one number each.
+__global__ __launch_bounds__(kPreBlock) void sort_rank_kernel(
+    const vpm_particles_t p, int n, const uint32_t* __restrict__ keys,
+    const int* __restrict__ idx, const uint32_t* __restrict__ samples, int* __restrict__ perm,
+    Src8* __restrict__ rec) {
+  constexpr int kGroup = kSortBlock / kSamples;
+  __shared__ uint32_t smp[(kBlockSortMax / kSortBlock) * (kSamples + 1)];
+  const int blocks = (n + kSortBlock - 1) / kSortBlock;
+  for (int q = threadIdx.x; q < blocks * kSamples; q += kPreBlock)
+    smp[q / kSamples * (kSamples + 1) + q % kSamples] = samples[q];
+  __syncthreads();
+  const int e = blockIdx.x * (kPreBlock / kSortLanes) + threadIdx.x / kSortLanes;
+  const int sub = threadIdx.x % kSortLanes;
+  if (e >= n) return;  // with its seven fellows: a key's lanes leave together
+  const uint32_t key = keys[e];
+  const int own = e / kSortBlock;
+  int rank = sub == 0 ? e % kSortBlock : 0;
+  for (int b = sub; b < blocks; b += kSortLanes) {
+    if (b == own) continue;
+    const uint32_t below = key + (b < own);  // earlier blocks' equal keys come first
+    const uint32_t* s = smp + b * (kSamples + 1);
+    int c = 0;
+#pragma unroll
+    for (int st = kSamples; st > 0; st >>= 1)
+      if (c + st <= kSamples && s[c + st - 1] < below) c += st;
+    int at = c * kGroup;
+    if (c < kSamples) {  // below the group's last key
+      const int len = n - b * kSortBlock;
+      const uint32_t* kb = keys + b * kSortBlock;
+#pragma unroll
+      for (int st = kGroup / 2; st > 0; st >>= 1)
+        if (at + st <= len && kb[at + st - 1] < below) at += st;
+    }
+    rank += at;
+  }
+#pragma unroll
+  for (int off = 1; off < kSortLanes; off <<= 1) rank += __shfl_xor(rank, off, 64);
+  const int i = idx[e];
+  if (sub == 0) perm[rank] = i;
+  if (!rec) return;
+  const double v = sub < 3   ? p.pos[sub * p.ld + i]
+                   : sub < 6 ? p.str[(sub - 3) * p.ld + i]
+                   : sub == 6 ? p.sigma[i]
+                   : p.nu     ? p.nu[i]
+                              : 0.0;
+  reinterpret_cast<double*>(rec + rank)[sub] = v;
 }
 
 __global__ __launch_bounds__(kPreBlock) void gather_kernel(const vpm_particles_t p, int n,
@@ -127,10 +245,11 @@ __global__ void fill_kernel(double* __restrict__ p, int64_t n, double v) {
 
 
 // Sorts particles by Morton key of their position.  Returns the permutation
-// (sorted k -> caller index) in `perm`.  Scratch: bbox_part (kBboxBlocks*6),
-// bbox (8), keys_in/keys_out/idx_in (n each) and cub_bytes of hipCUB storage.
+// (sorted k -> caller index) in `perm` and, if `rec` is not null, the packed
+// records in that order.  Scratch: bbox_part (kBboxBlocks*6), bbox (8),
+// kin (n + kSamples), kout/iin (n each) and cub_bytes of hipCUB storage.
 inline int morton_sort(const vpm_particles_t* p, double* bbox_part, double* bbox, uint32_t* kin,
-                       uint32_t* kout, int* iin, int* perm, void* cub, size_t cub_bytes,
+                       uint32_t* kout, int* iin, int* perm, void* cub, size_t cub_bytes, Src8* rec,
                        hipStream_t st) {
   const int64_t n = p->n;
   const int ni = static_cast<int>(n);
@@ -138,6 +257,16 @@ inline int morton_sort(const vpm_particles_t* p, double* bbox_part, double* bbox
   hipLaunchKernelGGL(bbox_partial_kernel, dim3(nbb), dim3(kPreBlock), 0, st, p->pos, p->ld, ni,
                      bbox_part);
   VPM_LAUNCH_CHECK("bbox_partial_kernel");
+  if (n <= kBlockSortMax) {
+    hipLaunchKernelGGL(sort_block_kernel, dim3(static_cast<unsigned>(ceil_div(n, kSortBlock))),
+                       dim3(kSortBlock), 0, st, p->pos, p->ld, ni, bbox_part, nbb, kout, iin, kin);
+    VPM_LAUNCH_CHECK("sort_block_kernel");
+    hipLaunchKernelGGL(sort_rank_kernel,
+                       dim3(static_cast<unsigned>(ceil_div(n, kPreBlock / kSortLanes))),
+                       dim3(kPreBlock), 0, st, *p, ni, kout, iin, kin, perm, rec);
+    VPM_LAUNCH_CHECK("sort_rank_kernel");
+    return VPM_OK;
+  }
   hipLaunchKernelGGL(bbox_final_kernel, dim3(1), dim3(64), 0, st, bbox_part, nbb, bbox);
   VPM_LAUNCH_CHECK("bbox_final_kernel");
   const int nb = static_cast<int>(ceil_div(n, kPreBlock));
@@ -146,15 +275,21 @@ inline int morton_sort(const vpm_particles_t* p, double* bbox_part, double* bbox
   VPM_LAUNCH_CHECK("morton_kernel");
   size_t cb = cub_bytes;
   VPM_HIP_TRY(hipcub::DeviceRadixSort::SortPairs(cub, cb, kin, kout, iin, perm, ni, 0, 30, st));
+  if (rec) {
+    hipLaunchKernelGGL(gather_kernel, dim3(nb), dim3(kPreBlock), 0, st, *p, ni,
+                       static_cast<const int*>(perm), rec);
+    VPM_LAUNCH_CHECK("gather_kernel");
+  }
   return VPM_OK;
 }
 
 inline int sort_temp_bytes(int64_t n, size_t* bytes) {
   *bytes = 0;
+  if (n <= kBlockSortMax) return VPM_OK;
   hipError_t e = hipcub::DeviceRadixSort::SortPairs(
       nullptr, *bytes, static_cast<const uint32_t*>(nullptr), static_cast<uint32_t*>(nullptr),
-      static_cast<const int*>(nullptr), static_cast<int*>(nullptr),
-      static_cast<int>(n > 0 ? n : 1), 0, 30, hipStream_t(0));
+      static_cast<const int*>(nullptr), static_cast<int*>(nullptr), static_cast<int>(n), 0, 30,
+      hipStream_t(0));
   if (e != hipSuccess) {
     set_error("hipcub SortPairs size query failed: %s", hipGetErrorString(e));
     return VPM_ERR_LAUNCH;
