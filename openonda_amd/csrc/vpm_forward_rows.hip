@@ -7,11 +7,12 @@
 // few target blocks of the FP32 kernels cost more than FP64 arithmetic does.
 // Reference arithmetic: ParticlesPhysicsCuda.py:159-191 (velocity), :396-440
 // (stretching), :500-525 (PSE), :319-346 (vorticity), :886-909 + :777
-// (enstrophy).  Bound: FP64 issue, 39 instructions per pair for velocity +
+// (enstrophy).  Bound: FP64 issue, 37 instructions per pair for velocity +
 // stretching with a uniform radius, 41 with sigma_ij.  Velocity + stretching
 // of a cloud of 50,021: 4.10 ms with sorted records staged in LDS (80 bytes
 // per pair and wave through the LDS return path, which bound it), 3.12 ms
-// here; a ring of 4,096 in the FP32-compensated precision 131 -> 40 us.
+// here (2.98 with kFold); a ring of 4,096 in the FP32-compensated precision
+// 131 -> 39 us.
 
 #include "vpm_forward_rows.h"
 
@@ -34,6 +35,13 @@ struct OpForward {
   // The set of a solver step with the plain kernels' arithmetic takes the
   // stretching's sum as they do: a_i x sum g (a_j - a_i) (vpm_plain.hip).
   static constexpr bool kDelta = OUT == (VPM_OUT_STRETCH | VPM_OUT_VORT | VPM_OUT_ENSTROPHY);
+  // With one radius s the factors' powers of it leave the pair: t^3 (1 + 1.5 w)
+  // = t^3 + (1.5 s^2) t^5, and s^2 of the vorticity's t^3 w^2 = s^2 t^5 w and
+  // s^3 of PSE's s t^3 w^3 = s^3 t^5 w^2 are applied in result().  Only where
+  // the stretching forms t^5 anyway: alone, the others stay finite for radii
+  // whose fifth power does not.  Velocity + stretching, 50,021 particles: 3.11
+  // -> 2.98 ms for two instructions of 39; a ring of 4,096 39.9 -> 39.4 us.
+  static constexpr bool kFold = UNIF && str;
   struct Acc {
     double u[3] = {0, 0, 0}, g[3] = {0, 0, 0}, s[3] = {0, 0, 0}, p[3] = {0, 0, 0},
            w[3] = {0, 0, 0}, e[3] = {0, 0, 0};
@@ -51,14 +59,16 @@ struct OpForward {
     }
     // sets with PSE or vorticity alone keep the reference's weight 0 at
     // infinite distance; with the others the pair is inf/inf there
-    double t1, t2, w;
+    double t1, t2, t3, t5, w;
     if constexpr (vel || str || pse || ens || UNIF) {
       t1 = (vel || str || ens) ? rsq64(D) : rsq64_inf(D);
       t2 = t1 * t1;
+      t3 = t2 * t1;
+      t5 = t3 * t2;
       w = s2 * t2;
     }
     if constexpr (vel || str) {
-      const double g = (t2 * t1) * fma(1.5, w, 1.0);
+      const double g = kFold ? fma(1.5 * s2, t5, t3) : t3 * fma(1.5, w, 1.0);
       const double cx = ry * s.az - rz * s.ay;
       const double cy = rz * s.ax - rx * s.az;
       const double cz = rx * s.ay - ry * s.ax;
@@ -72,14 +82,14 @@ struct OpForward {
         a.g[1] = fma(g, kDelta ? s.ay - t.ay : s.ay, a.g[1]);
         a.g[2] = fma(g, kDelta ? s.az - t.az : s.az, a.g[2]);
         const double e = fma(t.ax, cx, fma(t.ay, cy, t.az * cz));
-        const double f = ((t2 * t1) * t2) * fma(7.5, w, 3.0) * e;
+        const double f = t5 * (kFold ? fma(7.5 * s2, t2, 3.0) : fma(7.5, w, 3.0)) * e;
         a.s[0] = fma(f, rx, a.s[0]);
         a.s[1] = fma(f, ry, a.s[1]);
         a.s[2] = fma(f, rz, a.s[2]);
       }
     }
     if constexpr (pse) {
-      const double f = (sg * (t2 * t1)) * (w * w * w);
+      const double f = kFold ? (t5 * w) * w : (sg * t3) * (w * w * w);
       a.p[0] = fma(f, s.ax - t.ax, a.p[0]);
       a.p[1] = fma(f, s.ay - t.ay, a.p[1]);
       a.p[2] = fma(f, s.az - t.az, a.p[2]);
@@ -87,7 +97,7 @@ struct OpForward {
     if constexpr (vort) {  // sigma_j, not sigma_ij (ParticlesPhysicsCuda.py:323,334-337)
       double x;
       if constexpr (UNIF) {
-        x = (t2 * t1) * (w * w);
+        x = kFold ? t5 * w : t3 * (w * w);
       } else {
         const double j2 = s.s * s.s;
         const double q1 = rsq64_inf(r2 + j2);
@@ -100,7 +110,7 @@ struct OpForward {
       a.w[2] = fma(x, s.az, a.w[2]);
     }
     if constexpr (ens) {
-      const double x = t1 * fma(2.2, w, 1.0);
+      const double x = UNIF ? fma(2.2 * s2, t3, t1) : t1 * fma(2.2, w, 1.0);
       a.e[0] = fma(x, s.ax, a.e[0]);
       a.e[1] = fma(x, s.ay, a.e[1]);
       a.e[2] = fma(x, s.az, a.e[2]);
@@ -124,9 +134,10 @@ struct OpForward {
       v[q++] = C * ((t.ax * a.g[1] - t.ay * a.g[0]) + a.s[2]);
     }
     if constexpr (pse)
-      for (int c = 0; c < 3; ++c) v[q++] = 105.0 * t.nu * C * a.p[c];
+      for (int c = 0; c < 3; ++c)
+        v[q++] = 105.0 * t.nu * C * (kFold ? (t.s * t.s * t.s) * a.p[c] : a.p[c]);
     if constexpr (vort)
-      for (int c = 0; c < 3; ++c) v[q++] = 7.5 * C * a.w[c];
+      for (int c = 0; c < 3; ++c) v[q++] = 7.5 * C * (kFold ? (t.s * t.s) * a.w[c] : a.w[c]);
     if constexpr (ens) v[q++] = fma(t.ax, a.e[0], fma(t.ay, a.e[1], t.az * a.e[2]));
   }
 };
