@@ -317,9 +317,12 @@ int adj_layout(int64_t n, const vpm_forward_opts_t* o, AdjLayout* L) {
 //   dA_j = C sum_i g (r x lam_i),  dX_j = C sum_i [g (a_j x lam_i) - f (r.(a_j x lam_i)) r].
 // The particles are the rows' targets and the points the sources (vpm_rows.h):
 // with r' = x_j - y_i = -r and c = r' x lam_i, dA_j = -C sum g c and
-// dX_j = C [a_j x sum g lam_i + sum f (a_j . c) r'].  Bound: FP64 issue, 40
-// instructions per pair (4,096 points, 131,072 particles: 794 us; 1820 us with
-// the points staged in LDS, IEEE root and division, and a_j x lam_i per pair).
+// dX_j = C [a_j x sum g lam_i + sum f (a_j . c) r'].  The radius is the
+// target's, so its square enters the factors as constants: t^3 (1 + 1.5 w) =
+// t^3 + (1.5 s^2) t^5.  Bound: FP64 issue, 38 instructions per pair (4,096
+// points, 131,072 particles: 765 us; 794 us with w = s^2 t^2 formed per pair;
+// 1820 us with the points staged in LDS, IEEE root and division, and a_j x
+// lam_i per pair).
 struct OpVelAtAdjoint {
   static constexpr bool kTargetData = true, kRadius = false, kNu = false, kSkipSelf = false;
   static constexpr int kOut = 6;
@@ -331,12 +334,12 @@ struct OpVelAtAdjoint {
     if (r2 > kEpsPair) {
       const double s2 = t.s * t.s;
       const double tt = rsq64(r2 + s2);
-      const double t2 = tt * tt, t3 = t2 * tt, w = s2 * t2;
-      const double g = t3 * ::fma(1.5, w, 1.0);
+      const double t2 = tt * tt, t3 = t2 * tt, t5 = t3 * t2;
+      const double g = ::fma(1.5 * s2, t5, t3);
       const double cx = ry * s.az - rz * s.ay;
       const double cy = rz * s.ax - rx * s.az;
       const double cz = rx * s.ay - ry * s.ax;
-      const double e = (t3 * t2) * ::fma(7.5, w, 3.0) *
+      const double e = t5 * ::fma(7.5 * s2, t2, 3.0) *
                        ::fma(t.ax, cx, ::fma(t.ay, cy, t.az * cz));
       a.A[0] = ::fma(-g, cx, a.A[0]);
       a.A[1] = ::fma(-g, cy, a.A[1]);
