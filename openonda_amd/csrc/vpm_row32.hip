@@ -479,12 +479,12 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
         for (int u = 0; u < R::kGroup * R::kStride; ++u) b[u] = rec[q * R::kStride + u];
       };
       auto group = [&](const float* b, float* nb, int qn) {
-        pair(b);
+        pair(b, qn - R::kGroup);
         __builtin_amdgcn_sched_barrier(0);
         load(nb, qn);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int u = 1; u < R::kGroup; ++u) pair(b + u * R::kStride);
+        for (int u = 1; u < R::kGroup; ++u) pair(b + u * R::kStride, qn - R::kGroup + u);
       };
       load(bA, 0);
 #pragma unroll 1
@@ -496,12 +496,11 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
     double g64s[3] = {0.0, 0.0, 0.0};
     if (S::str && (fp64 || c == own)) {
       if constexpr (S::str) {
-        // near chunks of FP64 rows, and the row's own chunk: valid sources only
         const int cnt = n - j0 < CH ? n - j0 : CH;
         const int self = c == own ? lane + (row * kRow - j0) : -1;
         const scalar_double_t* str =
             (const scalar_double_t*)(reinterpret_cast<const double*>(src + j0));
-        if (fp64) {
+        if (fp64) {  // near chunks of FP64 rows: valid sources only
           const Src8 tr = target();
           const double ai[3] = {tr.ax, tr.ay, tr.az};
 #pragma unroll R::kNear
@@ -512,23 +511,23 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
             pair32<OUT, UNIF, true>(part, g64s, t, f, aj, ai, eps, kc, q == self);
           }
         } else {
-#pragma unroll 1
-          for (int q = 0; q < cnt; ++q) {
-            float f[R::kStride];
-            load1(f, q);
+          // the row's own chunk, streamed like the others: one record at a time
+          // each pair waited for its load, and the wave with this chunk held up
+          // its row (velocity + stretching, cloud of 9,000: 113 -> 110 us)
+          stream([&](const float* f, int q) {
             pair32<OUT, UNIF, false>(part, g64s, t, f, nullptr, nullptr, eps, kc, q == self);
-          }
+          });
         }
       }
     } else if (!R::kMoment || is_near) {
-      stream([&](const float* f) {
+      stream([&](const float* f, int) {
         pair32<OUT, UNIF, false>(part, g64s, t, f, nullptr, nullptr, eps, kc, false);
       });
     } else if constexpr (R::kMoment) {
       constexpr float es = R::kE3 ? 3.0f : 1.0f;
       const float p[3] = {es * (t.ay * t.z - t.az * t.y), es * (t.az * t.x - t.ax * t.z),
                           es * (t.ax * t.y - t.ay * t.x)};
-      stream([&](const float* f) { pair_far<OUT>(part, t, p, f, kc); });
+      stream([&](const float* f, int) { pair_far<OUT>(part, t, p, f, kc); });
       // u += x_i x G + H of the chunk, in FP64
       const double x = X - box[0], y = Y - box[1], z = Z - box[2];
       const double gx = part[kG + 0], gy = part[kG + 1], gz = part[kG + 2];
