@@ -192,9 +192,11 @@ def main(argv=None):
     # calibrated FETCH_SIZE + WRITE_SIZE runs summarised under profiles/
     from openonda_amd import profiling
 
-    cfg = P.tile_configs()[args.tile_config if args.tile_config >= 0
-                           else P.tile_config_default(outputs)]
-    kernel_name = "fused_kernel<float, 3u, true, {}, {}, {}, {}, {}>".format(*cfg)
+    if args.tile_config >= 0:
+        cfg = P.tile_configs()[args.tile_config]
+        kernel_name = "fused_kernel<float, 3u, true, {}, {}, {}, {}, {}>".format(*cfg)
+    else:
+        kernel_name = "row32_kernel<3u, true, false>"
     traffic = profiling.load_traffic(traffic_workload(n), kernel_name)
     # executed FP32 flops per pair of this kernel instance, from the VALU
     # instruction counters summarised under profiles/ (FMA 2, others 1)
@@ -392,8 +394,7 @@ def main(argv=None):
         torch.cuda.synchronize()
         ring_ms = e0.elapsed_time(e1) / 10
         rpairs = float(nr) * float(nr)
-        rcfg = P.tile_configs()[P.tile_config_default(router)]
-        rkernel = "fused_kernel<float, 7u, true, {}, {}, {}, {}, {}>".format(*rcfg)
+        rkernel = "row32_kernel<7u, true, false>"
         rach = FLOPS_PER_PAIR_VEL_STRETCH_PSE * rpairs / (ring_ms * 1e-3) / 1e12
         rroof = {"bound": "valu", "achieved": rach, "peak": FP32_VECTOR_PEAK_TFLOPS,
                  "unit": "TFLOP/s", "frac": rach / FP32_VECTOR_PEAK_TFLOPS, "kernel": rkernel,
