@@ -164,20 +164,11 @@ __device__ __forceinline__ RowTarget row_target(const RowArgs& a, int64_t i) {
   return t;
 }
 
-// Vector operators.  grid (rows, splits).
+// Sources [b, e) against one target per lane, the row at row0.
 template <class Op>
-__global__ __launch_bounds__(kRowBlock, 4) void row_kernel(RowArgs a) {
-  constexpr int NA = Op::kOut;               // vector components
-  constexpr int NV = NA + (Op::kSum ? 1 : 0);  // + one scalar summed over the targets
-  __shared__ double red[kRowWaves][NV][kRow];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kRow;
-  const RowTarget t = row_target<Op>(a, row0 + lane);
-  const RowSources<Op> src(a);
-  int64_t b, e;
-  row_share(0, a.n, static_cast<int>(blockIdx.y) * kRowWaves + wave, a.splits * kRowWaves, &b, &e);
-  typename Op::Acc acc{};
+__device__ __forceinline__ void row_range(typename Op::Acc& acc, const RowTarget& t,
+                                          const RowSources<Op>& src, int64_t row0, int64_t b,
+                                          int64_t e) {
   if constexpr (Op::kSkipSelf) {  // the row's own particles [o0, o1): j != i
     const int64_t o0 = row0 < b ? b : (row0 < e ? row0 : e);
     const int64_t o1 = row0 + kRow < b ? b : (row0 + kRow < e ? row0 + kRow : e);
@@ -193,6 +184,32 @@ __global__ __launch_bounds__(kRowBlock, 4) void row_kernel(RowArgs a) {
   } else {
     row_sweep<Op>(acc, t, src, b, e);
   }
+}
+
+// Value q of target i: to its split's partials, or to the output.
+__device__ __forceinline__ void row_store(const RowArgs& a, int na, int q, int64_t pm, int64_t i,
+                                          double s) {
+  if (a.part)
+    a.part[(static_cast<int64_t>(blockIdx.y) * na + q) * pm + i] = s;
+  else if (i < a.m && a.out[q / 3])
+    a.out[q / 3][(q % 3) * a.ld_out + i] = s;
+}
+
+// Vector operators.  grid (rows, splits).
+template <class Op>
+__global__ __launch_bounds__(kRowBlock, 4) void row_kernel(RowArgs a) {
+  constexpr int NA = Op::kOut;               // vector components
+  constexpr int NV = NA + (Op::kSum ? 1 : 0);  // + one scalar summed over the targets
+  __shared__ double red[kRowWaves][NV][kRow];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kRow;
+  const RowTarget t = row_target<Op>(a, row0 + lane);
+  const RowSources<Op> src(a);
+  int64_t b, e;
+  row_share(0, a.n, static_cast<int>(blockIdx.y) * kRowWaves + wave, a.splits * kRowWaves, &b, &e);
+  typename Op::Acc acc{};
+  row_range<Op>(acc, t, src, row0, b, e);
   double v[NV];
   Op::result(acc, t, v);
 #pragma unroll
@@ -206,13 +223,57 @@ __global__ __launch_bounds__(kRowBlock, 4) void row_kernel(RowArgs a) {
     if (q == NA) {
       s = wave_sum(i < a.m ? s : 0.0);
       if (lane == 0) a.sums[static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x] = s;
-    } else if (a.part) {
-      const int64_t pm = static_cast<int64_t>(gridDim.x) * kRow;
-      a.part[(static_cast<int64_t>(blockIdx.y) * NA + q) * pm + i] = s;
-    } else if (i < a.m && a.out[q / 3]) {
-      a.out[q / 3][(q % 3) * a.ld_out + i] = s;
+    } else {
+      row_store(a, NA, q, static_cast<int64_t>(gridDim.x) * kRow, i, s);
     }
   }
+}
+
+// The same with a row per wave: all eight waves sweep the same sources, held
+// together by a barrier per kWideTile, so that a source's cache lines are
+// fetched once for 512 targets.  grid (ceil(rows / 8), splits).
+constexpr int kWideTile = 512;
+
+template <class Op>
+__global__ __launch_bounds__(kRowBlock, 4) void row_wide_kernel(RowArgs a, int rows) {
+  constexpr int NA = Op::kOut;
+  constexpr int NV = NA + (Op::kSum ? 1 : 0);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = static_cast<int>(blockIdx.x) * kRowWaves + wave;
+  const int64_t row0 = static_cast<int64_t>(row) * kRow;
+  const RowTarget t = row_target<Op>(a, row0 + lane);
+  const RowSources<Op> src(a);
+  int64_t b, e;
+  row_share(0, a.n, static_cast<int>(blockIdx.y), a.splits, &b, &e);
+  typename Op::Acc acc{};
+#pragma unroll 1
+  for (; b < e; b += kWideTile) {  // the same trips in every wave
+    __syncthreads();
+    row_range<Op>(acc, t, src, row0, b, e - b < kWideTile ? e : b + kWideTile);
+  }
+  if (row >= rows) return;
+  double v[NV];
+  Op::result(acc, t, v);
+  const int64_t i = row0 + lane;
+#pragma unroll
+  for (int q = 0; q < NA; ++q) row_store(a, NA, q, static_cast<int64_t>(rows) * kRow, i, v[q]);
+  if constexpr (Op::kSum) {
+    const double s = wave_sum(i < a.m ? v[NA] : 0.0);
+    if (lane == 0) a.sums[static_cast<int64_t>(blockIdx.y) * rows + row] = s;
+  }
+}
+
+// When a row per wave pays: the component arrays lie a multiple of 4 MiB
+// apart, so a source's seven values fall into the same cache sets, and eight
+// waves at eight places of them evict each other's lines.  Velocity of 2^20
+// particles 1349 -> 1033 ms (2^20 + 24: 958 without), velocity + stretching
+// 2037 -> 1329 (1468 as the tiled FP64 pass with sorted records).  Other
+// strides keep the eight-fold split: 600,011 particles 332 ms against 375,
+// 1,300,021 1549 against 1582; 2^18, 2 MiB apart, 62 against 64.
+constexpr int64_t kWideStride = int64_t{1} << 19, kWideMin = int64_t{1} << 18;
+inline bool row_wide_wanted(const RowArgs& a, int64_t rows) {
+  return a.ld % kWideStride == 0 && a.n >= kWideMin && rows >= kWideMin / kRow;
 }
 
 // Adds the splits in order.  grid (targets / 256, components).
@@ -320,8 +381,13 @@ int row_launch(RowArgs a, void* ws, size_t ws_bytes, hipStream_t st, const char*
     *sums = a.sums;
     *nsums = rows * k;
   }
-  hipLaunchKernelGGL(row_kernel<Op>, dim3(static_cast<unsigned>(rows), k), dim3(kRowBlock), 0, st,
-                     a);
+  if (row_wide_wanted(a, rows))
+    hipLaunchKernelGGL(row_wide_kernel<Op>,
+                       dim3(static_cast<unsigned>(ceil_div(rows, kRowWaves)), k), dim3(kRowBlock),
+                       0, st, a, static_cast<int>(rows));
+  else
+    hipLaunchKernelGGL(row_kernel<Op>, dim3(static_cast<unsigned>(rows), k), dim3(kRowBlock), 0,
+                       st, a);
   VPM_LAUNCH_CHECK(name);
   if (k > 1 && Op::kOut > 0) {
     hipLaunchKernelGGL(row_reduce_kernel, dim3(static_cast<unsigned>(ceil_div(a.m, 256)), Op::kOut),
