@@ -1419,16 +1419,18 @@ int layout(int64_t n, const vpm_forward_opts_t* o, WsLayout* L, bool need_cub = 
   L->scratch_vec = take(3 * N * sizeof(double));
   L->split_bytes = std::min(split_capacity(n, o), split_cap);
   L->split = take(L->split_bytes);
+  // Records and boxes of the kernels that run: the row pass's (8 numbers per
+  // box), else the tiled kernels' far records (6), + one group of records read
+  // ahead past the last chunk.
   const bool far = wants_far_records(o), rows = row32_asked(o);
   const int64_t nn = n > 0 ? n : 1;
-  // + one group of records read ahead past the last chunk
-  L->far_rec = take(far ? (static_cast<size_t>(ceil_div(nn, kMaxFarChunk)) * kMaxFarChunk +
-                           kFarGroup) * kMaxFarStride * sizeof(float)
-                    : rows ? row32_record_bytes(n)
-                           : 0);
-  L->far_box = take(far    ? static_cast<size_t>(ceil_div(nn, kMinFarChunk)) * 6 * sizeof(double)
-                    : rows ? row32_box_bytes(n)
-                           : 0);
+  L->far_rec = take(rows  ? row32_record_bytes(n)
+                    : far ? (static_cast<size_t>(ceil_div(nn, kMaxFarChunk)) * kMaxFarChunk +
+                             kFarGroup) * kMaxFarStride * sizeof(float)
+                          : 0);
+  L->far_box = take(rows  ? row32_box_bytes(n)
+                    : far ? static_cast<size_t>(ceil_div(nn, kMinFarChunk)) * 6 * sizeof(double)
+                          : 0);
   size_t cub_bytes = 0;
   if (need_cub && (!o || !o->presorted)) {
     const int rc = sort_temp_bytes(n, &cub_bytes);

@@ -1,0 +1,66 @@
+"""Workspace sizes of the forward passes: what a query returns covers what the
+call writes.
+
+Host part: the row pass writes the same records and chunk boxes for a uniform
+radius as for per-particle radii, so both need the same workspace.  GPU part:
+every output set in a workspace of exactly the queried size, with guard bytes
+behind it.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from openonda_amd import _lib as L
+
+MASKS = [1, 2, 3, 4, 7, 8, 16, 24, 26, 27, 31]
+
+
+def forward_bytes(n, mask, mode, presorted, tile=-1, precision=L.PREC_F32C):
+    o = L.ForwardOpts(mask, precision, mode, presorted, tile)
+    return L.load().vpm_forward_workspace_bytes(n, C.byref(o))
+
+
+@pytest.mark.parametrize("presorted", [0, 1])
+@pytest.mark.parametrize("mask", MASKS)
+def test_row_pass_workspace_does_not_depend_on_the_radius_mode(mask, presorted):
+    # sorted sets above 65,536 ask the device for the radix sort's scratch
+    for n in (8192, 8193, 9000, 20011, 34914, 65536) + ((300001, 1 << 20) if presorted else ()):
+        uniform = forward_bytes(n, mask, L.SIGMA_UNIFORM, presorted)
+        assert uniform == forward_bytes(n, mask, L.SIGMA_GENERAL, presorted) > 0, (n, mask)
+
+
+GUARD = 1 << 16
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("general", [False, True])
+@pytest.mark.parametrize("mask", MASKS)
+def test_forward_stays_inside_its_workspace(gpu, mask, general):
+    import torch
+
+    from openonda_amd import flow_models as FM
+    from openonda_amd import physics as P
+
+    rng = np.random.default_rng(mask)
+    for n in (1, 700, 8191, 8192, 9000, 20011, 66001):
+        x, a, s, _ = FM.random_cloud(n, seed=n)
+        if general:
+            s = s * rng.uniform(0.8, 1.25, n)
+        d = (P.to_soa(x), P.to_soa(a), torch.from_numpy(s).cuda(),
+             torch.full((n,), 1e-3, dtype=torch.float64, device="cuda"))
+        p = P._particles(*d)
+        mode = L.SIGMA_GENERAL if general else L.SIGMA_UNIFORM
+        for precision in (L.PREC_F32C, L.PREC_F64):
+            for presorted in (0, 1):
+                print(f"[workspace] mask={mask} n={n} general={general} precision={precision} "
+                      f"presorted={presorted}", flush=True)
+                nb = forward_bytes(n, mask, mode, presorted, precision=precision)
+                ws = torch.full((nb + GUARD,), 0xA5, dtype=torch.uint8, device="cuda")
+                o = L.ForwardOpts(mask, precision, mode, presorted, -1)
+                out = torch.zeros((4, 3, n), dtype=torch.float64, device="cuda")
+                ens = torch.zeros(1, dtype=torch.float64, device="cuda")
+                fo = L.ForwardOut(n, *[out[q].data_ptr() for q in range(4)], ens.data_ptr())
+                L.call("vpm_forward", C.byref(p), C.byref(o), C.byref(fo), ws.data_ptr(), nb,
+                       P._stream(d[0]))
+                assert bool((ws[nb:] == 0xA5).all()), (n, precision, presorted)
