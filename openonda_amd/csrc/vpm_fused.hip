@@ -2143,8 +2143,11 @@ int vpm_autotune(const vpm_particles_t* p, const vpm_forward_opts_t* opts, vpm_f
   if (ws_bytes < vpm_autotune_workspace_bytes(p ? p->n : 0, opts))
     return fail(VPM_ERR_WORKSPACE, "vpm_autotune: workspace < vpm_autotune_workspace_bytes");
   vpm_forward_opts_t o = *opts;
-  o.tile_config = -1;
-  int rc = vpm_forward_prepare(p, &o, workspace, ws_bytes, stream);  // sorts once
+  // Sorts once.  With a tile shape: its layout is one that the query covers
+  // (the row pass's may be larger), and the sorted records lie in the same
+  // place for every shape.
+  o.tile_config = 0;
+  int rc = vpm_forward_prepare(p, &o, workspace, ws_bytes, stream);
   if (rc) return rc;
   hipStream_t st = as_stream(stream);
   hipEvent_t e0 = nullptr, e1 = nullptr;

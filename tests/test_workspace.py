@@ -3,8 +3,8 @@ call writes.
 
 Host part: the row pass writes the same records and chunk boxes for a uniform
 radius as for per-particle radii, so both need the same workspace.  GPU part:
-every output set in a workspace of exactly the queried size, with guard bytes
-behind it.
+every output set, and the library's autotuner, in a workspace of exactly the
+queried size, with guard bytes behind it.
 """
 import ctypes as C
 
@@ -64,3 +64,31 @@ def test_forward_stays_inside_its_workspace(gpu, mask, general):
                 L.call("vpm_forward", C.byref(p), C.byref(o), C.byref(fo), ws.data_ptr(), nb,
                        P._stream(d[0]))
                 assert bool((ws[nb:] == 0xA5).all()), (n, precision, presorted)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("general", [False, True])
+@pytest.mark.parametrize("mask,n", [(1, 1000), (1, 4096), (3, 4096), (4, 5120), (7, 9001), (8, 1000),
+                                    (31, 1000), (27, 20011)])
+def test_autotune_accepts_the_workspace_it_asks_for(gpu, mask, n, general):
+    import torch
+
+    from openonda_amd import flow_models as FM
+    from openonda_amd import physics as P
+
+    x, a, s, _ = FM.random_cloud(n, seed=n)
+    d = (P.to_soa(x), P.to_soa(a), torch.from_numpy(s).cuda(),
+         torch.full((n,), 1e-3, dtype=torch.float64, device="cuda"))
+    p = P._particles(*d)
+    o = L.ForwardOpts(mask, L.PREC_F32C, L.SIGMA_GENERAL if general else L.SIGMA_UNIFORM, 0, -1)
+    print(f"[workspace] autotune mask={mask} n={n} general={general}", flush=True)
+    nb = L.load().vpm_autotune_workspace_bytes(n, C.byref(o))
+    ws = torch.full((nb + GUARD,), 0xA5, dtype=torch.uint8, device="cuda")
+    out = torch.zeros((4, 3, n), dtype=torch.float64, device="cuda")
+    ens = torch.zeros(1, dtype=torch.float64, device="cuda")
+    fo = L.ForwardOut(n, *[out[q].data_ptr() for q in range(4)], ens.data_ptr())
+    best = C.c_int(-1)
+    L.call("vpm_autotune", C.byref(p), C.byref(o), C.byref(fo), ws.data_ptr(), nb,
+           P._stream(d[0]), 1, C.byref(best), None)
+    assert 0 <= best.value < L.load().vpm_tile_config_count()
+    assert bool((ws[nb:] == 0xA5).all())
