@@ -16,10 +16,10 @@
 // times the larger radius) of sets with velocity, stretching and a uniform
 // radius take the moment form (pair_far).  Stretching: rows of coherent
 // strengths (coherent_wave) take the sum of g alpha_j and the triple product
-// in FP64 on near chunks and in FP32 on far ones, the others in FP32
-// everywhere, as in the tiled kernels (vpm_fused.hip, which also measures
-// why); sets with vorticity or enstrophy and without PSE sum in FP64 on near
-// chunks in every row.
+// in FP64, the others in FP32, as in the tiled kernels (vpm_fused.hip, which
+// also measures why); sets with vorticity or enstrophy and without PSE sum in
+// FP64 in every row.  With a uniform radius and more outputs than the
+// stretching, far chunks are summed in FP32 in every row (kFarFp32).
 //
 // With s = sigma_ij, D = r^2 + s^2, t = D^-1/2 and w = s^2 t^2 no reciprocal
 // of s is needed: (rho^2 + 2.5) / (A^5/2 s^3) = t^3 (1 + 1.5 w) and so on
@@ -28,9 +28,9 @@
 // Bound: FP32 issue (velocity alone 2.45e12 pairs/s, 1.55 wave64 instructions
 // per clock and CU; the moment form 1.8e12).  Tiled kernels -> here, per call.
 // N = 100,000: velocity 4.80 -> 4.17 ms, with per-particle radii 6.80 -> 4.78;
-// stretching of a ring 9.51 -> 7.40, 11.5 -> 7.31; PSE 5.81 -> 4.92, 6.96 ->
+// stretching of a ring 8.92 -> 8.32, 10.9 -> 8.60; PSE 5.81 -> 4.92, 6.96 ->
 // 5.78; vorticity + enstrophy 4.97 -> 4.73, 7.41 -> 5.98; all five with
-// per-particle radii 16.0 -> 14.7 (cloud), 19.4 -> 15.4 (ring).  Velocity +
+// per-particle radii 15.3 -> 13.5 (cloud), 18.3 -> 16.9 (ring).  Velocity +
 // stretching: cloud of 2^20 614 -> 605, of 20,000 0.448 -> 0.328, ring of
 // 131,072 12.8 -> 11.1; with PSE: ring of 131,072 15.7 -> 13.1, leapfrogging
 // rings of 65,536 4.30 -> 3.49.
@@ -70,6 +70,13 @@ struct Rec32 {
   static constexpr bool kLo = OUT & VPM_OUT_PSE;
   static constexpr bool kMoment = UNIF && (OUT & VPM_OUT_VEL) && (OUT & VPM_OUT_STRETCH);
   static constexpr bool kE3 = kMoment && kLo;
+  // Stretching: rows that sum in FP64 per pair do so on near chunks only, or
+  // on every chunk.  FP32 sums of g alpha_j leave 1e-7 of |alpha_i| |G|, and
+  // along a tube of parallel strengths nothing else is left.  FP64 everywhere
+  // costs a ring of 100,000 with per-particle radii 8.6 ms instead of 7.3
+  // (stretching; tiled kernels 10.9), a cloud, whose rows are not coherent,
+  // nothing.
+  static constexpr bool kFarFp32 = UNIF && OUT != VPM_OUT_STRETCH;
   static constexpr int kLoAt = kMoment ? 9 : UNIF ? 6 : 8;
   static constexpr int kStride = kLo ? 12 : kMoment ? 9 : UNIF ? 6 : 8;
   static constexpr int kGroup = kLo ? 2 : kMaxGroup32;
@@ -410,6 +417,8 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
       if (a.g64_mode == VPM_G64_AUTO) g64 = coherent_wave<1>(&ti, &valid);
     }
     g64 = __builtin_amdgcn_readfirstlane(static_cast<int>(g64)) != 0;
+  }
+  if constexpr (S::str && R::kFarFp32) {
     const double p[3] = {X, Y, Z};
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
@@ -435,7 +444,7 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
   int seen = 0;
   for (int c = split * kRowWaves + wave; c < nchunk; c += parts, ++seen) {
     bool is_near = true;
-    if constexpr (S::str) {
+    if constexpr (S::str && R::kFarFp32) {
       // far tests for 64 of the wave's chunks at a time, one per lane
       if ((seen & 63) == 0) {
         const int64_t cc = c + static_cast<int64_t>(lane) * parts;
@@ -500,7 +509,7 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
         const int self = c == own ? lane + (row * kRow - j0) : -1;
         const scalar_double_t* str =
             (const scalar_double_t*)(reinterpret_cast<const double*>(src + j0));
-        if (fp64) {  // near chunks of FP64 rows: valid sources only
+        if (fp64) {  // valid sources only
           const Src8 tr = target();
           const double ai[3] = {tr.ax, tr.ay, tr.az};
 #pragma unroll R::kNear
