@@ -87,7 +87,8 @@ __device__ __forceinline__ void cross(const double* a, const double* b, double* 
 }
 
 // One wave per chunk; lanes past n write zero data far away (every term
-// vanishes; PSE's powers of t underflow to 0 at that distance).
+// vanishes; PSE's powers of t underflow to 0 at that distance).  The box is
+// that of the finite coordinates, as in vpm_row32.hip.
 __global__ __launch_bounds__(kAdjChunk) void adj32_records_kernel(Adj32Args A) {
   const int c = blockIdx.x, n = static_cast<int>(A.p.n);
   const int k = c * kAdjChunk + static_cast<int>(threadIdx.x);
@@ -100,12 +101,13 @@ __global__ __launch_bounds__(kAdjChunk) void adj32_records_kernel(Adj32Args A) {
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
     x[q] = held(g.x[q] * scale);
-    const double lo = wave_min(ok ? x[q] : INFINITY), hi = wave_max(ok ? x[q] : -INFINITY);
-    cen[q] = 0.5 * (lo + hi);
+    const bool in = ok && isfinite(x[q]);
+    const double lo = wave_min(in ? x[q] : INFINITY), hi = wave_max(in ? x[q] : -INFINITY);
+    cen[q] = lo <= hi ? 0.5 * (lo + hi) : 0.0;
     x[q] -= cen[q];
     if (threadIdx.x == 0) {
       box[q] = cen[q];
-      box[3 + q] = 0.5 * (hi - lo);
+      box[3 + q] = lo <= hi ? 0.5 * (hi - lo) : 0.0;
     }
   }
   const double big = wave_max(ok ? g.s * scale : 0.0);

@@ -92,7 +92,9 @@ __device__ __forceinline__ double held(double v) {  // rounded here, not fused i
 
 // The records and box of chunk c of a set of n sorted particles, by one
 // workgroup of kChunk lanes; rec and box_ are the set's.  Lanes past n write
-// zero-strength padding far away, which adds exactly 0.
+// zero-strength padding far away, which adds exactly 0.  The box is that of
+// the finite coordinates: a particle at infinity keeps an infinite offset (PSE
+// and vorticity weigh it 0) and leaves its chunk's others theirs.
 template <unsigned OUT, bool UNIF>
 __device__ __forceinline__ void row32_records(const Src8* __restrict__ src, int n, int c,
                                               float* __restrict__ rec, double* __restrict__ box_) {
@@ -108,7 +110,8 @@ __device__ __forceinline__ void row32_records(const Src8* __restrict__ src, int 
   const double sig = g.s * scale;
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
-    const double lo = wave_min(ok ? p[q] : INFINITY), hi = wave_max(ok ? p[q] : -INFINITY);
+    const bool in = ok && isfinite(p[q]);
+    const double lo = wave_min(in ? p[q] : INFINITY), hi = wave_max(in ? p[q] : -INFINITY);
     if (lane == 0) {
       red[q][wave] = lo;
       red[3 + q][wave] = hi;
@@ -127,10 +130,10 @@ __device__ __forceinline__ void row32_records(const Src8* __restrict__ src, int 
       lo = fmin(lo, red[q][w]);
       hi = fmax(hi, red[3 + q][w]);
     }
-    cen[q] = 0.5 * (lo + hi);
+    cen[q] = lo <= hi ? 0.5 * (lo + hi) : 0.0;
     if (threadIdx.x == 0) {
       box[q] = cen[q];
-      box[3 + q] = 0.5 * (hi - lo);
+      box[3 + q] = lo <= hi ? 0.5 * (hi - lo) : 0.0;
     }
   }
   if (threadIdx.x == 0) {
