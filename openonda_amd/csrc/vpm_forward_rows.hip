@@ -57,11 +57,11 @@ struct OpForward {
     } else {
       D = fma(rx, rx, fma(ry, ry, fma(rz, rz, s2)));
     }
-    // sets with PSE or vorticity alone keep the reference's weight 0 at
-    // infinite distance; with the others the pair is inf/inf there
+    // PSE and the vorticity have the reference's weight 0 at infinite distance;
+    // the others are inf/inf there
     double t1, t2, t3, t5, w;
     if constexpr (vel || str || pse || ens || UNIF) {
-      t1 = (vel || str || ens) ? rsq64(D) : rsq64_inf(D);
+      t1 = (pse || (vort && UNIF)) ? rsq64_inf(D) : rsq64(D);
       t2 = t1 * t1;
       t3 = t2 * t1;
       t5 = t3 * t2;

@@ -63,17 +63,17 @@ def reference():
                                      ("vel", "stretch", "pse"),
                                      ("stretch", "vort", "enstrophy"),
                                      ("vel", "stretch", "vort", "enstrophy"), ALL], ids="-".join)
-@pytest.mark.parametrize("n", [9000])
-def test_forward(gpu, reference, outputs, general, n):
+@pytest.mark.parametrize("n,precision", [(300, "f32c"), (9000, "f32c"), (1500, "f64")])
+def test_forward(gpu, reference, outputs, general, n, precision):
     i, sample, ref = reference(n, general)
     x, a, s, nu = particles(n, general)
     x[n // 2] = np.inf
     d = dev(x, a, s, nu)
-    print(f"[infinity] n={n} {outputs} general={general}", flush=True)
-    got = P.forward(*d, outputs=outputs, precision="f32c",
+    print(f"[infinity] n={n} {outputs} general={general} {precision}", flush=True)
+    got = P.forward(*d, outputs=outputs, precision=precision,
                     sigma_mode="general" if general else "uniform")
     for k in set(outputs) & {"pse", "vort"}:
-        assert rel(P.from_soa(got[k])[i][sample], ref[k]) <= TOL["f32c"], k
+        assert rel(P.from_soa(got[k])[i][sample], ref[k]) <= TOL[precision], k
 
 
 @pytest.mark.parametrize("general", [False, True])
