@@ -20,6 +20,7 @@ struct Adj32Args {
   double* part;         // split partials, or null
   size_t part_cap;
   int max_splits;       // 0: automatic
+  bool unif;            // one radius
 };
 
 size_t adj32_record_bytes(int64_t n);
@@ -27,6 +28,6 @@ size_t adj32_box_bytes(int64_t n);
 size_t adj32_split_bytes(int64_t n);
 
 // mask: VPM_OUT_VEL | STRETCH | PSE, the cotangents present.
-int adj32_run(const Adj32Args& a, unsigned mask, bool unif, hipStream_t st);
+int adj32_run(const Adj32Args& a, unsigned mask, hipStream_t st);
 
 }  // namespace vpm

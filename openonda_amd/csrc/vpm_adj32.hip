@@ -7,7 +7,8 @@
 // six numbers the particle needs (dL/dx, dL/dalpha), so neither 21 FP64
 // totals per lane nor 21 split partials are kept.
 //
-// With r = x_m - x_j, sc = 1/sigma (lengths are in units of sigma), per pair
+// With r = x_m - x_j, sc = 1/sigma (lengths are in units of a uniform radius;
+// with per-particle radii as they are, sc = 1), per pair
 //   near: c = r x a_j, k = lam_j x r - sc Q_j,
 //         E = lam_m.c - a_m.k + a_j.(sc P_m), psi = a_m.c
 //   far (box gap above 4 radii), with m_j = a_j x x_j, v_j = lam_j x x_j + sc Q_j
@@ -59,6 +60,10 @@ __device__ __forceinline__ double held(double v) {  // rounded here, not fused i
   return v;
 }
 
+__device__ __forceinline__ double adj_scale(const Adj32Args& A) {
+  return A.unif ? 1.0 / A.p.sigma[0] : 1.0;
+}
+
 // A particle's data in FP64, by sorted index.
 struct AdjParticle {
   double x[3], a[3], l[3], m[3], z[3], s;
@@ -93,7 +98,7 @@ __global__ __launch_bounds__(kAdjChunk) void adj32_records_kernel(Adj32Args A) {
   const int c = blockIdx.x, n = static_cast<int>(A.p.n);
   const int k = c * kAdjChunk + static_cast<int>(threadIdx.x);
   const bool ok = k < n;
-  const double scale = 1.0 / A.p.sigma[A.perm ? A.perm[0] : 0];
+  const double scale = adj_scale(A);
   AdjParticle g{};
   if (ok) g = adj_particle(A, k);
   double x[3], cen[3];
@@ -181,12 +186,13 @@ __device__ __forceinline__ void adj_weights(AdjW& w_, const AdjT32& t, const flo
     s = t.hs + f[15];
     s2 = s * s;
   }
-  const float t1 = __builtin_amdgcn_rsqf(dot3(d, d, s2));
+  float t1 = __builtin_amdgcn_rsqf(dot3(d, d, s2));
+  if constexpr (vs)
+    if (self) t1 = 0.0f;  // all weights 0, also where a small radius' t7 is infinite
   const float t2 = t1 * t1, t3 = t2 * t1, t5 = t3 * t2;
   const float w = UNIF ? t2 : s2 * t2;
   if constexpr (vs) {
     w_.g = UNIF ? __builtin_fmaf(k.c15, t5, t3) : t3 * __builtin_fmaf(k.c15, w, 1.0f);
-    if (self) w_.g = 0.0f;
     w_.f = t5 * __builtin_fmaf(k.c75, w, k.c3);
   }
   if constexpr ((OUT & VPM_OUT_STRETCH) != 0)
@@ -298,7 +304,7 @@ __global__ __launch_bounds__(kRowBlock, kAdjWaves) void adj32_kernel(Adj32Args A
   const int row = blockIdx.x, n = static_cast<int>(A.p.n);
   const int kt = row * kRow + lane;
   const bool valid = kt < n;
-  const double scale = 1.0 / A.p.sigma[A.perm ? A.perm[0] : 0];
+  const double scale = adj_scale(A);
   AdjParticle g{};
   g.s = 1.0;
   if (valid) g = adj_particle(A, kt);
@@ -487,7 +493,7 @@ __global__ __launch_bounds__(256) void adj32_reduce_kernel(Adj32Args A, int spli
   if (k >= A.p.n) return;
   double s = 0.0;
   for (int i = 0; i < splits; ++i) s += A.part[(static_cast<int64_t>(i) * kAdjOut + q) * pld + k];
-  const double scale = 1.0 / A.p.sigma[A.perm ? A.perm[0] : 0], s2 = scale * scale;
+  const double scale = adj_scale(A), s2 = scale * scale;
   const int64_t o = A.perm ? A.perm[k] : k;
   if (q < 3) A.dpos[q * A.ld + o] = kOneOverFourPi * s2 * scale * s;
   else A.dstr[(q - 3) * A.ld + o] = kOneOverFourPi * s2 * s;
@@ -548,8 +554,8 @@ size_t adj32_split_bytes(int64_t n) {
   return k > 1 ? static_cast<size_t>(k) * kAdjOut * rows * kRow * sizeof(double) : 0;
 }
 
-int adj32_run(const Adj32Args& a, unsigned mask, bool unif, hipStream_t st) {
-  return unif ? launch_mask<true>(a, mask, st) : launch_mask<false>(a, mask, st);
+int adj32_run(const Adj32Args& a, unsigned mask, hipStream_t st) {
+  return a.unif ? launch_mask<true>(a, mask, st) : launch_mask<false>(a, mask, st);
 }
 
 }  // namespace vpm

@@ -460,8 +460,8 @@ int vpm_adjoint(const vpm_particles_t* p, const vpm_adjoint_in_t* in, const vpm_
   return adj32_run(Adj32Args{*p, in->lam, in->mu, in->xi, in->ld, perm, out->dpos, out->dstr,
                              out->ld, reinterpret_cast<float*>(ws + L.rec),
                              reinterpret_cast<double*>(ws + L.box), static_cast<double*>(part),
-                             L.split_bytes, o->max_splits},
-                   mask, o->sigma_mode == VPM_SIGMA_UNIFORM, st);
+                             L.split_bytes, o->max_splits, o->sigma_mode == VPM_SIGMA_UNIFORM},
+                   mask, st);
 }
 
 int vpm_induced_velocity_at_adjoint(const vpm_points_t* targets, const vpm_particles_t* src,

@@ -58,7 +58,9 @@ constexpr int kRow32Waves = 6;
 // Record layout: offset (3), strength (3); then with the moment form the
 // moment alpha x offset (3; three times it with PSE, pair_far), with
 // per-particle radii sigma/2 and sigma^2; with PSE the low parts
-// alpha - fp32(alpha).  Lengths in units of the first particle's radius.
+// alpha - fp32(alpha).  Lengths in units of a uniform radius; with per-particle
+// radii as they are: any one particle's radius may be far from the others',
+// and the powers of t leave FP32 where distances are 1e8 units.
 // Two groups are in registers at once: of four records, or of two where a
 // record has twelve floats and four would spill scalar registers (velocity +
 // stretching + PSE, cloud of 131,072: 11.4 against 12.5 ms, ring 13.4 against
@@ -103,7 +105,7 @@ __device__ __forceinline__ void row32_records(const Src8* __restrict__ src, int 
   const int k = c * R::kChunk + static_cast<int>(threadIdx.x);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const bool ok = k < n;
-  const double scale = 1.0 / src[0].s;
+  const double scale = UNIF ? 1.0 / src[0].s : 1.0;
   Src8 g{};
   if (ok) g = src[k];
   const double p[3] = {held(g.x * scale), held(g.y * scale), held(g.z * scale)};
@@ -388,7 +390,7 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kt = row * kRow + lane;
   const bool valid = kt < n;
-  const double scale = 1.0 / src[0].s;
+  const double scale = UNIF ? 1.0 / src[0].s : 1.0;
   Src8 ti{0, 0, 0, 0, 0, 0, 1, 0};
   if (valid) ti = src[kt];
   const double X = held(ti.x * scale), Y = held(ti.y * scale), Z = held(ti.z * scale);
@@ -593,7 +595,7 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
     for (int q = 0; q < 3; ++q) G[q] = tot[0][S::nacc + q][lane];
   }
   double ens = 0.0;
-  if (valid) ens = store_target<OUT, true>(a, target(), perm ? perm[kt] : kt, T, G, scale);
+  if (valid) ens = store_target<OUT, UNIF>(a, target(), perm ? perm[kt] : kt, T, G, scale);
   if constexpr (S::ens) {
     ens = wave_sum(ens);
     if (lane == 0) a.ens_part[blockIdx.x] = ens;
@@ -702,7 +704,7 @@ int launch(FusedArgs a, float* rec, double* box, hipStream_t st, int* nblocks) {
   *nblocks = rows;
   if (k > 1) {
     const int rb = static_cast<int>(ceil_div(a.n, 256));
-    hipLaunchKernelGGL((split_reduce_kernel<OUT, true>), dim3(rb), dim3(256), 0, st, a, k);
+    hipLaunchKernelGGL((split_reduce_kernel<OUT, UNIF>), dim3(rb), dim3(256), 0, st, a, k);
     VPM_LAUNCH_CHECK("split_reduce_kernel");
     *nblocks = rb;
   }
