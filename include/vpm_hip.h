@@ -200,7 +200,8 @@ size_t vpm_forward_workspace_bytes(int64_t n, const vpm_forward_opts_t* opts);
 /* vpm_forward = vpm_forward_prepare + vpm_forward_run on the same workspace.
  * prepare sorts (unless presorted) and packs the particles into the
  * workspace; run executes the pair pass and the reductions.  run may be
- * repeated on one prepared workspace while the particles are unchanged. */
+ * repeated on one prepared workspace while the particles are unchanged.
+ * Outputs may take the place of the inputs. */
 int vpm_forward(const vpm_particles_t* p, const vpm_forward_opts_t* opts,
                 vpm_forward_out_t* out, void* workspace, size_t ws_bytes, void* stream);
 

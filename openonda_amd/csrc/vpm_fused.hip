@@ -1949,6 +1949,40 @@ int check_forward_out(const vpm_particles_t* p, const vpm_forward_opts_t* o,
   return VPM_OK;
 }
 
+// Positions, strengths, radii and viscosities one behind the other.
+__global__ __launch_bounds__(kPreBlock) void copy_particles_kernel(const vpm_particles_t p,
+                                                                   double* __restrict__ out) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPreBlock + threadIdx.x;
+  if (i >= p.n) return;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    out[c * p.n + i] = p.pos[c * p.ld + i];
+    out[(3 + c) * p.n + i] = p.str[c * p.ld + i];
+  }
+  out[6 * p.n + i] = p.sigma[i];
+  out[7 * p.n + i] = p.nu ? p.nu[i] : 0.0;
+}
+
+// Whether a requested output lies over one of the inputs.
+bool writes_inputs(const vpm_particles_t* p, const vpm_forward_opts_t* o,
+                   const vpm_forward_out_t* out) {
+  auto meet = [](const double* a, int64_t na, const double* b, int64_t nb) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return a && b && x < y + nb * sizeof(double) && y < x + na * sizeof(double);
+  };
+  auto any = [&](const double* v, int64_t len) {
+    return meet(v, len, p->pos, 2 * p->ld + p->n) || meet(v, len, p->str, 2 * p->ld + p->n) ||
+           meet(v, len, p->sigma, p->n) || meet(v, len, p->nu, p->n);
+  };
+  const unsigned want = o->outputs;
+  const int64_t len = 2 * out->ld + p->n;
+  return ((want & VPM_OUT_VEL) && any(out->vel, len)) ||
+         ((want & VPM_OUT_STRETCH) && any(out->stretch, len)) ||
+         ((want & VPM_OUT_PSE) && any(out->pse, len)) ||
+         ((want & VPM_OUT_VORT) && any(out->vort, len)) ||
+         ((want & VPM_OUT_ENSTROPHY) && any(out->enstrophy, 1));
+}
+
 // The pass itself, from the sorted records of forward_prepare_impl.
 int forward_run_impl(const vpm_particles_t* p, const vpm_forward_opts_t* o,
                      vpm_forward_out_t* out, char* ws, const WsLayout& L, hipStream_t st) {
@@ -1963,9 +1997,20 @@ int forward_run_impl(const vpm_particles_t* p, const vpm_forward_opts_t* o,
   }
   const unsigned mask = forward_rows_wanted(n, o) || row32_asked(o) ? row_mask(want)
                                                                      : kernel_mask(want);
-  if (forward_rows_wanted(n, o))
-    return forward_rows(p, o, out, mask, reinterpret_cast<double*>(ws + L.ens_part),
+  if (forward_rows_wanted(n, o)) {
+    // These rows read the caller's arrays while others are stored: outputs in
+    // the inputs' place are summed from a copy, in the records' region.
+    vpm_particles_t q = *p;
+    if (writes_inputs(p, o, out)) {
+      double* c = reinterpret_cast<double*>(ws + L.src8);
+      hipLaunchKernelGGL(copy_particles_kernel, dim3(static_cast<unsigned>(ceil_div(n, kPreBlock))),
+                         dim3(kPreBlock), 0, st, *p, c);
+      VPM_LAUNCH_CHECK("copy_particles_kernel");
+      q = vpm_particles_t{n, n, c, c + 3 * n, c + 6 * n, c + 7 * n};
+    }
+    return forward_rows(&q, o, out, mask, reinterpret_cast<double*>(ws + L.ens_part),
                         L.split_bytes ? ws + L.split : nullptr, L.split_bytes, st);
+  }
   // Unrequested outputs of a superset kernel share one scratch region; a
   // thread writes only its own target's rows there, so they cannot race.
   double* scratch = reinterpret_cast<double*>(ws + L.scratch_vec);
