@@ -101,14 +101,17 @@ def _src(x, a, s, nu=None, targets=None):
     # memory 14 (8,192: 56 and 26); large sets stay pageable, so that torch's
     # pinned-memory cache stays small.
     k = 7 if nu is None else 8
-    buf = torch.empty((k, n), dtype=torch.float64, pin_memory=0 < k * n * 8 <= _PINNED_BYTES)
+    pinned = 0 < k * n * 8 <= _PINNED_BYTES
+    buf = torch.empty((k, n), dtype=torch.float64, pin_memory=pinned)
     rows = buf.numpy()
     rows[0:3] = x.T
     rows[3:6] = a.T
     rows[6] = s
     if nu is not None:
         rows[7] = nu
-    d = buf.to(dev, non_blocking=True)
+    # only a pinned buffer outlives the call (torch's allocator keeps it until
+    # the copy is done); a pageable one is copied before this returns
+    d = buf.to(dev, non_blocking=pinned)
     out = [d[0:3], d[3:6], d[6]]
     if nu is not None:
         out.append(d[7])

@@ -185,3 +185,26 @@ def test_drop_in_rejects_non_positive_radii_and_negative_viscosity():
     with pytest.raises(L.NonFiniteError, match="viscosities"):
         H.get_strength_gradients_PSE(x, a, np.full(3, 0.1), np.array([1e-3, -1e-9, 0.0]))
     assert issubclass(L.NonFiniteError, ValueError)
+
+
+def test_pageable_upload_is_a_blocking_copy(monkeypatch):
+    """Sets too large for a pinned buffer: the buffer is dropped when the call
+    returns, so its copy must be done by then."""
+    from openonda_amd import ParticlesPhysicsHip as H
+
+    n = H._PINNED_BYTES // (7 * 8) + 1
+    rng = np.random.default_rng(0)
+    x, a, s = rng.normal(size=(n, 3)), rng.normal(size=(n, 3)), np.full(n, 0.1)
+    asked = []
+    to = torch.Tensor.to
+
+    def spy(self, *args, **kw):
+        asked.append(kw.get("non_blocking", False))
+        return to(self, *args, **kw)
+
+    monkeypatch.setattr(H, "_dev", lambda: torch.device("cpu"))
+    monkeypatch.setattr(torch.Tensor, "to", spy)
+    dx, da, ds = H._src(x, a, s)
+    assert asked == [False]
+    assert np.array_equal(dx.numpy(), x.T) and np.array_equal(da.numpy(), a.T)
+    assert np.array_equal(ds.numpy(), s)
