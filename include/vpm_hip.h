@@ -317,6 +317,7 @@ typedef struct vpm_adjoint_out {
   double* dstr;         /* [3][ld] dL/dalpha, overwritten */
 } vpm_adjoint_out_t;
 
+/* Enough for either precision; opts (may be NULL): presorted. */
 size_t vpm_adjoint_workspace_bytes(int64_t n, const vpm_forward_opts_t* opts);
 int vpm_adjoint(const vpm_particles_t* p, const vpm_adjoint_in_t* in,
                 const vpm_forward_opts_t* opts, vpm_adjoint_out_t* out, void* workspace,

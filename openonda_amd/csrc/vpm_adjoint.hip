@@ -272,7 +272,7 @@ int adj64_run(const RowArgs& a, unsigned mask, const double* rec, void* part, si
 constexpr int64_t kAdjRowsMax = 5120;
 
 bool adj_rows_wanted(int64_t n, const vpm_forward_opts_t* o) {
-  return !o || o->precision == VPM_PREC_F64 || n <= kAdjRowsMax;
+  return o->precision == VPM_PREC_F64 || n <= kAdjRowsMax;
 }
 
 struct AdjLayout {
@@ -400,10 +400,18 @@ using namespace vpm;
 
 extern "C" {
 
+// Enough for either precision, so that one workspace serves both.
 size_t vpm_adjoint_workspace_bytes(int64_t n, const vpm_forward_opts_t* opts) {
-  AdjLayout L{};
-  if (adj_layout(n, opts, &L) != VPM_OK) return 0;
-  return L.total;
+  vpm_forward_opts_t o{};
+  o.presorted = opts ? opts->presorted : 0;
+  size_t most = 0;
+  for (const int precision : {VPM_PREC_F64, VPM_PREC_F32C}) {
+    o.precision = precision;
+    AdjLayout L{};
+    if (adj_layout(n, &o, &L) != VPM_OK) return 0;
+    most = std::max(most, L.total);
+  }
+  return most;
 }
 
 int vpm_adjoint(const vpm_particles_t* p, const vpm_adjoint_in_t* in, const vpm_forward_opts_t* o,

@@ -2,8 +2,9 @@
 call writes.
 
 Host part: the row pass writes the same records and chunk boxes for a uniform
-radius as for per-particle radii, so both need the same workspace.  GPU part:
-every output set, and the library's autotuner, in a workspace of exactly the
+radius as for per-particle radii, so both need the same workspace; the
+adjoint's query serves both precisions.  GPU part: every output set, the
+adjoint, a batch and the library's autotuner in a workspace of exactly the
 queried size, with guard bytes behind it.
 """
 import ctypes as C
@@ -28,6 +29,18 @@ def test_row_pass_workspace_does_not_depend_on_the_radius_mode(mask, presorted):
     for n in (8192, 8193, 9000, 20011, 34914, 65536) + ((300001, 1 << 20) if presorted else ()):
         uniform = forward_bytes(n, mask, L.SIGMA_UNIFORM, presorted)
         assert uniform == forward_bytes(n, mask, L.SIGMA_GENERAL, presorted) > 0, (n, mask)
+
+
+@pytest.mark.parametrize("n", [1, 5120, 5121, 9000, 20011, 65536])
+def test_adjoint_workspace_serves_every_precision(n):
+    """One query, with any options or none, covers every call on n particles
+    in the caller's order."""
+    lib = L.load()
+    sizes = [lib.vpm_adjoint_workspace_bytes(n, None)]
+    for precision in (L.PREC_F64, L.PREC_F32C):
+        o = L.ForwardOpts(3, precision, L.SIGMA_UNIFORM, 0, -1)
+        sizes.append(lib.vpm_adjoint_workspace_bytes(n, C.byref(o)))
+    assert len(set(sizes)) == 1 and sizes[0] > 0
 
 
 GUARD = 1 << 16
@@ -92,3 +105,60 @@ def test_autotune_accepts_the_workspace_it_asks_for(gpu, mask, n, general):
            P._stream(d[0]), 1, C.byref(best), None)
     assert 0 <= best.value < L.load().vpm_tile_config_count()
     assert bool((ws[nb:] == 0xA5).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("general", [False, True])
+@pytest.mark.parametrize("n", [1, 700, 5120, 5121, 9000, 20011, 66001])
+def test_adjoint_stays_inside_its_workspace(gpu, n, general):
+    import torch
+
+    from openonda_amd import flow_models as FM
+    from openonda_amd import physics as P
+
+    x, a, s, _ = FM.random_cloud(n, seed=n)
+    d = (P.to_soa(x), P.to_soa(a), torch.from_numpy(s).cuda(),
+         torch.full((n,), 1e-3, dtype=torch.float64, device="cuda"))
+    p = P._particles(*d)
+    cot = torch.ones((3, 3, n), dtype=torch.float64, device="cuda")
+    out = torch.zeros((2, 3, n), dtype=torch.float64, device="cuda")
+    for precision in (L.PREC_F32C, L.PREC_F64):
+        for presorted in (0, 1):
+            print(f"[workspace] adjoint n={n} general={general} precision={precision} "
+                  f"presorted={presorted}", flush=True)
+            o = L.ForwardOpts(3, precision, L.SIGMA_GENERAL if general else L.SIGMA_UNIFORM,
+                              presorted, -1)
+            nb = L.load().vpm_adjoint_workspace_bytes(n, C.byref(o))
+            ws = torch.full((nb + GUARD,), 0xA5, dtype=torch.uint8, device="cuda")
+            ci = L.AdjointIn(n, *[cot[q].data_ptr() for q in range(3)])
+            co = L.AdjointOut(n, out[0].data_ptr(), out[1].data_ptr())
+            L.call("vpm_adjoint", C.byref(p), C.byref(ci), C.byref(o), C.byref(co),
+                   ws.data_ptr(), nb, P._stream(d[0]))
+            assert bool((ws[nb:] == 0xA5).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [[1], [64, 0, 65, 3], [50] * 40, [9000, 128, 5001], [20011]],
+                         ids=str)
+def test_batch_stays_inside_its_workspace(gpu, sizes):
+    import torch
+
+    from openonda_amd import batch as B
+    from openonda_amd import flow_models as FM
+
+    sets = []
+    for i, n in enumerate(sizes):
+        x, a, s, _ = FM.random_cloud(max(n, 1), seed=i)
+        sets.append((x[:n], a[:n], s[:n], np.full(n, 1e-3)))
+    for rows in (True, False):
+        for les in (True, False):
+            print(f"[workspace] batch {sizes[:4]} rows={rows} les={les}", flush=True)
+            bs = B.BatchedSystem(sets, dt=0.01, les=les)
+            bs.set_launch(bs.tile_config, rows=rows)
+            nb = L.load().vpm_batch_workspace_bytes(bs.n, bs.nsets, bs.desc.n_items)
+            bs.ws = torch.full((nb + GUARD,), 0xA5, dtype=torch.uint8, device="cuda")
+            bs.wsb = nb
+            torch.cuda.synchronize()
+            bs.evaluate(bs.x, bs.a, bs.stage_mask, True, bs.stream.cuda_stream)
+            bs.synchronize()
+            assert bool((bs.ws[nb:] == 0xA5).all())
