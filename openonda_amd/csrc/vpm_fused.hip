@@ -1,6 +1,6 @@
 // Tiled all-pairs forward pass: the batched launch, the tile shapes a caller
-// asks for by index, and sets too large for vpm_forward_noalloc's array with
-// the row pass's records.  (Other single-set calls run vpm_row32.hip or
+// asks for by index, and sets without the far form that are too large for
+// vpm_forward_noalloc's array with the row pass's records.  (Other single-set calls run vpm_row32.hip or
 // vpm_forward_rows.hip.)
 //
 // One pass over all (target, source) pairs computes any subset of the GPU
@@ -1409,7 +1409,7 @@ int layout(int64_t n, const vpm_forward_opts_t* o, WsLayout* L, bool need_cub = 
   };
   L->bbox_part = take(kBboxBlocks * 6 * sizeof(double));
   L->bbox = take(8 * sizeof(double));
-  L->keys_in = take((N + kSamples) * sizeof(uint32_t));
+  L->keys_in = take((n <= kBlockSortMax ? N + kSamples : N) * sizeof(uint32_t));
   L->keys_out = take(N * sizeof(uint32_t));
   L->idx_in = take(N * sizeof(int));
   L->perm = take(N * sizeof(int));
@@ -2128,7 +2128,8 @@ int vpm_forward_noalloc(const vpm_particles_t* p, const vpm_forward_opts_t* o,
   WsLayout L{};
   if ((rc = layout(p->n, o, &L, true, 0))) return rc;
   // sets whose records of the row pass no longer fit run the tiled kernels,
-  // which need none
+  // which need none unless their far form applies (wants_far_records: then
+  // theirs are as large, and this changes nothing)
   vpm_forward_opts_t tiled = *o;
   if (L.total > kScratchBytes && row32_asked(o)) {
     tiled.tile_config = default_config(kernel_mask(o->outputs),

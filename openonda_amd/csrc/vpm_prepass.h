@@ -247,7 +247,8 @@ __global__ void fill_kernel(double* __restrict__ p, int64_t n, double v) {
 // Sorts particles by Morton key of their position.  Returns the permutation
 // (sorted k -> caller index) in `perm` and, if `rec` is not null, the packed
 // records in that order.  Scratch: bbox_part (kBboxBlocks*6), bbox (8),
-// kin (n + kSamples), kout/iin (n each) and cub_bytes of hipCUB storage.
+// kin (n, and kSamples more up to kBlockSortMax), kout/iin (n each) and
+// cub_bytes of hipCUB storage.
 inline int morton_sort(const vpm_particles_t* p, double* bbox_part, double* bbox, uint32_t* kin,
                        uint32_t* kout, int* iin, int* perm, void* cub, size_t cub_bytes, Src8* rec,
                        hipStream_t st) {

@@ -31,6 +31,16 @@ def test_row_pass_workspace_does_not_depend_on_the_radius_mode(mask, presorted):
         assert uniform == forward_bytes(n, mask, L.SIGMA_GENERAL, presorted) > 0, (n, mask)
 
 
+def test_largest_allocation_free_set():
+    """A set without source splits needs 104 bytes per particle, 8 more per 64 of
+    them, and 25 KB: 2,577,764 particles in the caller's order fit the
+    allocation-free call's 256 MiB."""
+    assert L.load().vpm_forward_noalloc_capacity() == 256 << 20
+    for mask, precision, tile in ((3, L.PREC_F64, -1), (31, L.PREC_F32C, 1)):
+        at = lambda n: forward_bytes(n, mask, L.SIGMA_GENERAL, 1, tile, precision)
+        assert at(2577764) <= 256 << 20 < at(2577765)
+
+
 @pytest.mark.parametrize("n", [1, 5120, 5121, 9000, 20011, 65536])
 def test_adjoint_workspace_serves_every_precision(n):
     """One query, with any options or none, covers every call on n particles
