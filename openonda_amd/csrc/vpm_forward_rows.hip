@@ -1,6 +1,6 @@
 // The fused forward pass in FP64 over the rows of vpm_rows.h: any subset of
 // the GPU plugin's outputs from one inverse root per pair, in the caller's
-// order (no sort, no packed records).
+// order (no sort; packed records from kRowRecordsMin particles on).
 //
 // It is the FP64 pass at every size, and the FP32-compensated pass's stand-in
 // for small sets (forward_rows_wanted), where the sort, the records and the
@@ -143,7 +143,7 @@ struct OpForward {
 };
 
 template <unsigned OUT, bool UNIF>
-int launch(const vpm_particles_t* p, const vpm_forward_opts_t* o, vpm_forward_out_t* out,
+int launch(const vpm_particles_t* p, const Src8* rec, const vpm_forward_opts_t* o, vpm_forward_out_t* out,
            double* ens_part, void* split, size_t split_bytes, hipStream_t st) {
   using Op = OpForward<OUT, UNIF>;
   RowArgs a{};
@@ -153,6 +153,7 @@ int launch(const vpm_particles_t* p, const vpm_forward_opts_t* o, vpm_forward_ou
   a.tld = a.ld = a.tqld = a.qld = p->ld;
   a.ts = a.s = p->sigma;
   a.tnu = a.nu = p->nu;
+  a.rec = rec;
   int v = 0;
   const unsigned want = o->outputs;
   if constexpr (Op::vel) a.out[v++] = (want & VPM_OUT_VEL) ? out->vel : nullptr;
@@ -163,8 +164,8 @@ int launch(const vpm_particles_t* p, const vpm_forward_opts_t* o, vpm_forward_ou
   a.sums = ens_part;
   double* sums = nullptr;
   int64_t nsums = 0;
-  const int rc = row_launch<Op>(a, split, split_bytes, st, "forward_rows", o->max_splits, &sums,
-                                &nsums);
+  const int rc = row_launch<Op, true>(a, split, split_bytes, st, "forward_rows", o->max_splits,
+                                      &sums, &nsums);
   if (rc) return rc;
   if (want & VPM_OUT_ENSTROPHY) {
     const double k = (1.0 / (8.0 * kPi)) * kOneOverFourPi;
@@ -176,11 +177,11 @@ int launch(const vpm_particles_t* p, const vpm_forward_opts_t* o, vpm_forward_ou
 }
 
 template <unsigned OUT>
-int launch_mode(const vpm_particles_t* p, const vpm_forward_opts_t* o, vpm_forward_out_t* out,
-                double* ens_part, void* split, size_t split_bytes, hipStream_t st) {
+int launch_mode(const vpm_particles_t* p, const Src8* rec, const vpm_forward_opts_t* o,
+                vpm_forward_out_t* out, double* ens_part, void* split, size_t split_bytes, hipStream_t st) {
   return o->sigma_mode == VPM_SIGMA_UNIFORM
-             ? launch<OUT, true>(p, o, out, ens_part, split, split_bytes, st)
-             : launch<OUT, false>(p, o, out, ens_part, split, split_bytes, st);
+             ? launch<OUT, true>(p, rec, o, out, ens_part, split, split_bytes, st)
+             : launch<OUT, false>(p, rec, o, out, ens_part, split, split_bytes, st);
 }
 
 int row_outputs(unsigned mask) {
@@ -195,17 +196,17 @@ size_t forward_rows_split_bytes(int64_t n, unsigned mask) {
   return row_workspace_bytes(n, n, row_outputs(mask), (mask & VPM_OUT_ENSTROPHY) != 0);
 }
 
-int forward_rows(const vpm_particles_t* p, const vpm_forward_opts_t* o, vpm_forward_out_t* out,
-                 unsigned mask, double* ens_part, void* split, size_t split_bytes,
+int forward_rows(const vpm_particles_t* p, const Src8* rec, const vpm_forward_opts_t* o,
+                 vpm_forward_out_t* out, unsigned mask, double* ens_part, void* split, size_t split_bytes,
                  hipStream_t st) {
   switch (mask) {
 #define VPM_ROWS(M) \
-  case M: return launch_mode<M>(p, o, out, ens_part, split, split_bytes, st);
+  case M: return launch_mode<M>(p, rec, o, out, ens_part, split, split_bytes, st);
     VPM_ROWS(1u) VPM_ROWS(2u) VPM_ROWS(3u) VPM_ROWS(4u) VPM_ROWS(7u) VPM_ROWS(8u) VPM_ROWS(16u)
     VPM_ROWS(24u) VPM_ROWS(26u)
     VPM_ROWS(27u)
 #undef VPM_ROWS
-    default: return launch_mode<31u>(p, o, out, ens_part, split, split_bytes, st);
+    default: return launch_mode<31u>(p, rec, o, out, ens_part, split, split_bytes, st);
   }
 }
 

@@ -1949,20 +1949,6 @@ int check_forward_out(const vpm_particles_t* p, const vpm_forward_opts_t* o,
   return VPM_OK;
 }
 
-// Positions, strengths, radii and viscosities one behind the other.
-__global__ __launch_bounds__(kPreBlock) void copy_particles_kernel(const vpm_particles_t p,
-                                                                   double* __restrict__ out) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kPreBlock + threadIdx.x;
-  if (i >= p.n) return;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    out[c * p.n + i] = p.pos[c * p.ld + i];
-    out[(3 + c) * p.n + i] = p.str[c * p.ld + i];
-  }
-  out[6 * p.n + i] = p.sigma[i];
-  out[7 * p.n + i] = p.nu ? p.nu[i] : 0.0;
-}
-
 // Whether a requested output lies over one of the inputs.
 bool writes_inputs(const vpm_particles_t* p, const vpm_forward_opts_t* o,
                    const vpm_forward_out_t* out) {
@@ -1998,17 +1984,17 @@ int forward_run_impl(const vpm_particles_t* p, const vpm_forward_opts_t* o,
   const unsigned mask = forward_rows_wanted(n, o) || row32_asked(o) ? row_mask(want)
                                                                      : kernel_mask(want);
   if (forward_rows_wanted(n, o)) {
-    // These rows read the caller's arrays while others are stored: outputs in
-    // the inputs' place are summed from a copy, in the records' region.
-    vpm_particles_t q = *p;
-    if (writes_inputs(p, o, out)) {
-      double* c = reinterpret_cast<double*>(ws + L.src8);
-      hipLaunchKernelGGL(copy_particles_kernel, dim3(static_cast<unsigned>(ceil_div(n, kPreBlock))),
-                         dim3(kPreBlock), 0, st, *p, c);
-      VPM_LAUNCH_CHECK("copy_particles_kernel");
-      q = vpm_particles_t{n, n, c, c + 3 * n, c + 6 * n, c + 7 * n};
+    // These rows read the particles while others are stored: outputs in the
+    // inputs' place are summed from records.
+    Src8* rec = nullptr;
+    if (n >= kRowRecordsMin || writes_inputs(p, o, out)) {
+      rec = reinterpret_cast<Src8*>(ws + L.src8);
+      hipLaunchKernelGGL(gather_kernel, dim3(static_cast<unsigned>(ceil_div(n, kPreBlock))),
+                         dim3(kPreBlock), 0, st, *p, static_cast<int>(n),
+                         static_cast<const int*>(nullptr), rec);
+      VPM_LAUNCH_CHECK("gather_kernel");
     }
-    return forward_rows(&q, o, out, mask, reinterpret_cast<double*>(ws + L.ens_part),
+    return forward_rows(p, rec, o, out, mask, reinterpret_cast<double*>(ws + L.ens_part),
                         L.split_bytes ? ws + L.split : nullptr, L.split_bytes, st);
   }
   // Unrequested outputs of a superset kernel share one scratch region; a
@@ -2157,7 +2143,7 @@ int vpm_forward_noalloc(const vpm_particles_t* p, const vpm_forward_opts_t* o,
 
 int vpm_forward(const vpm_particles_t* p, const vpm_forward_opts_t* o, vpm_forward_out_t* out,
                 void* workspace, size_t ws_bytes, void* stream) {
-  // the rows read the particles in the caller's order: nothing to prepare
+  // the rows run in the caller's order: no sort to prepare
   if (p && o && forward_rows_wanted(p->n, o))
     return vpm_forward_run(p, o, out, workspace, ws_bytes, stream);
   int rc = vpm_forward_prepare(p, o, workspace, ws_bytes, stream);

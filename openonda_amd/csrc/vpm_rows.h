@@ -62,6 +62,7 @@ struct RowArgs {
   int64_t qld;
   const double* s;      // [n]
   const double* nu;     // [n]
+  const Src8* rec;      // self evaluations over records: the particles, else null
   double* out[4];       // vector outputs, [3][ld_out] each; a null one is not stored
   int64_t ld_out;
   double* part;         // split partials [split][component][rows * 64], or null
@@ -85,6 +86,7 @@ typedef __attribute__((address_space(4))) const double scalar_double_t;
 // Scalar-loaded view of the sources.
 template <class Op>
 struct RowSources {
+  static constexpr bool kRecords = false;
   scalar_double_t *x, *y, *z, *ax, *ay, *az, *s, *nu;
   __device__ explicit RowSources(const RowArgs& a) {
     x = (scalar_double_t*)a.pos;
@@ -104,14 +106,33 @@ struct RowSources {
   }
 };
 
+// The same of packed records: one 64-byte line per source where the arrays
+// take one of each, which evict one another where the arrays lie a multiple of
+// 256 KiB apart (see kRowRecordsMin in vpm_forward_rows.h).
+template <class Op>
+struct RowRecords {
+  static constexpr bool kRecords = true;
+  scalar_double_t* r;
+  __device__ explicit RowRecords(const RowArgs& a) {
+    r = (scalar_double_t*)reinterpret_cast<const double*>(a.rec);
+  }
+  __device__ __forceinline__ RowSource at(int64_t j) const {
+    scalar_double_t* q = r + j * 8;
+    RowSource v{q[0], q[1], q[2], q[3], q[4], q[5], 0.0, 0.0};
+    if constexpr (Op::kRadius) v.s = q[6];
+    if constexpr (Op::kNu) v.nu = q[7];
+    return v;
+  }
+};
+
 // Sources [j, j1) that need a test per pair: pair(k, source) for each k.  Two
 // loads in flight: one at a time, every source cost its load's whole latency,
 // and the wave with the row's own particles held up its workgroup (FP64
 // velocity + stretching of 4,096 particles 36.5 -> 34.4 us, LES step of 4,001
 // 140.5 -> 138.7); four spill scalar registers (all outputs but PSE of 2,503
 // particles 31.6 us with one, 31.0 with two, 32.0 with four).
-template <class Op, class F>
-__device__ __forceinline__ void row_few(const RowSources<Op>& src, int64_t j, int64_t j1, F pair) {
+template <class Src, class F>
+__device__ __forceinline__ void row_few(const Src& src, int64_t j, int64_t j1, F pair) {
   for (; j1 - j >= 2; j += 2) {
     const RowSource s0 = src.at(j), s1 = src.at(j + 1);
     pair(j, s0);
@@ -120,9 +141,9 @@ __device__ __forceinline__ void row_few(const RowSources<Op>& src, int64_t j, in
   if (j < j1) pair(j, src.at(j));
 }
 
-template <class Op>
+template <class Op, class Src>
 __device__ __forceinline__ void row_sweep(typename Op::Acc& acc, const RowTarget& t,
-                                          const RowSources<Op>& src, int64_t j, int64_t j1) {
+                                          const Src& src, int64_t j, int64_t j1) {
   for (; j1 - j >= kRowGroup; j += kRowGroup) {
     RowSource s[kRowGroup];
 #pragma unroll
@@ -143,12 +164,17 @@ __device__ __forceinline__ void row_share(int64_t lo, int64_t hi, int k, int par
   *e = hi - *b < per ? hi : *b + per;
 }
 
-template <class Op>
+template <class Op, bool RECORDS = false>
 __device__ __forceinline__ RowTarget row_target(const RowArgs& a, int64_t i) {
   RowTarget t{};
   t.i = i;
   t.s = 1.0;
-  if (i < a.m) {
+  if constexpr (RECORDS) {
+    if (i < a.m) {
+      const Src8 r = a.rec[i];
+      t = RowTarget{r.x, r.y, r.z, r.ax, r.ay, r.az, r.s, 0.0, r.nu, i};
+    }
+  } else if (i < a.m) {
     t.x = a.tpos[i];
     t.y = a.tpos[a.tld + i];
     t.z = a.tpos[2 * a.tld + i];
@@ -165,10 +191,9 @@ __device__ __forceinline__ RowTarget row_target(const RowArgs& a, int64_t i) {
 }
 
 // Sources [b, e) against one target per lane, the row at row0.
-template <class Op>
+template <class Op, class Src>
 __device__ __forceinline__ void row_range(typename Op::Acc& acc, const RowTarget& t,
-                                          const RowSources<Op>& src, int64_t row0, int64_t b,
-                                          int64_t e) {
+                                          const Src& src, int64_t row0, int64_t b, int64_t e) {
   if constexpr (Op::kSkipSelf) {  // the row's own particles [o0, o1): j != i
     const int64_t o0 = row0 < b ? b : (row0 < e ? row0 : e);
     const int64_t o1 = row0 + kRow < b ? b : (row0 + kRow < e ? row0 + kRow : e);
@@ -196,7 +221,7 @@ __device__ __forceinline__ void row_store(const RowArgs& a, int na, int q, int64
 }
 
 // Vector operators.  grid (rows, splits).
-template <class Op>
+template <class Op, class Src>
 __global__ __launch_bounds__(kRowBlock, 4) void row_kernel(RowArgs a) {
   constexpr int NA = Op::kOut;               // vector components
   constexpr int NV = NA + (Op::kSum ? 1 : 0);  // + one scalar summed over the targets
@@ -204,8 +229,8 @@ __global__ __launch_bounds__(kRowBlock, 4) void row_kernel(RowArgs a) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kRow;
-  const RowTarget t = row_target<Op>(a, row0 + lane);
-  const RowSources<Op> src(a);
+  const RowTarget t = row_target<Op, Src::kRecords>(a, row0 + lane);
+  const Src src(a);
   int64_t b, e;
   row_share(0, a.n, static_cast<int>(blockIdx.y) * kRowWaves + wave, a.splits * kRowWaves, &b, &e);
   typename Op::Acc acc{};
@@ -264,13 +289,16 @@ __global__ __launch_bounds__(kRowBlock, 4) void row_wide_kernel(RowArgs a, int r
   }
 }
 
-// When a row per wave pays: the component arrays lie a multiple of 4 MiB
-// apart, so a source's seven values fall into the same cache sets, and eight
-// waves at eight places of them evict each other's lines.  Velocity of 2^20
-// particles 1349 -> 1033 ms (2^20 + 24: 958 without), velocity + stretching
-// 2037 -> 1329 (1468 as the tiled FP64 pass with sorted records).  Other
-// strides keep the eight-fold split: 600,011 particles 332 ms against 375,
-// 1,300,021 1549 against 1582; 2^18, 2 MiB apart, 62 against 64.
+// When a row per wave pays (sums over arrays; the fused pass has records
+// there): the component arrays lie a multiple of 4 MiB apart, so a source's
+// seven values fall into the same cache sets, and eight waves at eight places
+// of them evict each other's lines.  Velocity of 2^20 particles 1465 -> 1066 ms,
+// of 2^19 327 -> 262; stretching of 2^20 2343 -> 1649.  2^18, 2 MiB apart, keeps
+// the eight-fold split: 62 ms against 65.  Odd multiples of 2 MiB and less are
+// not in the rule, though they collide from 393,216 particles on (786,432: 832
+// ms, 579 with a row per wave; 425,984: 217 and 214).  row_splits, made for
+// eight waves that share a row's sources, is not tuned for this kernel: these
+// sizes have rows enough for one or two splits.
 constexpr int64_t kWideStride = int64_t{1} << 19, kWideMin = int64_t{1} << 18;
 inline bool row_wide_wanted(const RowArgs& a, int64_t rows) {
   return a.ld % kWideStride == 0 && a.n >= kWideMin && rows >= kWideMin / kRow;
@@ -363,8 +391,8 @@ inline size_t row_workspace_bytes(int64_t m, int64_t n, int na, bool sum = false
 // ws may be null or smaller than row_workspace_bytes: fewer splits then.
 // max_splits: 0 or the most splits to use.  kSum operators write one partial
 // per workgroup to a.sums (room for the rows), or behind the split partials;
-// *sums and *nsums say where and how many.
-template <class Op>
+// *sums and *nsums say where and how many.  RECORDS: a.rec may be set.
+template <class Op, bool RECORDS = false>
 int row_launch(RowArgs a, void* ws, size_t ws_bytes, hipStream_t st, const char* name,
                int max_splits = 0, double** sums = nullptr, int64_t* nsums = nullptr) {
   if (a.m == 0) return VPM_OK;
@@ -381,13 +409,21 @@ int row_launch(RowArgs a, void* ws, size_t ws_bytes, hipStream_t st, const char*
     *sums = a.sums;
     *nsums = rows * k;
   }
-  if (row_wide_wanted(a, rows))
+  const dim3 grid(static_cast<unsigned>(rows), k);
+  bool records = false;
+  if constexpr (RECORDS) {
+    records = a.rec != nullptr;
+    if (records)
+      hipLaunchKernelGGL((row_kernel<Op, RowRecords<Op>>), grid, dim3(kRowBlock), 0, st, a);
+  }
+  if (records)
+    ;
+  else if (row_wide_wanted(a, rows))
     hipLaunchKernelGGL(row_wide_kernel<Op>,
                        dim3(static_cast<unsigned>(ceil_div(rows, kRowWaves)), k), dim3(kRowBlock),
                        0, st, a, static_cast<int>(rows));
   else
-    hipLaunchKernelGGL(row_kernel<Op>, dim3(static_cast<unsigned>(rows), k), dim3(kRowBlock), 0,
-                       st, a);
+    hipLaunchKernelGGL((row_kernel<Op, RowSources<Op>>), grid, dim3(kRowBlock), 0, st, a);
   VPM_LAUNCH_CHECK(name);
   if (k > 1 && Op::kOut > 0) {
     hipLaunchKernelGGL(row_reduce_kernel, dim3(static_cast<unsigned>(ceil_div(a.m, 256)), Op::kOut),
