@@ -66,8 +66,11 @@ constexpr int kRow32Waves = 6;
 // stretching + PSE, cloud of 131,072: 11.4 against 12.5 ms, ring 13.4 against
 // 13.8).  Chunks of 128 sources halve the moment form's set-up and fold per chunk;
 // with the LES outputs 64 keep the vorticity's partials as short as they were
-// (rel-L2 1.0e-7 against 1.5e-7 on a ring of 20,000).
-template <unsigned OUT, bool UNIF>
+// (rel-L2 1.0e-7 against 1.5e-7 on a ring of 20,000), and in a batch every
+// output's, whose tiled launch folds 64 (velocity of 24 sets, mean rel-L2
+// 1.14e-7 with 64, 1.56e-7 with 128, tiled 1.45e-7; a stage with PSE 4.29 and
+// 4.34 ms, tiled 7.37).
+template <unsigned OUT, bool UNIF, bool BATCH = false>
 struct Rec32 {
   static constexpr bool kLo = OUT & VPM_OUT_PSE;
   static constexpr bool kMoment = UNIF && (OUT & VPM_OUT_VEL) && (OUT & VPM_OUT_STRETCH);
@@ -84,7 +87,7 @@ struct Rec32 {
   static constexpr int kGroup = kLo ? 2 : kMaxGroup32;
   static constexpr int kNear = kLo ? 4 : 2;  // sources in flight in the FP64 loop
   static constexpr int kChunk =
-      kMoment && !(OUT & (VPM_OUT_VORT | VPM_OUT_ENSTROPHY)) ? kMaxChunk32 : kMinChunk32;
+      kMoment && !BATCH && !(OUT & (VPM_OUT_VORT | VPM_OUT_ENSTROPHY)) ? kMaxChunk32 : kMinChunk32;
 };
 
 __device__ __forceinline__ double held(double v) {  // rounded here, not fused into its use
@@ -97,10 +100,10 @@ __device__ __forceinline__ double held(double v) {  // rounded here, not fused i
 // zero-strength padding far away, which adds exactly 0.  The box is that of
 // the finite coordinates: a particle at infinity keeps an infinite offset (PSE
 // and vorticity weigh it 0) and leaves its chunk's others theirs.
-template <unsigned OUT, bool UNIF>
+template <unsigned OUT, bool UNIF, bool BATCH>
 __device__ __forceinline__ void row32_records(const Src8* __restrict__ src, int n, int c,
                                               float* __restrict__ rec, double* __restrict__ box_) {
-  using R = Rec32<OUT, UNIF>;
+  using R = Rec32<OUT, UNIF, BATCH>;
   __shared__ double red[7][R::kChunk / 64];
   const int k = c * R::kChunk + static_cast<int>(threadIdx.x);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -175,7 +178,7 @@ __device__ __forceinline__ void row32_records(const Src8* __restrict__ src, int 
 template <unsigned OUT, bool UNIF>
 __global__ __launch_bounds__((Rec32<OUT, UNIF>::kChunk)) void row32_records_kernel(
     const Src8* __restrict__ src, int n, float* __restrict__ rec, double* __restrict__ box) {
-  row32_records<OUT, UNIF>(src, n, static_cast<int>(blockIdx.x), rec, box);
+  row32_records<OUT, UNIF, false>(src, n, static_cast<int>(blockIdx.x), rec, box);
 }
 
 struct Tgt32 {
@@ -372,7 +375,7 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
       return;
     }
     const int64_t c0 = b.chunk0[it.set];
-    rec_ = b.rec + c0 * Rec32<OUT, UNIF>::kChunk * Rec32<OUT, UNIF>::kStride;
+    rec_ = b.rec + c0 * Rec32<OUT, UNIF, BATCH>::kChunk * Rec32<OUT, UNIF, BATCH>::kStride;
     box_ = b.box + c0 * kBox32;
     n = it.n;
     row = it.row;
@@ -381,7 +384,7 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
     if (part_out) part_out += it.off;
   }
   using S = Slots<OUT>;
-  using R = Rec32<OUT, UNIF>;
+  using R = Rec32<OUT, UNIF, BATCH>;
   constexpr int NS = S::nslot, CH = R::kChunk;
   // FP64 totals of each wave's share (kept here, not in registers: they are
   // touched once per chunk) and, at the end, their sums
@@ -629,9 +632,9 @@ __global__ __launch_bounds__(1024) void row32_chunks_kernel(const int* __restric
 
 // Workgroup g builds chunk g of all sets' chunks (its set by binary search).
 template <unsigned OUT>
-__global__ __launch_bounds__((Rec32<OUT, true>::kChunk)) void row32_set_records_kernel(
+__global__ __launch_bounds__((Rec32<OUT, true, true>::kChunk)) void row32_set_records_kernel(
     Row32Batch b, const Src8* __restrict__ src) {
-  using R = Rec32<OUT, true>;
+  using R = Rec32<OUT, true, true>;
   const int g = blockIdx.x;
   if (g >= b.chunk0[b.nsets]) return;  // uniform over the workgroup
   int lo = 0, hi = b.nsets - 1;
@@ -642,7 +645,7 @@ __global__ __launch_bounds__((Rec32<OUT, true>::kChunk)) void row32_set_records_
   }
   const int off = b.set_off[lo];
   const int64_t c0 = b.chunk0[lo];
-  row32_records<OUT, true>(src + off, b.set_off[lo + 1] - off, g - static_cast<int>(c0),
+  row32_records<OUT, true, true>(src + off, b.set_off[lo + 1] - off, g - static_cast<int>(c0),
                            b.rec + c0 * R::kChunk * R::kStride, b.box + c0 * kBox32);
 }
 
@@ -713,7 +716,7 @@ int launch(FusedArgs a, float* rec, double* box, hipStream_t st, int* nblocks) {
 
 template <unsigned OUT>
 int launch_batch(FusedArgs a, const Row32Batch& b, hipStream_t st) {
-  using R = Rec32<OUT, true>;
+  using R = Rec32<OUT, true, true>;
   const int64_t groups = static_cast<int64_t>(b.n_items) * b.rows_per_item;
   if (groups == 0 || a.n == 0) return VPM_OK;
   const int k = a.part ? b.splits : 1;
