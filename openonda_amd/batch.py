@@ -44,16 +44,36 @@ def work_list(sizes, targets_per_item):
     return (np.array(item_set, dtype=np.int32), np.array(item_block, dtype=np.int32), first, count)
 
 
+def row_pass_pays(sizes) -> bool:
+    """Whether the row pass outruns the persistent tiled launch on sets of these
+    sizes (RK4 steps, half rings and half clouds, tiled / rows).
+
+    A row's eight waves share its set's sources: a few hundred leave most of
+    them idle (100,000 particles in sets of 130 534 / 678 us, 20,000 in sets of
+    130 290 / 330, of 300 363 / 333).  The tiled launch gives a set's target
+    blocks one workgroup each and needs more than a set per CU (256) to fill
+    the device: up to that many sets the rows win (100,000 particles in sets of
+    400 620 / 604, of 1,000 1052 / 880), beyond it from 1,500 particles per set
+    on (400,000 in sets of 500 1564 / 1653, of 1,000 2637 / 2700, of 1,500 3557 /
+    3241).  Sets of uneven size count by their pairs.
+    """
+    n = np.asarray(sizes, dtype=np.float64)
+    if n.sum() == 0:
+        return True
+    size = float((n * n).sum() / n.sum())
+    return bool(size >= 256 and (n.sum() <= 256 * size or size >= 1500))
+
+
 class BatchedSystem:
     """Particle sets [(x (N_i,3), alpha (N_i,3), sigma (N_i,), nu (N_i,)), ...]."""
 
     def __init__(self, sets, dt, precision="f32c", tile_config=-1, pse=True, les=True,
                  device=None, grid=0, resort_every=0, autotune_cache=None):
-        """``tile_config``: -1 (rows of 64 targets, one workgroup each), an
-        index of physics.tile_configs() (the persistent tiled launch), or
-        "auto" (the batch autotuner's
-        cached (shape, grid) for this output set and total pair count, else
-        the default).  ``grid``: persistent workgroups (0: as many as fit on
+        """``tile_config``: -1 (rows of 64 targets, one workgroup each, where
+        :func:`row_pass_pays`, else the persistent tiled launch in its default
+        shape), an index of physics.tile_configs() (the tiled launch in that
+        shape), or "auto" (the batch autotuner's cached (shape, grid) for this
+        output set and total pair count, else the default).  ``grid``: persistent workgroups (0: as many as fit on
         the device).  ``resort_every``: re-sort the sets by Morton key every
         that many steps, eager or replayed (0: only at the first step)."""
         P.require_gpu()
@@ -76,7 +96,7 @@ class BatchedSystem:
 
             self.autotuned = autotune.best_batch_config(sizes, self.stage_mask, path=autotune_cache)
             tile_config, grid = self.autotuned if self.autotuned else (-1, grid)
-        rows = tile_config < 0 and grid == 0 and precision == "f32c"
+        rows = tile_config < 0 and grid == 0 and precision == "f32c" and row_pass_pays(sizes)
         self.tile_config = (int(tile_config) if tile_config >= 0
                             else int(L.load().vpm_batch_tile_config_default(self.stage_mask)))
         for k, s in enumerate(sets):

@@ -208,3 +208,12 @@ def test_pageable_upload_is_a_blocking_copy(monkeypatch):
     assert asked == [False]
     assert np.array_equal(dx.numpy(), x.T) and np.array_equal(da.numpy(), a.T)
     assert np.array_equal(ds.numpy(), s)
+
+
+@pytest.mark.parametrize("sizes,rows", [
+    ([300], True), ([40000], True), ([64] * 2, False), ([50] * 300, False), ([60] * 3000, False),
+    ([130] * 769, False), ([300] * 66, True), ([500] * 200, True), ([500] * 800, False),
+    ([1500] * 266, True), ([30000] * 96, True), ([1, 63, 64, 129, 3000], True), ([], True),
+    ([0, 0], True)])
+def test_batches_of_small_sets_keep_the_tiled_launch(sizes, rows):
+    assert B.row_pass_pays(sizes) is rows
