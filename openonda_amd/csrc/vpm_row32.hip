@@ -13,13 +13,12 @@
 // wait in LDS meanwhile.
 //
 // Far chunks (gap between the row's and the chunk's boxes above kFarGap32
-// times the larger radius) of sets with velocity, stretching and a uniform
-// radius take the moment form (pair_far).  Stretching: rows of coherent
+// times the larger radius) of sets with stretching, another output and a
+// uniform radius take the moment form (pair_far).  Stretching: rows of coherent
 // strengths (coherent_wave) take the sum of g alpha_j and the triple product
 // in FP64, the others in FP32, as in the tiled kernels (vpm_fused.hip, which
 // also measures why); sets with vorticity or enstrophy and without PSE sum in
-// FP64 in every row.  With a uniform radius and more outputs than the
-// stretching, far chunks are summed in FP32 in every row (kFarFp32).
+// FP64 in every row.  The moment form is FP32 in every row.
 //
 // With s = sigma_ij, D = r^2 + s^2, t = D^-1/2 and w = s^2 t^2 no reciprocal
 // of s is needed: (rho^2 + 2.5) / (A^5/2 s^3) = t^3 (1 + 1.5 w) and so on
@@ -73,15 +72,14 @@ constexpr int kRow32Waves = 6;
 template <unsigned OUT, bool UNIF, bool BATCH = false>
 struct Rec32 {
   static constexpr bool kLo = OUT & VPM_OUT_PSE;
-  static constexpr bool kMoment = UNIF && (OUT & VPM_OUT_VEL) && (OUT & VPM_OUT_STRETCH);
+  // Far chunks take the moment form, in FP32 in every row.  Without it rows
+  // that sum the stretching in FP64 per pair do so on every chunk: FP32 sums of
+  // g alpha_j leave 1e-7 of |alpha_i| |G|, and along a tube of parallel
+  // strengths nothing else is left.  FP64 everywhere costs a ring of 100,000
+  // with per-particle radii 8.6 ms instead of 7.3 (stretching; tiled kernels
+  // 10.9), a cloud, whose rows are not coherent, nothing.
+  static constexpr bool kMoment = UNIF && (OUT & VPM_OUT_STRETCH) && OUT != VPM_OUT_STRETCH;
   static constexpr bool kE3 = kMoment && kLo;
-  // Stretching: rows that sum in FP64 per pair do so on near chunks only, or
-  // on every chunk.  FP32 sums of g alpha_j leave 1e-7 of |alpha_i| |G|, and
-  // along a tube of parallel strengths nothing else is left.  FP64 everywhere
-  // costs a ring of 100,000 with per-particle radii 8.6 ms instead of 7.3
-  // (stretching; tiled kernels 10.9), a cloud, whose rows are not coherent,
-  // nothing.
-  static constexpr bool kFarFp32 = UNIF && OUT != VPM_OUT_STRETCH;
   static constexpr int kLoAt = kMoment ? 9 : UNIF ? 6 : 8;
   static constexpr int kStride = kLo ? 12 : kMoment ? 9 : UNIF ? 6 : 8;
   static constexpr int kGroup = kLo ? 2 : kMaxGroup32;
@@ -279,9 +277,10 @@ __device__ __forceinline__ void pair32(float* acc, double* g64, const Tgt32& t, 
   }
 }
 
-// The far-field moment form of velocity + stretching with a uniform radius
-// (pair_moment in vpm_fused.hip derives and measures it): 29 instructions per
-// pair, p = alpha_i x x_i (three times it with PSE).
+// The far-field moment form of the stretching with a uniform radius, with or
+// without the velocity (pair_moment in vpm_fused.hip derives and measures it):
+// 29 instructions per pair with it, p = alpha_i x x_i (three times it with
+// PSE).
 template <unsigned OUT>
 __device__ __forceinline__ void pair_far(float* acc, const Tgt32& t, const float* p, const float* f,
                                          const PairConst<float>& k) {
@@ -296,9 +295,11 @@ __device__ __forceinline__ void pair_far(float* acc, const Tgt32& t, const float
   acc[kG + 0] = __builtin_fmaf(g, f[3], acc[kG + 0]);
   acc[kG + 1] = __builtin_fmaf(g, f[4], acc[kG + 1]);
   acc[kG + 2] = __builtin_fmaf(g, f[5], acc[kG + 2]);
-  acc[kH + 0] = __builtin_fmaf(g, f[6], acc[kH + 0]);
-  acc[kH + 1] = __builtin_fmaf(g, f[7], acc[kH + 1]);
-  acc[kH + 2] = __builtin_fmaf(g, f[8], acc[kH + 2]);
+  if constexpr (S::vel) {
+    acc[kH + 0] = __builtin_fmaf(g, f[6], acc[kH + 0]);
+    acc[kH + 1] = __builtin_fmaf(g, f[7], acc[kH + 1]);
+    acc[kH + 2] = __builtin_fmaf(g, f[8], acc[kH + 2]);
+  }
   float e = f[3] * p[0];
   e = __builtin_fmaf(f[4], p[1], e);
   e = __builtin_fmaf(f[5], p[2], e);
@@ -426,7 +427,7 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
     }
     g64 = __builtin_amdgcn_readfirstlane(static_cast<int>(g64)) != 0;
   }
-  if constexpr (S::str && R::kFarFp32) {
+  if constexpr (R::kMoment) {
     const double p[3] = {X, Y, Z};
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
   int seen = 0;
   for (int c = split * kRowWaves + wave; c < nchunk; c += parts, ++seen) {
     bool is_near = true;
-    if constexpr (S::str && R::kFarFp32) {
+    if constexpr (R::kMoment) {
       // far tests for 64 of the wave's chunks at a time, one per lane
       if ((seen & 63) == 0) {
         const int64_t cc = c + static_cast<int64_t>(lane) * parts;
@@ -545,15 +546,16 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
       const float p[3] = {es * (t.ay * t.z - t.az * t.y), es * (t.az * t.x - t.ax * t.z),
                           es * (t.ax * t.y - t.ay * t.x)};
       stream([&](const float* f, int) { pair_far<OUT>(part, t, p, f, kc); });
-      // u += x_i x G + H of the chunk, in FP64
-      const double x = X - box[0], y = Y - box[1], z = Z - box[2];
-      const double gx = part[kG + 0], gy = part[kG + 1], gz = part[kG + 2];
-      constexpr double hs = R::kE3 ? 1.0 / 3.0 : 1.0;
-      double* u = &tot[wave][0][lane];
-      u[0] += (y * gz - z * gy) + static_cast<double>(part[kH + 0]) * hs;
-      u[kRow] += (z * gx - x * gz) + static_cast<double>(part[kH + 1]) * hs;
-      u[2 * kRow] += (x * gy - y * gx) + static_cast<double>(part[kH + 2]) * hs;
-      part[kH + 0] = part[kH + 1] = part[kH + 2] = 0.0f;
+      if constexpr (S::vel) {  // u += x_i x G + H of the chunk, in FP64
+        const double x = X - box[0], y = Y - box[1], z = Z - box[2];
+        const double gx = part[kG + 0], gy = part[kG + 1], gz = part[kG + 2];
+        constexpr double hs = R::kE3 ? 1.0 / 3.0 : 1.0;
+        double* u = &tot[wave][0][lane];
+        u[0] += (y * gz - z * gy) + static_cast<double>(part[kH + 0]) * hs;
+        u[kRow] += (z * gx - x * gz) + static_cast<double>(part[kH + 1]) * hs;
+        u[2 * kRow] += (x * gy - y * gx) + static_cast<double>(part[kH + 2]) * hs;
+        part[kH + 0] = part[kH + 1] = part[kH + 2] = 0.0f;
+      }
       if constexpr (S::pse) {
         part[kP + 0] = __builtin_fmaf(-t.ax, part[kT9], part[kP + 0]);
         part[kP + 1] = __builtin_fmaf(-t.ay, part[kT9], part[kP + 1]);
