@@ -154,7 +154,7 @@ struct AdjT32 {
 // Constants in VGPRs (literal operands halve an instruction's issue rate);
 // h75, h2625 carry the factor -2 sc of their term.
 struct AdjK {
-  float c15, c3, c75, c105, c945, h75, h2625;
+  float c15, c3, c75, c105, c945, h75, h2625, c45;
 };
 
 // FP32 sums of a chunk: G = g a_j, L = g lam_j, A, B, X, Y = f phi a_j,
@@ -186,7 +186,8 @@ __device__ __forceinline__ void adj_weights(AdjW& w_, const AdjT32& t, const flo
     s = t.hs + f[15];
     s2 = s * s;
   }
-  float t1 = __builtin_amdgcn_rsqf(dot3(d, d, s2));
+  const float D = dot3(d, d, s2);
+  float t1 = __builtin_amdgcn_rsqf(D);
   if constexpr (vs)
     if (self) t1 = 0.0f;  // all weights 0, also where a small radius' t7 is infinite
   const float t2 = t1 * t1, t3 = t2 * t1, t5 = t3 * t2;
@@ -198,7 +199,12 @@ __device__ __forceinline__ void adj_weights(AdjW& w_, const AdjT32& t, const flo
   if constexpr ((OUT & VPM_OUT_STRETCH) != 0)
     w_.h = (t5 * t2) * __builtin_fmaf(k.h2625, w, k.h75);
   if constexpr ((OUT & VPM_OUT_PSE) != 0) {
-    w_.p = UNIF ? (t5 * t2) * t2 : (s * t3) * (w * w * w);
+    if constexpr (UNIF) {
+      w_.p = (t5 * t2) * t2;
+    } else {  // as in vpm_row32.hip: 1 - D t2 takes t2's roundings out of its powers
+      const float r = fminf(__builtin_fmaf(-D, t2, 1.0f), 1.0f);
+      w_.p = ((s * t3) * (w * w * w)) * __builtin_fmaf(k.c45, r, 1.0f);
+    }
     w_.q = w_.p * t2;
   }
 }
@@ -342,9 +348,10 @@ __global__ __launch_bounds__(kRowBlock, kAdjWaves) void adj32_kernel(Adj32Args A
   __syncthreads();
 
   AdjK k{1.5f, 3.0f, 7.5f, 105.0f, 945.0f, static_cast<float>(-15.0 * scale),
-         static_cast<float>(-52.5 * scale)};
+         static_cast<float>(-52.5 * scale), 4.5f};
   asm volatile("" : "+v"(k.c15), "+v"(k.c3), "+v"(k.c75), "+v"(k.c105), "+v"(k.c945),
                "+v"(k.h75), "+v"(k.h2625));
+  if constexpr (pse && !UNIF) asm volatile("" : "+v"(k.c45));
   AdjAcc acc{};
   const int nchunk = (n + kAdjChunk - 1) / kAdjChunk;
   const int parts = splits * kRowWaves;

@@ -117,6 +117,7 @@ __device__ __forceinline__ double store_target(const FusedArgs& a, const Src8& t
 template <typename Real>
 struct PairConst {
   Real c15, c75, c22, c3, c25;
+  Real c45;  // the row pass with per-particle radii
 };
 
 // Constant-address-space view of the records: a load through it with a

@@ -27,9 +27,9 @@
 // Bound: FP32 issue (velocity alone 2.45e12 pairs/s, 1.55 wave64 instructions
 // per clock and CU; the moment form 1.8e12).  Tiled kernels -> here, per call.
 // N = 100,000: velocity 4.80 -> 4.17 ms, with per-particle radii 6.80 -> 4.78;
-// stretching of a ring 8.92 -> 8.32, 10.9 -> 8.60; PSE 5.81 -> 4.92, 6.96 ->
-// 5.78; vorticity + enstrophy 4.97 -> 4.73, 7.41 -> 5.98; all five with
-// per-particle radii 15.3 -> 13.5 (cloud), 18.3 -> 16.9 (ring).  Velocity +
+// stretching of a ring 8.92 -> 8.32, 10.9 -> 8.60; PSE 5.81 -> 4.92, 6.75 ->
+// 5.4; vorticity + enstrophy 4.97 -> 4.73, 7.15 -> 6.15; all five with
+// per-particle radii 15.7 -> 14.3 (cloud), 18.8 -> 17.6 (ring).  Velocity +
 // stretching: cloud of 2^20 614 -> 605, of 20,000 0.448 -> 0.328, ring of
 // 131,072 12.8 -> 11.1; with PSE: ring of 131,072 15.7 -> 13.1, leapfrogging
 // rings of 65,536 4.30 -> 3.49.
@@ -56,8 +56,8 @@ constexpr int kRow32Waves = 6;
 
 // Record layout: offset (3), strength (3); then with the moment form the
 // moment alpha x offset (3; three times it with PSE, pair_far), with
-// per-particle radii sigma/2 and sigma^2; with PSE the low parts
-// alpha - fp32(alpha).  Lengths in units of a uniform radius; with per-particle
+// per-particle radii sigma/2 and sigma^-2, with vorticity sigma^-3 behind them
+// (with PSE last); with PSE the low parts alpha - fp32(alpha).  Lengths in units of a uniform radius; with per-particle
 // radii as they are: any one particle's radius may be far from the others',
 // and the powers of t leave FP32 where distances are 1e8 units.
 // Two groups are in registers at once: of four records, or of two where a
@@ -81,7 +81,11 @@ struct Rec32 {
   static constexpr bool kMoment = UNIF && (OUT & VPM_OUT_STRETCH) && OUT != VPM_OUT_STRETCH;
   static constexpr bool kE3 = kMoment && kLo;
   static constexpr int kLoAt = kMoment ? 9 : UNIF ? 6 : 8;
-  static constexpr int kStride = kLo ? 12 : kMoment ? 9 : UNIF ? 6 : 8;
+  static constexpr int kIs3At = kLo ? 11 : 8;
+  static constexpr int kStride = kLo                                ? 12
+                                 : kMoment || (!UNIF && (OUT & VPM_OUT_VORT)) ? 9
+                                 : UNIF                                       ? 6
+                                                                              : 8;
   static constexpr int kGroup = kLo ? 2 : kMaxGroup32;
   static constexpr int kNear = kLo ? 4 : 2;  // sources in flight in the FP64 loop
   static constexpr int kChunk =
@@ -163,13 +167,15 @@ __device__ __forceinline__ void row32_records(const Src8* __restrict__ src, int 
     r[8] = ok ? static_cast<float>(ms * (g.ax * y - g.ay * x)) : 0.0f;
   } else if constexpr (!UNIF) {
     r[6] = ok ? static_cast<float>(0.5 * sig) : 0.5f;
-    r[7] = ok ? static_cast<float>(sig * sig) : 1.0f;
+    r[7] = ok ? static_cast<float>(1.0 / (sig * sig)) : 1.0f;
+    if constexpr (!R::kLo && R::kStride > 8) r[8] = ok ? static_cast<float>(1.0 / (sig * sig * sig)) : 1.0f;
   }
   if constexpr (R::kLo) {
     r[R::kLoAt] = static_cast<float>(g.ax - static_cast<double>(ax));
     r[R::kLoAt + 1] = static_cast<float>(g.ay - static_cast<double>(ay));
     r[R::kLoAt + 2] = static_cast<float>(g.az - static_cast<double>(az));
     for (int q = R::kLoAt + 3; q < R::kStride; ++q) r[q] = 0.0f;
+    if constexpr (!UNIF) r[R::kIs3At] = ok ? static_cast<float>(1.0 / (sig * sig * sig)) : 1.0f;
   }
 }
 
@@ -250,7 +256,17 @@ __device__ __forceinline__ void pair32(float* acc, double* g64, const Tgt32& t, 
   }
   if constexpr (S::pse) {
     const float* lo = f + Rec32<OUT, UNIF>::kLoAt;
-    const float v = UNIF ? (t3 * t3) * t3 : (s * t3) * (w * w * w);
+    float v;
+    if constexpr (UNIF) {
+      v = (t3 * t3) * t3;
+    } else {
+      // t2 carries the root's and its own rounding, the ninth power of t 4.5 of
+      // them (PSE of rings and clouds with per-particle radii, rel-L2 1.13
+      // times the tiled kernels' without this, 0.8 with)
+      // 1 - D t2, exact but for one rounding (of no weight at infinity)
+      const float r = fminf(__builtin_fmaf(-D, t2, 1.0f), 1.0f);
+      v = ((s * t3) * (w * w * w)) * __builtin_fmaf(k.c45, r, 1.0f);
+    }
     acc[kP + 0] += v * ((f[3] - t.ax) + (lo[0] - t.lx));
     acc[kP + 1] += v * ((f[4] - t.ay) + (lo[1] - t.ly));
     acc[kP + 2] += v * ((f[5] - t.az) + (lo[2] - t.lz));
@@ -260,9 +276,11 @@ __device__ __forceinline__ void pair32(float* acc, double* g64, const Tgt32& t, 
     if constexpr (UNIF) {
       v = t3 * (t2 * t2);
     } else {  // sigma_j, not sigma_ij (ParticlesPhysicsCuda.py:323,334-337)
-      const float q1 = __builtin_amdgcn_rsqf(r2 + f[7]);
-      const float q2 = q1 * q1, wj = f[7] * q2;
-      v = (q2 * q1) * (wj * wj);
+      // in units of sigma_j: near sources 1 + r^2 / sigma_j^2 carries less of
+      // the factors' rounding than r^2 + sigma_j^2 (rel-L2 1.04 times as large)
+      const float q1 = __builtin_amdgcn_rsqf(__builtin_fmaf(r2, f[7], 1.0f));
+      const float q2 = q1 * q1;
+      v = ((q2 * q2) * (q2 * q1)) * f[Rec32<OUT, UNIF>::kIs3At];
     }
     v = r2 > eps ? v : 0.0f;
     acc[kW + 0] += v * f[3];
@@ -443,8 +461,9 @@ __global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
   for (int q = 0; q < kNAcc; ++q) part[q] = 0.0f;
 #pragma unroll
   for (int q = 0; q < NS; ++q) tot[wave][q][lane] = 0.0;
-  PairConst<float> kc{1.5f, 7.5f, 2.2f, 3.0f, 2.5f};  // in VGPRs (see PairConst)
+  PairConst<float> kc{1.5f, 7.5f, 2.2f, 3.0f, 2.5f, 4.5f};  // in VGPRs (see PairConst)
   asm volatile("" : "+v"(kc.c15), "+v"(kc.c75), "+v"(kc.c22), "+v"(kc.c3), "+v"(kc.c25));
+  if constexpr (!UNIF) asm volatile("" : "+v"(kc.c45));
 
   const int nchunk = (n + CH - 1) / CH;
   const int parts = splits * kRowWaves;
