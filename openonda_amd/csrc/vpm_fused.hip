@@ -1,6 +1,7 @@
 // Tiled all-pairs forward pass: the batched launch, the tile shapes a caller
-// asks for by index, and sets without the far form that are too large for
-// vpm_forward_noalloc's array with the row pass's records.  (Other single-set calls run vpm_row32.hip or
+// asks for by index, the stretching alone of many particles (vpm_row32.h), and
+// sets without the far form that are too large for vpm_forward_noalloc's array
+// with the row pass's records.  (Other single-set calls run vpm_row32.hip or
 // vpm_forward_rows.hip.)
 //
 // One pass over all (target, source) pairs computes any subset of the GPU
@@ -1368,8 +1369,8 @@ bool wants_far_records(const vpm_forward_opts_t* o) {
   return (m & VPM_OUT_VEL) && (m & VPM_OUT_STRETCH);
 }
 
-bool row32_asked(const vpm_forward_opts_t* o) {
-  return o && row32_wanted(o);
+bool row32_asked(int64_t n, const vpm_forward_opts_t* o) {
+  return o && row32_wanted(n, o);
 }
 
 // FP64 partial slots per target of a source split (see Slots::nslot)
@@ -1383,7 +1384,7 @@ int split_slots(unsigned mask) {
 size_t split_capacity(int64_t n, const vpm_forward_opts_t* o) {
   if (!o || n <= 0) return 0;
   if (forward_rows_wanted(n, o)) return forward_rows_split_bytes(n, row_mask(o->outputs));
-  if (row32_asked(o)) return row32_split_bytes(n, row_mask(o->outputs));
+  if (row32_asked(n, o)) return row32_split_bytes(n, row_mask(o->outputs));
   const int c = effective_config(kernel_mask(o->outputs), o->sigma_mode == VPM_SIGMA_UNIFORM,
                                  o->tile_config < kNumCfgs ? o->tile_config : -1);
   const int br = kCfgs[c].block * kCfgs[c].r, tile = kCfgs[c].tile;
@@ -1422,7 +1423,7 @@ int layout(int64_t n, const vpm_forward_opts_t* o, WsLayout* L, bool need_cub = 
   // Records and boxes of the kernels that run: the row pass's (8 numbers per
   // box), else the tiled kernels' far records (6), + one group of records read
   // ahead past the last chunk.
-  const bool far = wants_far_records(o), rows = row32_asked(o);
+  const bool far = wants_far_records(o), rows = row32_asked(n, o);
   const int64_t nn = n > 0 ? n : 1;
   L->far_rec = take(rows  ? row32_record_bytes(n)
                     : far ? (static_cast<size_t>(ceil_div(nn, kMaxFarChunk)) * kMaxFarChunk +
@@ -1981,7 +1982,7 @@ int forward_run_impl(const vpm_particles_t* p, const vpm_forward_opts_t* o,
     }
     return VPM_OK;
   }
-  const unsigned mask = forward_rows_wanted(n, o) || row32_asked(o) ? row_mask(want)
+  const unsigned mask = forward_rows_wanted(n, o) || row32_asked(n, o) ? row_mask(want)
                                                                      : kernel_mask(want);
   if (forward_rows_wanted(n, o)) {
     // These rows read the particles while others are stored: outputs in the
@@ -2029,7 +2030,7 @@ int forward_run_impl(const vpm_particles_t* p, const vpm_forward_opts_t* o,
   int nblocks = 0;
   const bool unif = o->sigma_mode == VPM_SIGMA_UNIFORM;
   const int cfg = effective_config(mask, unif, o->tile_config);
-  int rc = row32_asked(o)
+  int rc = row32_asked(n, o)
                ? row32_run(a, mask, unif, reinterpret_cast<float*>(ws + L.far_rec),
                            reinterpret_cast<double*>(ws + L.far_box), st, &nblocks)
                : dispatch(a, mask, unif, cfg, st, &nblocks);
@@ -2117,7 +2118,7 @@ int vpm_forward_noalloc(const vpm_particles_t* p, const vpm_forward_opts_t* o,
   // which need none unless their far form applies (wants_far_records: then
   // theirs are as large, and this changes nothing)
   vpm_forward_opts_t tiled = *o;
-  if (L.total > kScratchBytes && row32_asked(o)) {
+  if (L.total > kScratchBytes && row32_asked(p->n, o)) {
     tiled.tile_config = default_config(kernel_mask(o->outputs),
                                        o->sigma_mode == VPM_SIGMA_UNIFORM);
     o = &tiled;

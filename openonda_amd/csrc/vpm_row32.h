@@ -5,11 +5,21 @@
 
 namespace vpm {
 
-// The row pass runs every FP32-compensated call that asks for no tile shape
-// (vpm_row32.hip has both sides measured: it was faster on every output set,
-// radius mode and size from 8,192 to 2^20).
-inline bool row32_wanted(const vpm_forward_opts_t* o) {
-  return o->precision == VPM_PREC_F32C && o->tile_config < 0;
+// The row pass runs every FP32-compensated call that asks for no tile shape,
+// but the stretching alone of many particles with a uniform radius
+// (vpm_row32.hip has both sides measured: it was faster on every other output
+// set, radius mode and size from 8,192 to 2^20).  That set has no moment form
+// that pays on rings, and sums in FP64 there on every chunk: each row reads
+// all particles again, where the tiled kernels read them once for 512 targets.
+// Tiled / rows, ms: ring of 131,072 15.4 / 14.4, 163,840 21.5 / 23.1, 400,009
+// 135 / 160; cloud of 131,072 11.2 / 11.0, 163,840 16.3 / 17.3, 400,009 101 /
+// 104.
+constexpr int64_t kRow32StretchMax = 131072;
+
+inline bool row32_wanted(int64_t n, const vpm_forward_opts_t* o) {
+  if (o->precision != VPM_PREC_F32C || o->tile_config >= 0) return false;
+  return n <= kRow32StretchMax || o->outputs != VPM_OUT_STRETCH ||
+         o->sigma_mode != VPM_SIGMA_UNIFORM;
 }
 
 // Bytes of the FP32 records, the chunk boxes and the split partials.

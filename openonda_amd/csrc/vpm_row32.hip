@@ -51,8 +51,11 @@ constexpr int kBox32 = 8;         // doubles per chunk box: centre, half-extent,
 constexpr double kFarGap32 = 4.0;
 // Waves per SIMD the registers must allow: 73 VGPRs for velocity + stretching
 // (cloud of 2^20: 605 ms; 641 at five waves, 687 at eight, where the records
-// spill scalar registers).
-constexpr int kRow32Waves = 6;
+// spill scalar registers); eight for the stretching alone, whose records and
+// sums are the smallest (cloud of 65,536 with a uniform radius 2.95 -> 2.81 ms,
+// ring 3.94 -> 3.81).
+template <unsigned OUT>
+constexpr int kRow32Waves = OUT == VPM_OUT_STRETCH ? 8 : 6;
 
 // Record layout: offset (3), strength (3); then with the moment form the
 // moment alpha x offset (3; three times it with PSE, pair_far), with
@@ -378,7 +381,7 @@ __device__ __forceinline__ bool row32_item(const Row32Batch& b, int w, Row32Item
 // with the set picked at its top: as a device function called from two kernels
 // the same body took up to 46 more VGPRs, into scratch.)
 template <unsigned OUT, bool UNIF, bool BATCH>
-__global__ __launch_bounds__(kRowBlock, kRow32Waves) void row32_kernel(
+__global__ __launch_bounds__(kRowBlock, kRow32Waves<OUT>) void row32_kernel(
     FusedArgs a, Row32Batch b, int splits, const float* __restrict__ rec_,
     const double* __restrict__ box_) {
   const int split = static_cast<int>(blockIdx.y);
