@@ -1,6 +1,6 @@
 // Tiled all-pairs forward pass: the batched launch, the tile shapes a caller
-// asks for by index, the stretching alone of many particles (vpm_row32.h), and
-// sets without the far form that are too large for vpm_forward_noalloc's array
+// asks for by index, two output sets of many particles (vpm_row32.h), and sets
+// without the far form that are too large for vpm_forward_noalloc's array
 // with the row pass's records.  (Other single-set calls run vpm_row32.hip or
 // vpm_forward_rows.hip.)
 //
@@ -1384,7 +1384,8 @@ int split_slots(unsigned mask) {
 size_t split_capacity(int64_t n, const vpm_forward_opts_t* o) {
   if (!o || n <= 0) return 0;
   if (forward_rows_wanted(n, o)) return forward_rows_split_bytes(n, row_mask(o->outputs));
-  if (row32_asked(n, o)) return row32_split_bytes(n, row_mask(o->outputs));
+  if (row32_asked(n, o))
+    return row32_split_bytes(n, row_mask(o->outputs), o->sigma_mode == VPM_SIGMA_UNIFORM);
   const int c = effective_config(kernel_mask(o->outputs), o->sigma_mode == VPM_SIGMA_UNIFORM,
                                  o->tile_config < kNumCfgs ? o->tile_config : -1);
   const int br = kCfgs[c].block * kCfgs[c].r, tile = kCfgs[c].tile;

@@ -5,27 +5,28 @@
 
 namespace vpm {
 
-// The row pass runs every FP32-compensated call that asks for no tile shape,
-// but the stretching alone of many particles with a uniform radius
-// (vpm_row32.hip has both sides measured: it was faster on every other output
-// set, radius mode and size from 8,192 to 2^20).  That set has no moment form
-// that pays on rings, and sums in FP64 there on every chunk: each row reads
-// all particles again, where the tiled kernels read them once for 512 targets.
-// Tiled / rows, ms: ring of 131,072 15.4 / 14.4, 163,840 21.5 / 23.1, 400,009
-// 135 / 160; cloud of 131,072 11.2 / 11.0, 163,840 16.3 / 17.3, 400,009 101 /
-// 104.
-constexpr int64_t kRow32StretchMax = 131072;
+// The row pass runs every FP32-compensated call that asks for no tile shape
+// (vpm_row32.hip has both sides measured), but two output sets that sum in FP64
+// on every chunk, where many particles no longer fit the L2: each row reads
+// them all again, where the tiled kernels read them once for 256 or 512
+// targets.  The stretching alone with a uniform radius, tiled / rows, ms: ring
+// of 131,072 15.4 / 14.4, 163,840 21.5 / 23.1, 400,009 135 / 160; cloud of
+// 131,072 11.2 / 11.0, 163,840 16.3 / 17.3.  PSE with vorticity or enstrophy and
+// per-particle radii: ring of 262,144 121 / 117, 400,009 286 / 298.
+constexpr int64_t kRow32StretchMax = 131072, kRow32AllMax = 262144;
 
 inline bool row32_wanted(int64_t n, const vpm_forward_opts_t* o) {
   if (o->precision != VPM_PREC_F32C || o->tile_config >= 0) return false;
-  return n <= kRow32StretchMax || o->outputs != VPM_OUT_STRETCH ||
-         o->sigma_mode != VPM_SIGMA_UNIFORM;
+  if (o->sigma_mode == VPM_SIGMA_UNIFORM)
+    return n <= kRow32StretchMax || o->outputs != VPM_OUT_STRETCH;
+  return n <= kRow32AllMax || !(o->outputs & VPM_OUT_PSE) ||
+         !(o->outputs & (VPM_OUT_VORT | VPM_OUT_ENSTROPHY));
 }
 
 // Bytes of the FP32 records, the chunk boxes and the split partials.
 size_t row32_record_bytes(int64_t n);
 size_t row32_box_bytes(int64_t n);
-size_t row32_split_bytes(int64_t n, unsigned mask);
+size_t row32_split_bytes(int64_t n, unsigned mask, bool unif);
 
 // Builds the records from the sorted particles a.src and runs the pass;
 // *nblocks: enstrophy partials written to a.ens_part.

@@ -710,13 +710,33 @@ int nslots(unsigned mask) {
   return c + ((mask & VPM_OUT_STRETCH) ? 3 : 0);
 }
 
+// Source splits.  Rows that sum in FP64 on every chunk read 88 bytes per
+// source, the FP64 strengths among them, and the workgroups in flight drift
+// apart: more than 16,384 sources do not stay in an XCD's L2, and the rows of a
+// ring then wait for it.  Such sets are split that far while the partials
+// stay below 512 MB.  Ring with per-particle radii, all five outputs: 98,304
+// particles 21.2 -> 17.3 ms, 131,072 34.7 -> 30.1 (tiled 19.5 and 32.1), 262,144
+// 146 -> 117 (121); velocity + stretching 11.6 -> 9.5, 17.8 -> 16.6, 71.9 -> 64.8;
+// clouds within 5% either way.
+constexpr int64_t kL2Sources = 16384;
+constexpr size_t kMaxPartials = size_t(512) << 20;
+
+int row32_splits(int64_t n, unsigned mask, bool unif) {
+  const int64_t rows = row_count(n);
+  const int k = row_splits(rows, n);
+  if (!(mask & VPM_OUT_STRETCH) || (unif && mask != VPM_OUT_STRETCH)) return k;
+  const size_t per = static_cast<size_t>(nslots(mask)) * rows * kRow * sizeof(double);
+  const int64_t fit = std::min<int64_t>(ceil_div(n, kL2Sources), kMaxPartials / per);
+  return std::max(k, static_cast<int>(fit));
+}
+
 template <unsigned OUT, bool UNIF>
 int launch(FusedArgs a, float* rec, double* box, hipStream_t st, int* nblocks) {
   using R = Rec32<OUT, UNIF>;
   const int rows = static_cast<int>(ceil_div(a.n, kRow));
   const int chunks = static_cast<int>(ceil_div(a.n, R::kChunk));
   const size_t per = static_cast<size_t>(Slots<OUT>::nslot) * rows * kRow * sizeof(double);
-  int k = std::min(row_splits(rows, a.n), std::max(1, chunks / kRowWaves));
+  int k = std::min(row32_splits(a.n, OUT, UNIF), std::max(1, chunks / kRowWaves));
   if (a.max_splits > 0) k = std::min(k, a.max_splits);
   if (!a.part || a.part_cap / per < 2) k = 1;
   else k = static_cast<int>(std::min<size_t>(k, a.part_cap / per));
@@ -776,9 +796,9 @@ size_t row32_box_bytes(int64_t n) {
   return static_cast<size_t>(ceil_div(n > 0 ? n : 1, kMinChunk32)) * kBox32 * sizeof(double);
 }
 
-size_t row32_split_bytes(int64_t n, unsigned mask) {
+size_t row32_split_bytes(int64_t n, unsigned mask, bool unif) {
   const int64_t rows = row_count(n);
-  const int k = row_splits(rows, n);
+  const int k = row32_splits(n, mask, unif);
   return k > 1 ? static_cast<size_t>(k) * nslots(mask) * rows * kRow * sizeof(double) : 0;
 }
 

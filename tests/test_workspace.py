@@ -2,8 +2,8 @@
 call writes.
 
 Host part: the row pass writes the same records and chunk boxes for a uniform
-radius as for per-particle radii, so both need the same workspace; the
-adjoint's query serves both precisions.  GPU part: every output set, the
+radius as for per-particle radii, so both need the same workspace but for
+whole source splits; the adjoint's query serves both precisions.  GPU part: every output set, the
 adjoint, a batch and the library's autotuner in a workspace of exactly the
 queried size, with guard bytes behind it.
 """
@@ -24,11 +24,16 @@ def forward_bytes(n, mask, mode, presorted, tile=-1, precision=L.PREC_F32C):
 
 @pytest.mark.parametrize("presorted", [0, 1])
 @pytest.mark.parametrize("mask", MASKS)
-def test_row_pass_workspace_does_not_depend_on_the_radius_mode(mask, presorted):
+def test_row_pass_workspace_differs_between_radius_modes_by_splits_only(mask, presorted):
     # sorted sets above 65,536 ask the device for the radix sort's scratch
-    for n in (8192, 8193, 9000, 20011, 34914, 65536) + ((300001, 1 << 20) if presorted else ()):
+    slots = 3 * bin(mask).count("1") + (3 if mask & L.OUT_STRETCH else 0)
+    for n in (8192, 8193, 9000, 16384, 20011, 34914, 65536) + ((100001, 131072) if presorted else ()):
         uniform = forward_bytes(n, mask, L.SIGMA_UNIFORM, presorted)
-        assert uniform == forward_bytes(n, mask, L.SIGMA_GENERAL, presorted) > 0, (n, mask)
+        general = forward_bytes(n, mask, L.SIGMA_GENERAL, presorted)
+        assert uniform > 0
+        if n <= 16384 or not mask & L.OUT_STRETCH:
+            assert uniform == general, (n, mask)
+        assert (general - uniform) % (slots * -(-n // 64) * 64 * 8) == 0, (n, mask)
 
 
 def test_largest_allocation_free_set():
@@ -66,7 +71,7 @@ def test_forward_stays_inside_its_workspace(gpu, mask, general):
     from openonda_amd import physics as P
 
     rng = np.random.default_rng(mask)
-    for n in (1, 700, 8191, 8192, 9000, 20011, 66001):
+    for n in (1, 700, 8191, 8192, 9000, 20011, 66001, 132000):
         x, a, s, _ = FM.random_cloud(n, seed=n)
         if general:
             s = s * rng.uniform(0.8, 1.25, n)
