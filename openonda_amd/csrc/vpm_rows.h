@@ -300,7 +300,12 @@ __global__ __launch_bounds__(kRowBlock, 4) void row_wide_kernel(RowArgs a, int r
 // eight waves that share a row's sources, is not tuned for this kernel: these
 // sizes have rows enough for one or two splits.
 constexpr int64_t kWideStride = int64_t{1} << 19, kWideMin = int64_t{1} << 18;
+// The same for up to eight sources at very many points, where eight waves per
+// row would have one source each (a million points: velocity of one source 29 ->
+// 13 us, of eight about 35 -> 17).
+constexpr int64_t kWideSources = 8, kWideRows = 6144;
 inline bool row_wide_wanted(const RowArgs& a, int64_t rows) {
+  if (a.n <= kWideSources && rows >= kWideRows) return true;
   return a.ld % kWideStride == 0 && a.n >= kWideMin && rows >= kWideMin / kRow;
 }
 
