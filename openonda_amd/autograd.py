@@ -122,7 +122,8 @@ class ProbeVelocity(torch.autograd.Function):
         n = pp.n
         dpos = torch.empty((3, n), dtype=torch.float64, device=pos.device)
         dstr = torch.empty((3, n), dtype=torch.float64, device=pos.device)
-        nb = L.load().vpm_induced_velocity_at_adjoint_workspace_bytes(tp.m, n)
+        nb = (L.load().vpm_induced_velocity_at_adjoint_workspace_bytes(tp.m, n)
+              if tp.m >= P.SPLIT_MIN else 0)
         ws = torch.empty(nb, dtype=torch.uint8, device=pos.device) if nb else None
         L.call("vpm_induced_velocity_at_adjoint_ws", C.byref(tp), C.byref(pp), gu.data_ptr(),
                P._ld(gu), dpos.data_ptr(), dstr.data_ptr(), max(n, 1),

@@ -119,9 +119,13 @@ def _variant(v):
 
 
 # ------------------------------------------------------------ plain drop-in
+SPLIT_MIN = 256  # sources: two splits of eight waves, sixteen sources each
+
+
 def _pair_sum(what, targets, p, pos, m, variant, out):
     o = _out_vec(out, pos, m)
-    nb = L.load().vpm_pair_sum_workspace_bytes(m, p.n)
+    # fewer sources than SPLIT_MIN are never split: no query (1 us of a call of 11)
+    nb = L.load().vpm_pair_sum_workspace_bytes(m, p.n) if p.n >= SPLIT_MIN else 0
     # a buffer per call, not the shared workspace: it belongs to the current
     # stream, and to the graph that captures the call
     ws = torch.empty(nb, dtype=torch.uint8, device=pos.device) if nb else None

@@ -58,6 +58,17 @@ def test_adjoint_workspace_serves_every_precision(n):
     assert len(set(sizes)) == 1 and sizes[0] > 0
 
 
+def test_sets_below_the_split_size_need_no_workspace():
+    from openonda_amd import physics as P
+
+    lib = L.load()
+    for m in (1, 64, 1000, 1 << 20):
+        for n in (0, 1, 255, P.SPLIT_MIN - 1):
+            assert lib.vpm_pair_sum_workspace_bytes(m, n) == 0
+            assert lib.vpm_induced_velocity_at_adjoint_workspace_bytes(n, m) == 0
+    assert lib.vpm_pair_sum_workspace_bytes(64, P.SPLIT_MIN) > 0
+
+
 GUARD = 1 << 16
 
 
