@@ -243,7 +243,7 @@ int vpm_tile_config_info(int index, int* block, int* targets_per_lane, int* tile
  * ms is not NULL, each configuration's mean time in ms[0..count).  The row
  * pass (tile_config = -1) has no shape and is not among them.  The workspace
  * must hold vpm_autotune_workspace_bytes (the largest layout).
- * Synchronises the stream.  (openonda_amd/autotune.py adds an
+ * Synchronises the stream.  (openonda_amd/autotune.py adds the row pass, an
  * accuracy check against the FP64 pass and a cache keyed by N.) */
 size_t vpm_autotune_workspace_bytes(int64_t n, const vpm_forward_opts_t* opts);
 int vpm_autotune(const vpm_particles_t* p, const vpm_forward_opts_t* opts, vpm_forward_out_t* out,

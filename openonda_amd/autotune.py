@@ -2,14 +2,15 @@
 
 The library instantiates the fused kernel for a set of tile shapes
 (``vpm_tile_config_info``: workgroup size, targets per lane, source tile,
-sub-tile length, compensation mode).  :func:`tune` times each candidate on
-the device with HIP events, measures its rel-L2 against the FP64 fused pass on
-the same input, and keeps the fastest one within the accuracy bound.  Results
-are cached in a JSON file keyed by (kernel, precision, output set, radius
-mode, N rounded to a power of two); :func:`best_config` reads the cache and
-``physics.forward(..., tile_config="auto")`` uses it.
+sub-tile length, compensation mode); tile configuration -1 is the default
+pass, which has no shape (the row pass).  :func:`tune` times it and each shape
+on the device with HIP events, measures their rel-L2 against the FP64 fused
+pass on the same input, and keeps the fastest one within the accuracy bound.
+Results are cached in a JSON file keyed by (kernel, precision, output set,
+radius mode, N rounded to a power of two); :func:`best_config` reads the cache
+and ``physics.forward(..., tile_config="auto")`` uses it.
 
-:func:`tune_batch` does the same for the batched persistent launch over
+:func:`tune_batch` does the same for the batched launches, the row pass and
 (tile shape x persistent grid size), keyed by output mask and total pair
 count; ``BatchedSystem(tile_config="auto")`` uses its choice.
 """
@@ -32,9 +33,13 @@ CACHE = Path(os.environ.get("VPM_AUTOTUNE_CACHE",
 _lock = threading.Lock()
 
 
+# What the candidates are; winners of other candidates do not apply.
+CANDIDATES = "rows+tiles"
+
+
 def _key(kernel, precision, outputs, sigma_mode, n):
     bucket = 0 if n <= 1 else int(round(math.log2(n)))
-    return f"{kernel}|{precision}|{'+'.join(sorted(outputs))}|{sigma_mode}|2^{bucket}"
+    return f"{CANDIDATES}|{kernel}|{precision}|{'+'.join(sorted(outputs))}|{sigma_mode}|2^{bucket}"
 
 
 def load_cache(path=None):
@@ -76,15 +81,17 @@ def _time(fn, reps):
 
 def tune(pos, alpha, sigma, nu=None, outputs=("vel", "stretch"), sigma_mode="uniform",
          max_rel=1e-6, reps=2, path=None, save=True):
-    """Times every tile configuration on this input; returns (best, report)
-    and (optionally) records the winner in the cache.  When no configuration
-    meets ``max_rel``, returns (None, report), caches nothing and warns."""
+    """Times the default pass (configuration -1, shape None) and every tile
+    configuration on this input; returns (best, report) -- the report lists
+    the tile configurations -- and (optionally) records the winner in the
+    cache.  When no candidate meets ``max_rel``, returns (None, report), caches
+    nothing and warns."""
     P.require_gpu()
     n = pos.shape[1]
     ref = P.forward(pos, alpha, sigma, nu, outputs=outputs, precision="f64",
                     sigma_mode=sigma_mode)
     report = []
-    for cfg, shape in enumerate(P.tile_configs()):
+    for cfg, shape in [(-1, None), *enumerate(P.tile_configs())]:
         res = {}
 
         def run():
@@ -101,11 +108,12 @@ def tune(pos, alpha, sigma, nu=None, outputs=("vel", "stretch"), sigma_mode="uni
             rel = max(rel, d)
         report.append({"config": cfg, "shape": shape, "ms": ms, "rel_l2": rel})
     ok = [r for r in report if r["rel_l2"] <= max_rel]
+    candidates, report = report, report[1:]
     if not ok:
-        # no shape meets the accuracy bound on this input: keep the library's
-        # default shape (nothing is cached, so tile_config="auto" falls back to it)
+        # no candidate meets the accuracy bound on this input: keep the library's
+        # default pass (nothing is cached, so tile_config="auto" falls back to it)
         warnings.warn(f"autotune: no tile configuration reached rel-L2 <= {max_rel:g} "
-                      f"(best {min(r['rel_l2'] for r in report):.2e}); nothing cached",
+                      f"(best {min(r['rel_l2'] for r in candidates):.2e}); nothing cached",
                       RuntimeWarning, stacklevel=2)
         return None, report
     best = min(ok, key=lambda r: r["ms"])
@@ -113,8 +121,8 @@ def tune(pos, alpha, sigma, nu=None, outputs=("vel", "stretch"), sigma_mode="uni
         with _lock:
             c = load_cache(path)
             c[_key("fused", "f32c", outputs, sigma_mode, n)] = {
-                "config": best["config"], "shape": list(best["shape"]), "ms": best["ms"],
-                "rel_l2": best["rel_l2"], "n": n, "candidates": report}
+                "config": best["config"], "shape": list(best["shape"] or ()), "ms": best["ms"],
+                "rel_l2": best["rel_l2"], "n": n, "candidates": candidates}
             save_cache(c, path)
     return best, report
 
@@ -122,7 +130,8 @@ def tune(pos, alpha, sigma, nu=None, outputs=("vel", "stretch"), sigma_mode="uni
 def device_tune(pos, alpha, sigma, nu=None, outputs=("vel", "stretch"), sigma_mode="uniform",
                 reps=2):
     """Timing-only tuning inside the library (``vpm_autotune``): one sort, every
-    tile configuration timed with HIP events.  Returns (best index, ms list)."""
+    tile configuration timed with HIP events (not the row pass, which has no
+    index).  Returns (best index, ms list)."""
     import ctypes as C
 
     from . import _lib as L
@@ -164,13 +173,13 @@ TUNE_BATCH_MAX_PARTICLES = 1 << 18
 def _batch_key(sizes, mask, precision="f32c"):
     pairs = float(np.sum(np.asarray(sizes, dtype=np.float64) ** 2))
     bucket = int(round(math.log2(pairs))) if pairs > 1 else 0
-    return f"batch|{precision}|mask{int(mask)}|pairs2^{bucket}|sets{len(sizes)}"
+    return f"{CANDIDATES}|batch|{precision}|mask{int(mask)}|pairs2^{bucket}|sets{len(sizes)}"
 
 
 def best_batch_config(sizes, mask, precision="f32c", path=None):
     """Cached (tile_config, grid) of the batched launch for sets of these
     sizes and this output mask (total pair count rounded to a power of two),
-    or None."""
+    or None; (-1, 0) is the row pass."""
     with _lock:
         c = load_cache(path)
     e = c.get(_batch_key(sizes, mask, precision))
@@ -179,8 +188,9 @@ def best_batch_config(sizes, mask, precision="f32c", path=None):
 
 def tune_batch(sets, pse=True, les=True, configs=None, grids=None, reps=2, max_rel=1e-6,
                path=None, save=True, log=None):
-    """Times the batched persistent launch (one stage-1 evaluation: velocity,
-    stretching and, as requested, PSE and the LES outputs, over every set) for
+    """Times the batched launch (one stage-1 evaluation: velocity, stretching
+    and, as requested, PSE and the LES outputs, over every set) as the row
+    pass (configuration -1, in ``configs`` unless others are given) and for
     each tile configuration x persistent grid size on these sets, checks every
     set's outputs against the FP64 batched pass (rel-L2 <= ``max_rel`` per
     set and output), and caches the fastest accurate (config, grid) under the
@@ -209,13 +219,14 @@ def tune_batch(sets, pse=True, les=True, configs=None, grids=None, reps=2, max_r
     del ref
     bs = B.BatchedSystem(sets, dt=0.0, precision="f32c", pse=pse, les=les)
     cus = torch.cuda.get_device_properties(bs.device).multi_processor_count
-    configs = list(range(len(P.tile_configs()))) if configs is None else list(configs)
+    configs = [-1, *range(len(P.tile_configs()))] if configs is None else list(configs)
     grids = [0, cus, 2 * cus, 3 * cus] if grids is None else list(grids)
     sl = [bs.set_slice(k) for k in range(bs.nsets)]
     report = []
+    default = int(L.load().vpm_batch_tile_config_default(mask))
     for cfg in configs:
-        for grid in grids:
-            bs.set_launch(cfg, grid)
+        for grid in grids if cfg >= 0 else [0]:
+            bs.set_launch(default if cfg < 0 else cfg, grid, rows=cfg < 0)
             run = lambda: bs.evaluate(bs.x, bs.a, mask, False, s)
             bs.evaluate(bs.x, bs.a, mask, True, s)  # sorts (first time) and warms
             bs.synchronize()
@@ -282,7 +293,7 @@ def main(argv=None):
     best, report = tune(P.to_soa(x, dev), P.to_soa(al, dev), torch.from_numpy(s).to(dev),
                         torch.from_numpy(np.full(a.n, 1e-3)).to(dev) if "pse" in outs else None,
                         outputs=outs, reps=a.reps, path=a.cache)
-    for r in report:
+    for r in report:  # the tile configurations
         print(f"config {r['config']} {tuple(r['shape'])}: {r['ms']:.2f} ms rel-L2 {r['rel_l2']:.2e}",
               flush=True)
     if best is None:

@@ -96,7 +96,8 @@ class BatchedSystem:
 
             self.autotuned = autotune.best_batch_config(sizes, self.stage_mask, path=autotune_cache)
             tile_config, grid = self.autotuned if self.autotuned else (-1, grid)
-        rows = tile_config < 0 and grid == 0 and precision == "f32c" and row_pass_pays(sizes)
+        rows = (tile_config < 0 and grid == 0 and precision == "f32c"
+                and (self.autotuned is not None or row_pass_pays(sizes)))
         self.tile_config = (int(tile_config) if tile_config >= 0
                             else int(L.load().vpm_batch_tile_config_default(self.stage_mask)))
         for k, s in enumerate(sets):
