@@ -409,19 +409,20 @@ def main(argv=None):
         log(f"[bench] ring forward pass alone: {ring_ms:.2f} ms, {rach:.1f} TFLOP/s "
             f"({rach / FP32_VECTOR_PEAK_TFLOPS:.3f} of peak)")
 
-    # ---- batched persistent launch, graph-replayed RK4 steps -----------------
+    # ---- batched launch, graph-replayed RK4 steps ----------------------------
     if not args.skip_batch:
         from openonda_amd import batch as B
 
         sets = FM.batch_instances()
         # the launch the batch autotuner cached for this workload, else the
-        # library's default shape (the sweep itself is limited to smaller
-        # batches: autotune.TUNE_BATCH_MAX_PARTICLES)
+        # default (the sweep itself is limited to smaller batches:
+        # autotune.TUNE_BATCH_MAX_PARTICLES)
         bs = B.BatchedSystem(sets, dt=0.005, precision="f32c", pse=True, les=True,
                              tile_config="auto")
+        launch = ("rows of 64 targets" if bs.rows
+                  else f"persistent, tile config {bs.tile_config}, grid {bs.grid}")
         log(f"[bench] batch: {bs.nsets} sets, N_total={bs.n}, {bs.n_items} work items, "
-            f"tile config {bs.tile_config}, grid {bs.grid} "
-            f"({'autotuned' if bs.autotuned else 'default'})")
+            f"{launch} ({'autotuned' if bs.autotuned else 'default'})")
         bs.step()          # sorts, eager
         bs.capture()
         bs.replay(1)       # warm
@@ -451,8 +452,9 @@ def main(argv=None):
         result["batch"] = {
             "workload": f"{bs.nsets} ring/cloud sets, N_i log-uniform in [2048, 131072], "
                         f"N_total={bs.n}; RK4 (velocity+stretching+PSE, LES filter per set), "
-                        f"one persistent launch per stage, HIP-graph replay",
-            "tile_config": bs.tile_config, "grid": bs.grid,
+                        f"every set in one pass per stage, HIP-graph replay",
+            "pass": launch, "tile_config": None if bs.rows else bs.tile_config,
+            "grid": None if bs.rows else bs.grid,
             "launch": "autotuned" if bs.autotuned else "default",
             "steps": args.batch_steps, "ms_per_step": bms / args.batch_steps,
             "pairs_per_s": pairs_step * args.batch_steps / (bms * 1e-3),

@@ -146,7 +146,9 @@ int vpm_get_total_enstrophy(const vpm_particles_t* p, int variant, double* resul
  * precision F32C: FP32 pair arithmetic on centred offsets of Morton-sorted
  * particles, FP32 partials of at most 128 sources folded into FP64 totals;
  * sets below 8,192 particles run the FP64 pass.
- * precision F64: the same sums in FP64 throughout, in the caller's order. */
+ * precision F64: the same sums in FP64 throughout, in the caller's order.
+ * A particle at infinity leaves the PSE and VORT sums (weight 0); the other
+ * outputs are inf/inf there in the reference and not defined here. */
 #define VPM_OUT_VEL 1u
 #define VPM_OUT_STRETCH 2u
 #define VPM_OUT_PSE 4u
@@ -164,9 +166,10 @@ typedef struct vpm_forward_opts {
   int32_t precision;    /* VPM_PREC_* */
   int32_t sigma_mode;   /* VPM_SIGMA_* */
   int32_t presorted;    /* 1: particles already spatially coherent, skip the Morton sort */
-  int32_t tile_config;  /* -1: the row pass (rows of 64 targets, no tiles); else an
-                         * index < vpm_tile_config_count(): the tiled F32C kernels
-                         * in that shape */
+  int32_t tile_config;  /* -1: the default pass (rows of 64 targets, no tiles; two
+                         * output sets of very many particles run the tiled F32C
+                         * kernels); else an index < vpm_tile_config_count(): the
+                         * tiled kernels in that shape */
   int32_t max_splits;   /* 0: automatic; k >= 1: at most k source splits.  When the
                          * target blocks alone cannot fill the device, the sources
                          * are split among workgroups and the FP64 partial sums
@@ -249,12 +252,13 @@ size_t vpm_autotune_workspace_bytes(int64_t n, const vpm_forward_opts_t* opts);
 int vpm_autotune(const vpm_particles_t* p, const vpm_forward_opts_t* opts, vpm_forward_out_t* out,
                  void* workspace, size_t ws_bytes, void* stream, int reps, int* best, float* ms);
 
-/* ---- batched persistent launch ------------------------------------------
+/* ---- many particle sets in one launch ------------------------------------
  * No counterpart in the reference (one particle set per call there).  Many
  * particle sets of uneven size are concatenated into one vpm_particles_t
  * (set s owns indices [set_off[s], set_off[s+1])), each with a uniform radius
  * of its own, and evaluated by one persistent launch whose workgroups pull
- * (set, target block) work items from a device counter.  Work lists are
+ * (set, target block) work items from a device counter (vpm_batch_run), or
+ * row by row (vpm_batch_run_rows).  Work lists are
  * built by the caller: items of one set are consecutive, sets ordered by
  * decreasing size, item_block[k] counts target blocks of
  * block*targets_per_lane particles of the tile config used.  Device arrays: */

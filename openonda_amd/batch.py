@@ -1,10 +1,12 @@
 """Many particle sets of uneven size advanced together on one GPU.
 
-Each RK4 stage of every set runs in ONE persistent launch (``vpm_batch_run``:
-workgroups pull (set, target block) items, largest set first), and a whole
-time step -- four stages, their axpys, the per-set LES filter and the final
-RK4 combination -- is captured once in a HIP graph and replayed
-(``vpm_graph_*``).  Sets keep a uniform radius each.
+Each RK4 stage sums the pairs of every set in one pass: rows of 64 targets, the
+largest set's first (``vpm_batch_run_rows``: chunk counts, records, rows and, for
+few sets, the sum of the source splits), or the persistent tiled launch whose
+workgroups pull (set, target block) items (``vpm_batch_run``), as
+:func:`row_pass_pays` has it.  A whole time step -- four stages, their axpys,
+the per-set LES filter and the final RK4 combination -- is captured once in a
+HIP graph and replayed (``vpm_graph_*``).  Sets keep a uniform radius each.
 
 The step integrates the coupled particle ODE with classical RK4:
 dx/dt = u(x, alpha), dalpha/dt = S(x, alpha) [+ D_PSE(x, alpha; nu + nu_t)].
@@ -73,8 +75,9 @@ class BatchedSystem:
         :func:`row_pass_pays`, else the persistent tiled launch in its default
         shape), an index of physics.tile_configs() (the tiled launch in that
         shape), or "auto" (the batch autotuner's cached (shape, grid) for this
-        output set and total pair count, else the default).  ``grid``: persistent workgroups (0: as many as fit on
-        the device).  ``resort_every``: re-sort the sets by Morton key every
+        output set and total pair count, else the default).  ``grid``:
+        persistent workgroups of the tiled launch (0: as many as fit on the
+        device).  ``resort_every``: re-sort the sets by Morton key every
         that many steps, eager or replayed (0: only at the first step)."""
         P.require_gpu()
         if precision not in ("f32c", "f64"):
@@ -195,7 +198,7 @@ class BatchedSystem:
         return m
 
     def evaluate(self, x, a, mask, resort, stream, vel=None, stretch=None):
-        """prepare + one persistent launch on ``stream`` (the system's),
+        """prepare + one pass over every set on ``stream`` (the system's),
         after the work already issued on the current stream (inputs written
         there, outputs allocated there).  Outputs go to ``vel``/``stretch``
         (default self.vel/self.str_), self.pse_, self.vort, self.enstrophy."""

@@ -9,7 +9,7 @@
 // (stretching), :500-525 (PSE), :319-346 (vorticity), :886-909 + :777
 // (enstrophy).  Bound: FP64 issue, 37 instructions per pair for velocity +
 // stretching with a uniform radius, 41 with sigma_ij.  Velocity + stretching
-// of a cloud of 50,021: 4.10 ms with sorted records staged in LDS (80 bytes
+// of a cloud of 50,021: 4.0 ms with sorted records staged in LDS (80 bytes
 // per pair and wave through the LDS return path, which bound it), 3.12 ms
 // here (2.98 with kFold); a ring of 4,096 in the FP32-compensated precision
 // 131 -> 39 us.

@@ -16,13 +16,12 @@
 // reference's powers of s and A do, up to a factor of ten in the lengths.
 // Bound: FP64 issue.  One MI355X, before and after (before: one target per
 // lane of 256-lane workgroups, so 63 workgroups at N = 16,007, pow and IEEE
-// division per pair): driver step with LES and RK2 at N = 16,007 44.3 -> 1.25
+// division per pair): driver step with LES and RK2 at N = 16,007 44.3 -> 1.08
 // ms, the three scalar sums at N = 20,011 36.6 -> 0.61 ms, velocity and
 // vorticity of 16,007 particles at 30,011 points 18.0 -> 0.84 ms, velocity
-// and stretching of 1,000 host particles 1.40 -> 0.20 ms with the copies.
-// Each operator keeps the reference's per-pair
-// differences and cross products, so the rounding of a pair is a few ulp of
-// that pair's own terms.
+// and stretching of 1,000 host particles 1.40 -> 0.15 ms with the copies.
+// Each operator keeps the reference's per-pair differences and cross products,
+// so the rounding of a pair is a few ulp of that pair's own terms.
 
 #include "vpm_rows.h"
 

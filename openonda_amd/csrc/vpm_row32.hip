@@ -816,7 +816,7 @@ int row32_run(const FusedArgs& a, unsigned mask, bool unif, float* rec, double* 
     VPM_ROW32(26u, false) VPM_ROW32(27u, false) VPM_ROW32(31u, false)
 #undef VPM_ROW32
     default:
-      return fail(VPM_ERR_ARG, "row32: output set has the far-field moment form");
+      return fail(VPM_ERR_ARG, "row32: unknown output set");
   }
 }
 

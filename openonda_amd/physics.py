@@ -225,9 +225,9 @@ def forward(pos, alpha, sigma, nu=None, outputs=("vel", "stretch"), precision="f
     tensor.  ``precision`` is "f32c" (FP32 pairs, compensated FP64 totals)
     or "f64".  ``sigma_mode`` "uniform" asserts sigma_i == sigma_0 (not
     checked), "general" uses sigma_ij per pair, "auto" checks on the device.
-    ``tile_config``: -1 (the row pass), an index of :func:`tile_configs` (the
-    tiled kernels in that shape), or
-    "auto" (the autotuner's cached winner for this N).
+    ``tile_config``: -1 (the default pass: rows), an index of
+    :func:`tile_configs` (the tiled kernels in that shape), or "auto" (the
+    autotuner's cached winner for this N).
     ``max_splits``: 0 lets the library split the sources among workgroups
     when the targets alone cannot fill the device (small N); k >= 1 caps
     the number of splits (1: never split).
