@@ -27,7 +27,7 @@
 // Bound: FP32 issue (velocity alone 2.45e12 pairs/s, 1.55 wave64 instructions
 // per clock and CU; the moment form 1.8e12).  Tiled kernels -> here, per call.
 // N = 100,000: velocity 4.80 -> 4.17 ms, with per-particle radii 6.80 -> 4.78;
-// stretching of a ring 8.92 -> 8.32, 10.9 -> 8.60; PSE 5.81 -> 4.92, 6.75 ->
+// stretching of a ring 8.92 -> 7.99, 10.9 -> 8.60; PSE 5.81 -> 4.92, 6.75 ->
 // 5.4; vorticity + enstrophy 4.97 -> 4.73, 7.15 -> 6.15; all five with
 // per-particle radii 15.7 -> 14.3 (cloud), 18.8 -> 17.6 (ring).  Velocity +
 // stretching: cloud of 2^20 614 -> 605, of 20,000 0.448 -> 0.328, ring of
@@ -60,9 +60,10 @@ constexpr int kRow32Waves = OUT == VPM_OUT_STRETCH ? 8 : 6;
 // Record layout: offset (3), strength (3); then with the moment form the
 // moment alpha x offset (3; three times it with PSE, pair_far), with
 // per-particle radii sigma/2 and sigma^-2, with vorticity sigma^-3 behind them
-// (with PSE last); with PSE the low parts alpha - fp32(alpha).  Lengths in units of a uniform radius; with per-particle
-// radii as they are: any one particle's radius may be far from the others',
-// and the powers of t leave FP32 where distances are 1e8 units.
+// (with PSE last); with PSE the low parts alpha - fp32(alpha).  Lengths in
+// units of a uniform radius; with per-particle radii as they are: any one
+// particle's radius may be far from the others', and the powers of t leave
+// FP32 where distances are 1e8 units.
 // Two groups are in registers at once: of four records, or of two where a
 // record has twelve floats and four would spill scalar registers (velocity +
 // stretching + PSE, cloud of 131,072: 11.4 against 12.5 ms, ring 13.4 against
@@ -85,10 +86,8 @@ struct Rec32 {
   static constexpr bool kE3 = kMoment && kLo;
   static constexpr int kLoAt = kMoment ? 9 : UNIF ? 6 : 8;
   static constexpr int kIs3At = kLo ? 11 : 8;
-  static constexpr int kStride = kLo                                ? 12
-                                 : kMoment || (!UNIF && (OUT & VPM_OUT_VORT)) ? 9
-                                 : UNIF                                       ? 6
-                                                                              : 8;
+  static constexpr bool kOwnVort = !UNIF && (OUT & VPM_OUT_VORT);
+  static constexpr int kStride = kLo ? 12 : kMoment || kOwnVort ? 9 : UNIF ? 6 : 8;
   static constexpr int kGroup = kLo ? 2 : kMaxGroup32;
   static constexpr int kNear = kLo ? 4 : 2;  // sources in flight in the FP64 loop
   static constexpr int kChunk =
@@ -171,14 +170,16 @@ __device__ __forceinline__ void row32_records(const Src8* __restrict__ src, int 
   } else if constexpr (!UNIF) {
     r[6] = ok ? static_cast<float>(0.5 * sig) : 0.5f;
     r[7] = ok ? static_cast<float>(1.0 / (sig * sig)) : 1.0f;
-    if constexpr (!R::kLo && R::kStride > 8) r[8] = ok ? static_cast<float>(1.0 / (sig * sig * sig)) : 1.0f;
+    if constexpr (R::kOwnVort && !R::kLo)
+      r[R::kIs3At] = ok ? static_cast<float>(1.0 / (sig * sig * sig)) : 1.0f;
   }
   if constexpr (R::kLo) {
     r[R::kLoAt] = static_cast<float>(g.ax - static_cast<double>(ax));
     r[R::kLoAt + 1] = static_cast<float>(g.ay - static_cast<double>(ay));
     r[R::kLoAt + 2] = static_cast<float>(g.az - static_cast<double>(az));
     for (int q = R::kLoAt + 3; q < R::kStride; ++q) r[q] = 0.0f;
-    if constexpr (!UNIF) r[R::kIs3At] = ok ? static_cast<float>(1.0 / (sig * sig * sig)) : 1.0f;
+    if constexpr (R::kOwnVort)
+      r[R::kIs3At] = ok ? static_cast<float>(1.0 / (sig * sig * sig)) : 1.0f;
   }
 }
 
